@@ -174,7 +174,17 @@ static void drop_caches(ilh_plan* pl, bool release = false)
 {
     ++pl->gen;
     if (pl->mov) pl->mov->drop_sources();
-    delete pl->dir;
+    // the Dirichlet solve data's buffers (the factor and the solve matrices,
+    // four N x N or more) serve the next geometry: freeing and allocating them
+    // at every one took 1.6 of a new-geometry solve's 6.0 ms (N = 1885)
+    if (pl->dir) {
+        delete pl->dir_spare;
+        pl->dir_spare = pl->dir;
+    }
+    if (release) {
+        delete pl->dir_spare;
+        pl->dir_spare = nullptr;
+    }
     delete pl->neu;
     delete pl->sto;
     pl->dir = pl->neu = nullptr;
@@ -795,12 +805,10 @@ extern "C" int ilh_inverse_laplacian_f32(ilh_plan* pl, int kind, float* out, con
 
 // --------------------------------------------------------------- Schur
 namespace {
-__global__ void k_rhs_sign(double* B, int n, double sign)   // B = sign K - I/2, K in B (n x n)
+__global__ void k_sub_half(double* B, int n)   // B -= I/2 (n x n)
 {
-    const size_t k = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-    if (k >= (size_t)n * n) return;
-    const int r = (int)(k % n), c = (int)(k / n);
-    B[k] = sign * B[k] - (r == c ? 0.5 : 0.0);
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < n) B[k + (size_t)n * k] -= 0.5;
 }
 
 __global__ void k_rhs_dir(double* B, int n)   // B = [K - I/2, -K - I/2], K in B[:, 0:n]
@@ -962,23 +970,26 @@ void build_schur(ilh_plan* pl, int kind, double scale, double* K)
 
 // create_RTLinvR = M diag(ds) with M = -E L^-1 E^T (the (E, E) assembly of
 // the LGF, exactly symmetric): M factored by the deflated Cholesky; false
-// when it meets a non-positive pivot
-bool sym_rtlinvr(ilh_plan* pl, SymFactor& F)
+// when it meets a non-positive pivot.  scratch: N x N entries.
+bool sym_rtlinvr(ilh_plan* pl, SymFactor& F, double* scratch)
 {
     const int N = pl->N;
     F.A.ensure(sizeof(double) * (size_t)N * N);
     assemble(pl, OP_E_PRIMAL, OP_E_PRIMAL, GK_PRIMAL, -1.0, false, F.A.as<double>());
-    return sym_factor(pl, F, N);
+    return sym_factor(pl, F, N, scratch);
 }
 
 void factor_into(ilh_plan* pl, SolveCache* sc, int kind)
 {
     const int N = schur_dim(pl, kind);
-    if (kind == ILH_SCHUR_RTLINVR && sym_rtlinvr(pl, sc->sym)) {
-        sc->use_sym = true;
-        return;
+    if (kind == ILH_SCHUR_RTLINVR) {
+        // the exterior solve matrix, formed next, is the factorisation's scratch
+        sc->M[0].ensure(sizeof(double) * (size_t)N * solve_ld(N));
+        if (sym_rtlinvr(pl, sc->sym, sc->M[0].as<double>())) {
+            sc->use_sym = true;
+            return;
+        }
     }
-    sc->sym = SymFactor();
     sc->use_sym = false;
     sc->LU.ensure(sizeof(double) * (size_t)N * N);
     sc->piv.ensure(sizeof(int) * (size_t)std::max(1, N));
@@ -1012,22 +1023,20 @@ static void dirichlet_matrix(ilh_plan* pl, SolveCache* sc, int k)
     const int N = pl->N;
     hipStream_t st = pl->ctx->stream;
     const double dx2 = pl->g.dx * pl->g.dx;
-    DevBuf B;
-    B.ensure(sizeof(double) * (size_t)N * N);
-    assemble(pl, OP_E_PRIMAL, OP_DS, GK_PRIMAL, dx2, false, B.as<double>());
-    k_rhs_sign<<<(unsigned)(((size_t)N * N + 255) / 256), 256, 0, st>>>(B.as<double>(), N, k ? -1.0 : 1.0);
+    const int ld = solve_ld(N);
+    sc->M[k].ensure(sizeof(double) * (size_t)N * ld);
+    double *B = sc->sym.A.as<double>(), *M = sc->M[k].as<double>();   // the factored matrix's storage is free
+    assemble(pl, OP_E_PRIMAL, OP_DS, GK_PRIMAL, k ? -dx2 : dx2, false, B);
+    k_sub_half<<<(N + 255) / 256, 256, 0, st>>>(B, N);
     ILH_HIP(hipGetLastError());
     if (sc->use_sym) {
         // S^-1 B = diag(1 / ds) M^-1 B
-        sym_solve(pl, sc->sym, B.as<double>(), N);
-        scale_rows_inv(st, B.as<double>(), N, N, pl->ds.as<double>(), 1.0);
+        sym_solve_rows(pl, sc->sym, B, N, pl->ds.as<double>(), 1.0, M, ld);
+        zero_pad_columns(st, M, N, ld);
     } else {
-        lu_solve_multi(pl, sc->LU.as<double>(), sc->piv.as<int>(), N, B.as<double>(), N);
+        lu_solve_multi(pl, sc->LU.as<double>(), sc->piv.as<int>(), N, B, N);
+        transpose(st, B, M, N, N, ld);
     }
-    const int ld = solve_ld(N);
-    sc->M[k].ensure(sizeof(double) * (size_t)N * ld);
-    transpose(st, B.as<double>(), sc->M[k].as<double>(), N, N, ld);
-    ILH_HIP(hipStreamSynchronize(st));   // B is released on return
 }
 
 // The plan's Dirichlet solve data: the factor of S, the exterior-data matrix
@@ -1039,14 +1048,15 @@ SolveCache* prepare_dirichlet(ilh_plan* pl, bool need_minus = true)
     if (!sc) {
         need_margin(pl, "Dirichlet solve");
         const int N = pl->N;
-        sc = new SolveCache();
+        sc = pl->dir_spare ? pl->dir_spare : new SolveCache();
+        pl->dir_spare = nullptr;
+        sc->minus_ok = false;
         try {
             if (N > 0) {
                 factor_into(pl, sc, ILH_SCHUR_RTLINVR);
                 dirichlet_matrix(pl, sc, 0);
                 merge_sources(pl, OP_R_PRIMAL, OP_DS, GK_PRIMAL, sc->terms1, sc->src1);
                 pin_source_pairs(pl, sc->src1);
-                ILH_HIP(hipStreamSynchronize(pl->ctx->stream));
             }
             sc->amp1.ensure(sizeof(double) * (size_t)std::max(1, 2 * N));
         } catch (...) {
@@ -1113,7 +1123,7 @@ void ilh::exact_inverse_rowmajor(ilh_plan* pl, double* Pd)
 {
     const int N = pl->N;
     SymFactor F;
-    if (sym_rtlinvr(pl, F)) {
+    if (sym_rtlinvr(pl, F, Pd)) {   // the inverse's rows are written after the factorisation
         sym_inverse_rowmajor(pl, F, pl->ds.as<double>(), 1.0, Pd);
         return;
     }
@@ -1149,6 +1159,7 @@ extern "C" int ilh_schur_factor(ilh_plan* pl, int kind)
         SolveCache* sc = new SolveCache();
         try {
             if (pl->N > 0) factor_into(pl, sc, kind);
+            sc->M[0].release();   // the factorisation's scratch: no solve matrix is formed here
         } catch (...) {
             delete sc;
             throw;
@@ -1171,8 +1182,7 @@ extern "C" int ilh_schur_solve(ilh_plan* pl, int kind, double* x, const double* 
                 ILH_HIP(hipMemcpyAsync(d_x, d_b, sizeof(double) * N, hipMemcpyDeviceToDevice, pl->ctx->stream));
             SolveCache* sc = pl->fac[kind];
             if (sc->use_sym) {
-                sym_solve(pl, sc->sym, d_x, 1);
-                scale_rows_inv(pl->ctx->stream, d_x, N, 1, pl->ds.as<double>(), 1.0);
+                sym_solve_rows(pl, sc->sym, d_x, 1, pl->ds.as<double>(), 1.0, d_x, 1);
             } else {
                 lu_solve_multi(pl, sc->LU.as<double>(), sc->piv.as<int>(), N, d_x, 1);
             }

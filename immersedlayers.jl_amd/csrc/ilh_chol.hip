@@ -25,6 +25,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 
 namespace ilh {
 
@@ -34,67 +35,123 @@ typedef double double4_t __attribute__((ext_vector_type(4)));
 // C (M x Nc) = beta C + alpha opA(A) opB(B), column-major, beta in {0, 1}
 // (BETA0: C is not read).  opA(A)[m][k] = A[m + lda k] (TA = 0) or
 // A[k + lda m] (TA = 1); opB(B)[k][n] = B[k + ldb n] (TB = 0) or B[n + ldb k]
-// (TB = 1).  LOWER: tiles lying wholly above the diagonal of a square C are
-// skipped (their entries are never read).  tri restricts the K range of each
-// tile to where a triangular operand is nonzero (its other triangle must hold
-// zeros): TRI_A_LOWER opA(A)[m][k] = 0 for k > m, TRI_A_UPPER for k < m,
-// TRI_B_LOWER opB(B)[k][n] = 0 for k < n, TRI_B_UPPER for k > n.
+// (TB = 1).  tri restricts the K range of each tile to where a triangular
+// operand is nonzero (entries of its other triangle outside its 64 x 64
+// diagonal blocks are never read): TRI_A_LOWER opA(A)[m][k] = 0 for k > m,
+// TRI_A_UPPER for k < m, TRI_B_LOWER opB(B)[k][n] = 0 for k < n, TRI_B_UPPER
+// for k > n.
 //
 // 64 x 64 tile per work-group of four waves, each wave a 32 x 32 quadrant of
 // 2 x 2 blocks of 16 x 16.  K runs in chunks of 16 through two LDS buffers:
 // the next chunk's global loads are in flight while the current one feeds the
-// matrix cores.  The product is formed transposed (the B tile as the MFMA's
-// first operand), so a lane's result entries run down a column of C and the
-// stores of 16 lanes cover 128 contiguous bytes.
+// matrix cores, and all of a chunk's LDS fragments are read before its 16
+// matrix instructions, so that they issue back to back (1024 of a chunk's
+// cycles; the wave's LDS wait is paid once per chunk).  The product is formed
+// transposed (the B tile as the MFMA's first operand), so a lane's result
+// entries run down a column of C and the stores of 16 lanes cover 128
+// contiguous bytes.  The bound is the matrix cores' FP64 rate (32 FMA cycles
+// per 16 x 16 x 4 product); the tiles with the longest K range of a triangular
+// operand are dispatched first.
 // v_mfma_f64_16x16x4f64 lane layout (checked on gfx950): first operand
 // X[i][k] at lane i + 16 k, second Y[k][j] at lane j + 16 k; lane l, item r
 // of the result holds D[l / 16 + 4 r][l % 16].
 static constexpr int GT = 64, GKC = 16;
 
-template <int TA, int TB, bool LOWER, bool BETA0>
+// A batch runs over blockIdx.z: operands at z times the strides, M (and K,
+// when k_is_m) clipped to what is left of m_total rows z m_step on.
+struct GemmBatch {
+    size_t sa = 0, sb = 0, sc = 0;
+    int m_total = 0, m_step = 0;
+    int k_is_m = 0;
+};
+// Epilogues: EPI_RANK1 C = alpha AB - 2 u[m] v[n]; EPI_DEFLATE
+// C = (AB - a[m] u[n] - 2 b[m] w[n]) / (c d[n]).
+enum { EPI_NONE = 0, EPI_RANK1 = 1, EPI_DEFLATE = 2 };
+struct GemmEpi {
+    const double *u = nullptr, *v = nullptr;                                         // EPI_RANK1
+    const double *a = nullptr, *b = nullptr, *wt = nullptr, *w1 = nullptr, *d = nullptr;   // EPI_DEFLATE
+    double c = 1.0;
+};
+
+template <int TA, int TB, bool BETA0, int EPI>
 // (A or B may be C itself when every work-group reads all the entries it
-// overwrites: the in-place panel and diagonal-block products below; hence no
-// __restrict__.)
+// overwrites; hence no __restrict__.)
 __global__ void __launch_bounds__(256) k_dgemm(int M, int Nc, int K, double alpha, const double* A, int lda,
-                                               const double* B, int ldb, double* C, int ldc, int tri)
+                                               const double* B, int ldb, double* C, int ldc, int tri, GemmBatch bt,
+                                               GemmEpi ep)
 {
     __shared__ double As[2][GKC][GT + 2];   // As[k][m]
     __shared__ double Bs[2][GKC][GT + 2];   // Bs[k][n]
-    const int m0 = blockIdx.x * GT, n0 = blockIdx.y * GT;
-    if (LOWER && m0 + GT - 1 < n0) return;
+    const int z = blockIdx.z;
+    A += bt.sa * z;
+    B += bt.sb * z;
+    C += bt.sc * z;
+    if (bt.m_step) {
+        M = min(M, bt.m_total - z * bt.m_step);
+        if (bt.k_is_m) K = min(K, M);
+    }
+    // triangular operands: tiles by falling K range, every second round of
+    // 256 (one per CU) backwards, so that the rounds' sums come out even
+    int bx = blockIdx.x, by = blockIdx.y;
+    if (tri != TRI_NONE) {
+        const int total = gridDim.x * gridDim.y;
+        int t = blockIdx.x + gridDim.x * blockIdx.y;
+        const int r0 = t & ~255;
+        if (r0 & 256) t = r0 + min(256, total - r0) - 1 - (t - r0);
+        if (tri == TRI_A_LOWER || tri == TRI_A_UPPER) {
+            bx = t / gridDim.y;
+            by = t % gridDim.y;
+            if (tri == TRI_A_LOWER) bx = gridDim.x - 1 - bx;
+        } else {
+            by = t / gridDim.x;
+            bx = t % gridDim.x;
+            if (tri == TRI_B_UPPER) by = gridDim.y - 1 - by;
+        }
+    }
+    const int m0 = bx * GT, n0 = by * GT;
+    if (m0 >= M || n0 >= Nc) return;
     int klo = 0, khi = K;
     if (tri == TRI_A_LOWER) khi = min(K, m0 + GT);
     else if (tri == TRI_A_UPPER) klo = m0;
     else if (tri == TRI_B_LOWER) klo = n0;
     else if (tri == TRI_B_UPPER) khi = min(K, n0 + GT);
-    const int kbase = klo / GKC * GKC;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
-    double ra[4], rb[4];
-    auto load = [&](int k0) {
+    // this thread's four elements of each operand's chunk.  Rows and columns
+    // past the end load the last one's entries (their products are not
+    // stored), and k past the end an entry that exists, zeroed on its way to
+    // LDS: the loads themselves carry no branch or use, so that three chunks
+    // of them stay in flight
+    const int am = TA == 0 ? tid & 63 : tid >> 4, ak = TA == 0 ? tid >> 6 : tid & 15;
+    const int bn = TB == 0 ? tid >> 4 : tid & 63, bk = TB == 0 ? tid & 15 : tid >> 6;
+    const double *pa[4], *pb[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int m = min(m0 + am + (TA == 0 ? 0 : 16 * j), M - 1), n = min(n0 + bn + (TB == 0 ? 16 * j : 0), Nc - 1);
+        const int k = klo + ak + (TA == 0 ? 4 * j : 0), kb = klo + bk + (TB == 0 ? 0 : 4 * j);
+        pa[j] = TA == 0 ? A + m + (size_t)lda * k : A + k + (size_t)lda * m;
+        pb[j] = TB == 0 ? B + kb + (size_t)ldb * n : B + n + (size_t)ldb * kb;
+    }
+    const size_t step_a = TA == 0 ? (size_t)lda * GKC : GKC, step_b = TB == 0 ? GKC : (size_t)ldb * GKC;
+    double pre[3][8];   // three chunks on the way: [0..3] of A, [4..7] of B
+    auto load = [&](int k0, double* r) {   // the chunk at k0 (in order: the pointers advance with it)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            int m, k;
-            if (TA == 0) { m = tid & 63; k = (tid >> 6) + 4 * j; }
-            else { k = tid & 15; m = (tid >> 4) + 16 * j; }
-            const int gm = m0 + m, gk = k0 + k;
-            ra[j] = (gm < M && gk >= klo && gk < khi) ? (TA == 0 ? A[gm + (size_t)lda * gk] : A[gk + (size_t)lda * gm])
-                                                      : 0.0;
-            int n, kb;
-            if (TB == 0) { kb = tid & 15; n = (tid >> 4) + 16 * j; }
-            else { n = tid & 63; kb = (tid >> 6) + 4 * j; }
-            const int gn = n0 + n, gkb = k0 + kb;
-            rb[j] = (gn < Nc && gkb >= klo && gkb < khi) ? (TB == 0 ? B[gkb + (size_t)ldb * gn] : B[gn + (size_t)ldb * gkb])
-                                                          : 0.0;
+            r[j] = *(k0 + ak + (TA == 0 ? 4 * j : 0) < khi ? pa[j] : A);
+            r[4 + j] = *(k0 + bk + (TB == 0 ? 0 : 4 * j) < khi ? pb[j] : B);
+            pa[j] += step_a;
+            pb[j] += step_b;
         }
     };
-    auto store = [&](int buf) {
+    auto store = [&](int k0, int buf, const double* r) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            if (TA == 0) As[buf][(tid >> 6) + 4 * j][tid & 63] = ra[j];
-            else As[buf][tid & 15][(tid >> 4) + 16 * j] = ra[j];
-            if (TB == 0) Bs[buf][tid & 15][(tid >> 4) + 16 * j] = rb[j];
-            else Bs[buf][(tid >> 6) + 4 * j][tid & 63] = rb[j];
+            const double va = k0 + ak + (TA == 0 ? 4 * j : 0) < khi ? r[j] : 0.0;
+            const double vb = k0 + bk + (TB == 0 ? 0 : 4 * j) < khi ? r[4 + j] : 0.0;
+            if (TA == 0) As[buf][(tid >> 6) + 4 * j][tid & 63] = va;
+            else As[buf][tid & 15][(tid >> 4) + 16 * j] = va;
+            if (TB == 0) Bs[buf][tid & 15][(tid >> 4) + 16 * j] = vb;
+            else Bs[buf][(tid >> 6) + 4 * j][tid & 63] = vb;
         }
     };
     double4_t acc[2][2];
@@ -102,76 +159,94 @@ __global__ void __launch_bounds__(256) k_dgemm(int M, int Nc, int K, double alph
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = (double4_t){0.0, 0.0, 0.0, 0.0};
-    const int nch = khi > kbase ? (khi - kbase + GKC - 1) / GKC : 0;
-    load(kbase);
-    store(0);
-    __syncthreads();
-    for (int c = 0; c < nch; ++c) {
-        const int buf = c & 1;
-        if (c + 1 < nch) load(kbase + (c + 1) * GKC);
+    const int nch = khi > klo ? (khi - klo + GKC - 1) / GKC : 0;
+    if (nch > 0) {
+        // chunk c is loaded three ahead, into the registers that chunk c - 3 left
 #pragma unroll
-        for (int kk = 0; kk < GKC; kk += 4) {
-            const int kr = kk + (lane >> 4);
-            double a[2], b[2];
+        for (int q = 0; q < 3; ++q) load(klo + q * GKC, pre[q]);
+        store(klo, 0, pre[0]);
+        lds_sync();
+    }
+    for (int c0 = 0; c0 < nch; c0 += 3) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i) a[i] = As[buf][kr][wm + 16 * i + (lane & 15)];
+        for (int q = 0; q < 3; ++q) {
+            const int c = c0 + q;
+            if (c >= nch) break;
+            const int buf = c & 1;
+            double a[4][2], b[4][2];
 #pragma unroll
-            for (int j = 0; j < 2; ++j) b[j] = Bs[buf][kr][wn + 16 * j + (lane & 15)];
+            for (int kk = 0; kk < 4; ++kk) {
+                const int kr = 4 * kk + (lane >> 4);
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+                for (int i = 0; i < 2; ++i) {
+                    a[kk][i] = As[buf][kr][wm + 16 * i + (lane & 15)];
+                    b[kk][i] = Bs[buf][kr][wn + 16 * i + (lane & 15)];
+                }
+            }
+            load(klo + (c + 3) * GKC, pre[q]);
 #pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j], a[i], acc[i][j], 0, 0, 0);
+            for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[kk][j], a[kk][i], acc[i][j], 0, 0, 0);
+            store(klo + (c + 1) * GKC, buf ^ 1, pre[(q + 1) % 3]);
+            lds_sync();
         }
-        if (c + 1 < nch) store(buf ^ 1);
-        __syncthreads();
     }
     // acc[i][j] item r of lane l: C row m0 + wm + 16 i + l % 16, column n0 + wn + 16 j + l / 16 + 4 r
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i) {
+        const int gm = m0 + wm + 16 * i + (lane & 15);
+        if (gm >= M) continue;
+        double e0 = 0.0, e1 = 0.0;
+        if (EPI == EPI_RANK1) e0 = ep.u[gm];
+        if (EPI == EPI_DEFLATE) { e0 = ep.a[gm]; e1 = ep.b[gm]; }
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int gm = m0 + wm + 16 * i + (lane & 15);
                 const int gn = n0 + wn + 16 * j + (lane >> 4) + 4 * r;
-                if (gm < M && gn < Nc) {
-                    double* p = C + gm + (size_t)ldc * gn;
-                    *p = BETA0 ? alpha * acc[i][j][r] : *p + alpha * acc[i][j][r];
-                }
+                if (gn >= Nc) continue;
+                double* p = C + gm + (size_t)ldc * gn;
+                if (EPI == EPI_RANK1) *p = alpha * acc[i][j][r] - 2.0 * e0 * ep.v[gn];
+                else if (EPI == EPI_DEFLATE)
+                    *p = (acc[i][j][r] - e0 * ep.wt[gn] - 2.0 * e1 * ep.w1[gn]) / (ep.c * ep.d[gn]);
+                else *p = BETA0 ? alpha * acc[i][j][r] : *p + alpha * acc[i][j][r];
             }
+    }
 }
 
 void dgemm(hipStream_t st, int ta, int tb, int M, int Nc, int K, double alpha, const double* A, int lda,
-           const double* B, int ldb, double beta, double* C, int ldc, bool lower, int tri)
+           const double* B, int ldb, double beta, double* C, int ldc, int tri)
 {
     if (M <= 0 || Nc <= 0) return;
     if (beta != 0.0 && beta != 1.0) fail(ILH_ERR_ARG, "dgemm: beta must be 0 or 1");
     const dim3 grid((M + GT - 1) / GT, (Nc + GT - 1) / GT);
     const bool b0 = beta == 0.0;
-#define ILH_DG(TA_, TB_, LO_, B0_) \
-    k_dgemm<TA_, TB_, LO_, B0_><<<grid, 256, 0, st>>>(M, Nc, K, alpha, A, lda, B, ldb, C, ldc, tri)
+#define ILH_DG(TA_, TB_, B0_) \
+    k_dgemm<TA_, TB_, B0_, EPI_NONE><<<grid, 256, 0, st>>>(M, Nc, K, alpha, A, lda, B, ldb, C, ldc, tri, GemmBatch(), GemmEpi())
     if (K <= 0) {
         if (!b0) return;
         alpha = 0.0;   // C = 0
     }
-    if (lower) {
-        if (ta != 0 || tb != 1 || b0) fail(ILH_ERR_ARG, "dgemm: the lower-triangle form is C += alpha A B^T");
-        ILH_DG(0, 1, true, false);
-    } else if (ta == 0 && tb == 0) {
-        if (b0) ILH_DG(0, 0, false, true); else ILH_DG(0, 0, false, false);
+    if (ta == 0 && tb == 0) {
+        if (b0) ILH_DG(0, 0, true); else ILH_DG(0, 0, false);
     } else if (ta == 0 && tb == 1) {
-        if (b0) ILH_DG(0, 1, false, true); else ILH_DG(0, 1, false, false);
+        if (b0) ILH_DG(0, 1, true); else ILH_DG(0, 1, false);
     } else if (ta == 1 && tb == 0) {
-        if (b0) ILH_DG(1, 0, false, true); else ILH_DG(1, 0, false, false);
+        if (b0) ILH_DG(1, 0, true); else ILH_DG(1, 0, false);
     } else {
-        if (b0) ILH_DG(1, 1, false, true); else ILH_DG(1, 1, false, false);
+        if (b0) ILH_DG(1, 1, true); else ILH_DG(1, 1, false);
     }
 #undef ILH_DG
     ILH_HIP(hipGetLastError());
 }
 
 // ------------------------------------------------------------- Cholesky
-static constexpr int CB = 64;   // block size of the factorisation and of the solves
+static constexpr int CB = 64;   // block size of the factorisation
+static constexpr int SB = 16;   // sub-block of a diagonal block: one matrix-core product
 
 __device__ __forceinline__ double readlane_d(double v, int lane)
 {
@@ -181,210 +256,396 @@ __device__ __forceinline__ double readlane_d(double v, int lane)
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-// Cholesky of the nb x nb diagonal block at (k0, k0) of A (lower triangle
-// used), written back into A's lower triangle, and the inverse of the factor
-// (nb x nb with the zeros of its upper triangle) into Winv (leading dimension ldw).
-// Work-group barriers, not arithmetic, set the time of a small factorisation,
-// so the block is processed in 16-wide sub-blocks: one wave factors a 16 x 16
-// diagonal sub-block on its own (lane i holds row i; the pivot and the column
-// of each step are broadcast with readlane, no barrier), then the work-group
-// solves the sub-panel below it and updates the trailing lower triangle.  The
-// inverse is built the same way: the four 16 x 16 diagonal inverses in
-// parallel (one wave each), then the off-diagonal blocks by their distance
-// from the diagonal.  A pivot that is not positive records its 1-based column
-// in *info (the first one only) and is replaced by 1, so that the kernel still
-// runs to its end.
-static constexpr int SB = 16;
-
-__global__ void __launch_bounds__(256) k_chol_diag(double* __restrict__ A, int lda, int k0, int nb,
-                                                   double* __restrict__ Winv, int ldw, int* __restrict__ info)
+// 1 / sqrt(x), x > 0 and of ordinary size: the hardware estimate and two
+// coupled Newton steps (Goldschmidt), to within an ulp or two
+__device__ __forceinline__ double rsqrt_nr(double x)
 {
-    __shared__ double T[CB][CB + 1];
-    __shared__ double X[CB][CB + 1];
-    __shared__ double Y[3][SB][SB + 1];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int e = tid; e < CB * CB; e += 256) {
-        const int r = e % CB, c = e / CB;
-        T[r][c] = (r < nb && c < nb) ? (r >= c ? A[(k0 + r) + (size_t)lda * (k0 + c)] : 0.0) : (r == c ? 1.0 : 0.0);
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+        const double r = __builtin_fma(-g, h, 0.5);
+        g = __builtin_fma(g, r, g);
+        h = __builtin_fma(h, r, h);
     }
-    __syncthreads();
-    for (int o = 0; o < CB; o += SB) {
-        // (a) the 16 x 16 diagonal sub-block, wave 0
+    return 2.0 * h;
+}
+
+// 64 x 64 blocks in LDS, row-major with one pad entry per row
+typedef double Block[CB][CB + 1];
+
+// X_bb = L_bb^-1 of the 16 x 16 diagonal sub-block b (lane c % 16 forms column
+// c by forward substitution; rd: reciprocals of L's diagonal).  Every wave that
+// needs X_bb calls this itself and then reads back only what it wrote (equal
+// values in the same places), so no barrier is needed.
+__device__ __forceinline__ void sub_inverse(const Block& T, const double* rd, Block& X, int b, int lane)
+{
+    const int o = b * SB, c = lane & 15;
+    double x[SB];
+#pragma unroll
+    for (int r = 0; r < SB; ++r) {
+        double v = r == c ? 1.0 : 0.0, v2 = 0.0;
+#pragma unroll
+        for (int k = 0; k < r; ++k) {
+            if (k & 1) v2 = __builtin_fma(-T[o + r][o + k], x[k], v2);
+            else v = __builtin_fma(-T[o + r][o + k], x[k], v);
+        }
+        x[r] = (v + v2) * rd[o + r];
+    }
+    if (lane < SB)
+#pragma unroll
+        for (int r = 0; r < SB; ++r) X[o + r][o + c] = x[r];
+}
+
+// X_ij = -X_ii sum_{k=j}^{i-1} L_ik X_kj for 16 x 16 sub-blocks, by one wave:
+// the inner sum's result layout is the second operand's layout of the outer
+// product, so nothing is exchanged in between
+__device__ __forceinline__ void sub_inverse_off(const Block& T, Block& X, int i, int j, int lane)
+{
+    const int lr = lane & 15, lk = lane >> 4;
+    double4_t y = (double4_t){0.0, 0.0, 0.0, 0.0};
+    for (int k = j; k < i; ++k)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            y = __builtin_amdgcn_mfma_f64_16x16x4f64(T[i * SB + lr][k * SB + 4 * q + lk], X[k * SB + 4 * q + lk][j * SB + lr],
+                                                     y, 0, 0, 0);
+    double4_t x = (double4_t){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        x = __builtin_amdgcn_mfma_f64_16x16x4f64(X[i * SB + lr][i * SB + 4 * q + lk], y[q], x, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) X[i * SB + lk + 4 * r][j * SB + lr] = -x[r];
+}
+
+// T_ij -= L_ib L_jb^T for 16 x 16 sub-blocks, by one wave
+__device__ __forceinline__ void sub_update(Block& T, int i, int j, int b, int lane)
+{
+    const int lr = lane & 15, lk = lane >> 4;
+    double4_t acc = (double4_t){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(T[i * SB + lr][b * SB + 4 * q + lk], T[j * SB + lr][b * SB + 4 * q + lk],
+                                                   acc, 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) T[i * SB + lk + 4 * r][j * SB + lr] -= acc[r];
+}
+
+// Cholesky of the 64 x 64 block in T (its lower triangle) by a work-group of
+// four waves, and the inverse of the factor in X's lower sub-blocks.  Column
+// panels of 16: wave 0 holds all 64 rows of the panel (lane = row) and factors
+// it alone, the pivot and the multipliers of each step broadcast with
+// readlane, so the rows below the diagonal sub-block cost nothing extra; the
+// next panel's update comes first, and everything else (the remaining
+// updates, the inverse's finished rows) runs on the other waves beside the
+// next panel.  Seven barriers; the chain of 64 pivot steps bounds it.
+// A pivot that is not positive records its 1-based column col0 + ... in *info
+// (the first one only) and is replaced by 1, so that the kernel still runs to
+// its end.
+__device__ __forceinline__ void chol_block(Block& T, Block& X, double* rd, int col0, int* info)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    auto finish_row = [&](int b) {   // waves 1..3: row b of the inverse
+        sub_inverse(T, rd, X, b, lane);
+        if (wave - 1 < b) sub_inverse_off(T, X, b, wave - 1, lane);
+    };
+#pragma unroll
+    for (int b = 0; b < CB / SB; ++b) {
+        const int o = b * SB;
         if (wave == 0) {
             double d[SB];
-            const int ri = lane < SB ? lane : 0;
 #pragma unroll
-            for (int c = 0; c < SB; ++c) d[c] = T[o + ri][o + c];
+            for (int c = 0; c < SB; ++c) d[c] = T[lane][o + c];
+            // the next pivot's reciprocal root is formed beside the rest of a
+            // step's updates; the scheduling barriers keep a step's broadcast
+            // values from piling up in scalar registers
+            double piv = readlane_d(d[0], o), rdv = 1.0;
+            int bad = 0;
+            double ri = 1.0;
 #pragma unroll
             for (int j = 0; j < SB; ++j) {
-                double piv = readlane_d(d[j], j);
-                if (!(piv > 0.0)) {
-                    if (lane == 0) atomicCAS(info, 0, k0 + o + j + 1);
-                    piv = 1.0;
+                if (j == 0) {
+                    bad = piv > 0.0 ? 0 : 1;
+                    piv = piv > 0.0 ? piv : 1.0;
+                    ri = rsqrt_nr(piv);
                 }
-                const double ljj = sqrt(piv), rinv = 1.0 / ljj;
-                const double lij = d[j] * rinv;
+                const double l = d[j] * ri;
+                d[j] = lane > o + j ? l : (lane == o + j ? piv * ri : 0.0);
+                rdv = lane == j ? ri : rdv;
+                if (j + 1 < SB) {
+                    d[j + 1] = __builtin_fma(-l, readlane_d(l, o + j + 1), d[j + 1]);
+                    piv = readlane_d(d[j + 1], o + j + 1);
+                    bad = bad == 0 && !(piv > 0.0) ? j + 2 : bad;
+                    piv = piv > 0.0 ? piv : 1.0;
+                    ri = rsqrt_nr(piv);
 #pragma unroll
-                for (int l = j + 1; l < SB; ++l) d[l] -= lij * readlane_d(lij, l);
-                d[j] = lane > j ? lij : (lane == j ? ljj : 0.0);
-            }
-            if (lane < SB)
-#pragma unroll
-                for (int c = 0; c < SB; ++c) T[o + lane][o + c] = c <= lane ? d[c] : 0.0;
-        }
-        __syncthreads();
-        const int rest = CB - o - SB;
-        if (rest > 0) {
-            // (b) sub-panel: rows o+16.. solve p L11^T = a (one thread per row)
-            if (tid < rest) {
-                const int r = o + SB + tid;
-                double p[SB];
-#pragma unroll
-                for (int c = 0; c < SB; ++c) {
-                    double v = T[r][o + c];
-#pragma unroll
-                    for (int k = 0; k < c; ++k) v -= p[k] * T[o + c][o + k];
-                    p[c] = v / T[o + c][o + c];
+                    for (int c = j + 2; c < SB; ++c) d[c] = __builtin_fma(-l, readlane_d(l, o + c), d[c]);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-#pragma unroll
-                for (int c = 0; c < SB; ++c) T[r][o + c] = p[c];
             }
-            __syncthreads();
-            // (c) trailing lower triangle: T[r][s] -= sum_k P[r][k] P[s][k]
-            for (int e = tid; e < rest * rest; e += 256) {
-                const int ri = e % rest, si = e / rest;
-                if (si > ri) continue;
-                const int r = o + SB + ri, sc = o + SB + si;
-                double acc = 0.0;
+            if (bad && lane == 0) atomicCAS(info, 0, col0 + o + bad);
+            if (lane < SB) rd[o + lane] = rdv;
+            if (lane >= o)
 #pragma unroll
-                for (int k = 0; k < SB; ++k) acc += T[r][o + k] * T[sc][o + k];
-                T[r][sc] -= acc;
+                for (int c = 0; c < SB; ++c) T[lane][o + c] = d[c];
+        } else if (b > 0) {
+            // updates by panel b - 1 beyond panel b: (2,2) (3,2) (3,3), then (3,3)
+            if (b == 1) sub_update(T, wave == 1 ? 2 : 3, wave == 3 ? 3 : 2, 0, lane);
+            if (b == 2 && wave == 1) sub_update(T, 3, 3, 1, lane);
+            finish_row(b - 1);
+        }
+        lds_sync();
+        if (b + 1 < CB / SB) {
+            if (b + 1 + wave < CB / SB) sub_update(T, b + 1 + wave, b + 1, b, lane);
+            lds_sync();
+        }
+    }
+    if (wave > 0) finish_row(CB / SB - 1);
+    lds_sync();
+}
+
+// One step of the right-looking blocked Cholesky of the m x m matrix A (lower
+// triangle): block column k is eliminated from every 64 x 64 tile (i, j),
+// k < j <= i, one work-group each,
+//     A_ij -= L_ik L_jk^T,   L_ik = A_ik W_kk^T,  W_kk = L_kk^-1,
+// and the work-group of tile (k+1, k+1) goes on to factor it and to invert the
+// factor (W_{k+1,k+1}), so that a step is one launch and the diagonal chain
+// runs beside the other tiles.  Every work-group forms the two panel blocks it
+// needs itself (the panel is small next to a separate launch for it); the one
+// of column k+1 keeps L_ik in Lb.  k = -1: tile (0, 0) is factored only.
+// Each wave forms 16 rows of both panel blocks, operands straight from memory
+// (16 rows are 128 contiguous bytes); a result item's layout is the operand
+// layout of one K step, so the blocks pass through LDS as they are.
+// Bound by the diagonal chain (update, 64 pivot steps, inverse); N = 1885
+// (30 steps): 22 us per step; the recursive form this replaced, three to
+// five launches per block around a 39 us diagonal kernel, took 85 us per block.
+__global__ void __launch_bounds__(256) k_chol_step(double* __restrict__ A, int lda, int m, int k, double* __restrict__ W,
+                                                   int ldw, double* __restrict__ Lb, int ldl, int* __restrict__ info)
+{
+    __shared__ double sm[2 * CB * (CB + 1)];
+    __shared__ double rd[CB];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lr = lane & 15, lk = lane >> 4;
+    const int wm = (wave & 1) * 2, wn = (wave >> 1) * 2;   // quadrant, in 16-blocks
+    int ti = 0, tj = 0;
+    if (k >= 0) {
+        const int t = blockIdx.x;
+        ti = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
+        while (ti * (ti + 1) / 2 > t) --ti;
+        while ((ti + 1) * (ti + 2) / 2 <= t) ++ti;
+        tj = t - ti * (ti + 1) / 2;
+    }
+    const int i0 = (k + 1 + ti) * CB, j0 = (k + 1 + tj) * CB;
+    double4_t c[2][2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = i0 + 16 * (wm + x) + lr, col = j0 + 16 * (wn + y) + lk + 4 * r;
+                c[x][y][r] = row < m && col < m ? A[row + (size_t)lda * col] : 0.0;
             }
-            __syncthreads();
+    if (k >= 0) {
+        const int k0 = k * CB;
+        const double* Wk = W + k0 + (size_t)ldw * k0;
+        // W_kk's fragments (its lower sub-blocks), then the wave's 16 rows of both panel blocks
+        double w[40], a[2][16];
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+            for (int q = 0; q < 4 * (cb + 1); ++q)
+                w[2 * cb * (cb + 1) + q] = Wk[16 * cb + lr + (size_t)ldw * (4 * q + lk)];
+        const bool two = ti != tj;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            if (p == 1 && !two) break;
+            const int row = min((p ? j0 : i0) + 16 * wave + lr, m - 1);   // rows past the end: copies of the last
+#pragma unroll
+            for (int q = 0; q < 16; ++q) a[p][q] = A[row + (size_t)lda * (k0 + 4 * q + lk)];
         }
-    }
-    for (int e = tid; e < nb * nb; e += 256) {
-        const int r = e % nb, c = e / nb;
-        if (r >= c) A[(k0 + r) + (size_t)lda * (k0 + c)] = T[r][c];
-    }
-    // inverse: the diagonal 16 x 16 inverses, wave b forms block b (lane c < 16: column c)
-    {
-        const int o = wave * SB, c = lane;
-        if (c < SB) {
-            double x[SB];
 #pragma unroll
-            for (int r = 0; r < SB; ++r) {
-                double v = r == c ? 1.0 : 0.0;
+        for (int p = 0; p < 2; ++p) {
+            if (p == 1 && !two) break;
 #pragma unroll
-                for (int k = 0; k < r; ++k) v -= T[o + r][o + k] * x[k];
-                x[r] = v / T[o + r][o + r];
+            for (int cb = 0; cb < 4; ++cb) {
+                double4_t l = (double4_t){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int q = 0; q < 4 * (cb + 1); ++q)
+                    l = __builtin_amdgcn_mfma_f64_16x16x4f64(w[2 * cb * (cb + 1) + q], a[p][q], l, 0, 0, 0);
+                // item r: row lr of the wave's 16, column 16 cb + 4 r + lk = the operand of K step 4 cb + r
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sm[p * CB * CB + (wave * 16 + 4 * cb + r) * 64 + lane] = l[r];
+                const int row = i0 + 16 * wave + lr;
+                if (p == 0 && tj == 0 && row < m)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) Lb[row + (size_t)ldl * (k0 + 16 * cb + 4 * r + lk)] = l[r];
+            }
+        }
+        lds_sync();
+        const double* sj = sm + (two ? CB * CB : 0);
+        double4_t u[2][2];
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) u[x][y] = (double4_t){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            double fa[2], fb[2];
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+                fa[x] = sm[((wm + x) * 16 + q) * 64 + lane];
+                fb[x] = sj[((wn + x) * 16 + q) * 64 + lane];
             }
 #pragma unroll
-            for (int r = 0; r < SB; ++r) X[o + r][o + c] = x[r];
-        }
-        for (int e = tid; e < CB * CB; e += 256) {   // zero the strict upper blocks
-            const int r = e % CB, cc = e / CB;
-            if (r / SB < cc / SB) X[r][cc] = 0.0;
-        }
-    }
-    __syncthreads();
-    // off-diagonal blocks (bi, bj), bi - bj = dist: X_ij = -X_ii sum_{k=j}^{i-1} L_ik X_kj
-    for (int dist = 1; dist < CB / SB; ++dist) {
-        const int nblk = CB / SB - dist;
-        for (int e = tid; e < nblk * SB * SB; e += 256) {
-            const int b = e / (SB * SB), rr = e % SB, cc = (e / SB) % SB;
-            const int bj = b, bi = b + dist;
-            double acc = 0.0;
-            for (int kb = bj; kb < bi; ++kb)
+            for (int x = 0; x < 2; ++x)
 #pragma unroll
-                for (int k = 0; k < SB; ++k) acc += T[bi * SB + rr][kb * SB + k] * X[kb * SB + k][bj * SB + cc];
-            Y[b][rr][cc] = acc;
+                for (int y = 0; y < 2; ++y) u[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[y], fa[x], u[x][y], 0, 0, 0);
         }
-        __syncthreads();
-        for (int e = tid; e < nblk * SB * SB; e += 256) {
-            const int b = e / (SB * SB), rr = e % SB, cc = (e / SB) % SB;
-            const int bj = b, bi = b + dist;
-            double acc = 0.0;
 #pragma unroll
-            for (int k = 0; k < SB; ++k) acc += X[bi * SB + rr][bi * SB + k] * Y[b][k][cc];
-            X[bi * SB + rr][bj * SB + cc] = -acc;
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) c[x][y] -= u[x][y];
+        if (blockIdx.x != 0) {
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int y = 0; y < 2; ++y)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const int row = i0 + 16 * (wm + x) + lr, col = j0 + 16 * (wn + y) + lk + 4 * r;
+                        if (row < m && col < m) A[row + (size_t)lda * col] = c[x][y][r];
+                    }
+            return;
         }
-        __syncthreads();
+        lds_sync();   // the panel blocks are read: their LDS becomes T and X
     }
-    for (int e = tid; e < nb * nb; e += 256) {
-        const int r = e % nb, c = e / nb;
-        Winv[r + (size_t)ldw * c] = X[r][c];
+    Block& T = *(Block*)sm;
+    Block& X = *(Block*)(sm + CB * (CB + 1));
+    const int nb = min(CB, m - i0);
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = 16 * (wm + x) + lr, col = 16 * (wn + y) + lk + 4 * r;
+                T[row][col] = row < nb && col < nb ? c[x][y][r] : (row == col ? 1.0 : 0.0);
+            }
+    lds_sync();
+    chol_block(T, X, rd, i0, info);
+    double* Wd = W + i0 + (size_t)ldw * i0;
+    for (int e = threadIdx.x; e < CB * CB; e += 256) {
+        const int r = e % CB, cc = e / CB;
+        if (r < nb && cc < nb) Wd[r + (size_t)ldw * cc] = r >= cc ? X[r][cc] : 0.0;
     }
 }
 
-// dst[i + ldd j] = src[i + lds j], i < rows, j < cols
-__global__ void k_copy2d(const double* __restrict__ src, int lds, double* __restrict__ dst, int ldd, int rows,
-                         int cols)
+// W = L^-1 of the m x m matrix A = L L^T (lower triangle read; A is scratch
+// afterwards): the diagonal blocks' inverses from the factorisation's steps,
+// then W21 = -W22 (L21 W11) for pairs of neighbouring diagonal blocks of 64,
+// 128, 256, ... rows, two batched products per size.  W's entries above its
+// 64 x 64 diagonal blocks are not written; Lb, T: m x m scratch.
+// *info (device, cleared by the caller): the 1-based column of the first
+// non-positive pivot.
+static void chol_factor(hipStream_t st, double* A, int lda, int m, double* W, double* Lb, double* T, int* info)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
-    if (i < rows && j < cols) dst[i + (size_t)ldd * j] = src[i + (size_t)lds * j];
-}
-
-// Recursive Cholesky of the n x n block at (koff, koff) of A (lower triangle),
-// which also forms W = L^-1 of that block (W's strict upper triangle must hold
-// zeros on entry).  With L = [L11 0; L21 L22] and W = L^-1 = [W11 0; W21 W22]:
-//   L21 = A21 W11^T,  A22 -= L21 L21^T,  W21 = -W22 (L21 W11),
-// halves split at multiples of CB, the leaves the diagonal-block kernel: the
-// work between leaves is large GEMMs on the matrix cores (the triangular
-// factors' zero halves skipped).  T: scratch of n/2 x n/2 at least.
-static void chol_rec(hipStream_t st, double* A, int lda, double* W, int ldw, int koff, int n, double* T, int* info)
-{
-    if (n <= CB) {
-        k_chol_diag<<<1, 256, 0, st>>>(A, lda, koff, n, W + koff + (size_t)ldw * koff, ldw, info);
-        ILH_HIP(hipGetLastError());
-        return;
+    const int nbk = (m + CB - 1) / CB;
+    for (int k = -1; k < nbk - 1; ++k) {
+        const int t = nbk - 1 - k;
+        k_chol_step<<<k < 0 ? 1 : t * (t + 1) / 2, 256, 0, st>>>(A, lda, m, k, W, m, Lb, m, info);
     }
-    const int n1 = ((n + 1) / 2 + CB - 1) / CB * CB, n2 = n - n1;
-    chol_rec(st, A, lda, W, ldw, koff, n1, T, info);
-    double* A21 = A + (koff + n1) + (size_t)lda * koff;
-    double* A22 = A + (koff + n1) + (size_t)lda * (koff + n1);
-    const double* W11 = W + koff + (size_t)ldw * koff;
-    double* W21 = W + (koff + n1) + (size_t)ldw * koff;
-    const double* W22 = W + (koff + n1) + (size_t)ldw * (koff + n1);
-    dgemm(st, 0, 1, n2, n1, n1, 1.0, A21, lda, W11, ldw, 0.0, T, n2, false, TRI_B_UPPER);   // L21
-    k_copy2d<<<dim3((n2 + 255) / 256, n1), 256, 0, st>>>(T, n2, A21, lda, n2, n1);
     ILH_HIP(hipGetLastError());
-    dgemm(st, 0, 1, n2, n2, n1, -1.0, A21, lda, A21, lda, 1.0, A22, lda, true);
-    chol_rec(st, A, lda, W, ldw, koff + n1, n2, T, info);
-    dgemm(st, 0, 0, n2, n1, n1, 1.0, A21, lda, W11, ldw, 0.0, T, n2, false, TRI_B_LOWER);   // L21 W11
-    dgemm(st, 0, 0, n2, n1, n2, -1.0, W22, ldw, T, n2, 0.0, W21, ldw, false, TRI_A_LOWER);
+    for (int s = CB; s < m; s *= 2) {
+        const int pairs = (m - s + 2 * s - 1) / (2 * s);
+        const size_t dd = (size_t)2 * s * (m + 1), off = s;   // from one pair's blocks to the next; row offset of 21
+        GemmBatch bt;
+        bt.sa = bt.sb = bt.sc = dd;
+        bt.m_total = m - s;
+        bt.m_step = 2 * s;
+        const dim3 grid((std::min(s, m - s) + GT - 1) / GT, s / GT, pairs);
+        // T21 = L21 W11
+        k_dgemm<0, 0, true, EPI_NONE><<<grid, 256, 0, st>>>(std::min(s, m - s), s, s, 1.0, Lb + off, m, W, m, T + off, m,
+                                                           TRI_B_LOWER, bt, GemmEpi());
+        // W21 = -W22 T21
+        bt.k_is_m = 1;
+        k_dgemm<0, 0, true, EPI_NONE><<<grid, 256, 0, st>>>(std::min(s, m - s), s, s, -1.0, W + off + (size_t)m * s, m,
+                                                           T + off, m, W + off, m, TRI_A_LOWER, bt, GemmEpi());
+    }
+    ILH_HIP(hipGetLastError());
 }
 
-// Cholesky of the n x n matrix A (lower triangle, leading dimension lda):
-// W (n x n, leading dimension n) receives L^-1; A's diagonal blocks hold L's,
-// the rest of A is scratch afterwards.  Returns 0, or the 1-based column of
-// the first non-positive pivot.
-int chol_factor(ilh_plan* pl, double* A, int n, int lda, double* W, double* T, int* info_dev)
+// ---------------------------------------- products of W with a few vectors
+// Y[r + ldy v] = sum_{k <= r} W[r + m k] X[k + ldx v] - 2 u[r] s[v]  (u may be
+// null), v < NV: one work-group of 16 waves per 16 rows; a wave takes four
+// columns of 16 rows at a time, every 64th, and the 64 partial sums are added
+// in a fixed order.  (One wave per 64 rows and column: 79 us at m = 1884, two
+// vectors, too few work-groups and loads in flight.)
+template <int NV>
+__global__ void __launch_bounds__(1024) k_wmv(const double* __restrict__ W, int m, const double* __restrict__ X, int ldx,
+                                              const double* __restrict__ u, const double* __restrict__ s,
+                                              double* __restrict__ Y, int ldy)
 {
-    hipStream_t st = pl->ctx->stream;
-    ILH_HIP(hipMemsetAsync(info_dev, 0, sizeof(int), st));
-    ILH_HIP(hipMemsetAsync(W, 0, sizeof(double) * (size_t)n * n, st));
-    chol_rec(st, A, lda, W, n, 0, n, T, info_dev);
-    int h = 0;
-    ILH_HIP(hipMemcpyAsync(&h, info_dev, sizeof(int), hipMemcpyDeviceToHost, st));
-    ILH_HIP(hipStreamSynchronize(st));
-    return h;
+    __shared__ double part[NV][64][17];
+    const int tid = threadIdx.x, lr = tid & 15, kq = tid >> 4;   // kq: column of the round, 0..63
+    const int r = blockIdx.x * 16 + lr, rc = min(r, m - 1), kend = min(m, (int)(blockIdx.x * 16 / 64 + 1) * 64);
+    double acc[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) acc[v] = 0.0;
+#pragma unroll 8
+    for (int k = kq; k < kend; k += 64) {
+        const double w = W[rc + (size_t)m * k];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) acc[v] = __builtin_fma(w, X[k + (size_t)ldx * v], acc[v]);
+    }
+#pragma unroll
+    for (int v = 0; v < NV; ++v) part[v][kq][lr] = acc[v];
+    __syncthreads();
+    if (tid < 16 * NV) {
+        const int v = tid >> 4;
+        double t = 0.0;
+        for (int q = 0; q < 64; ++q) t += part[v][q][lr];
+        if (r < m) Y[r + (size_t)ldy * v] = u ? t - 2.0 * u[r] * s[v] : t;
+    }
 }
 
-// X <- (L L^T)^-1 X = W^T (W X) (X n x nrhs, leading dimension ldx; T n x nrhs scratch)
-void chol_solve(ilh_plan* pl, const double* W, int n, double* X, int ldx, int nrhs, double* T)
+// z_v[p] = sum_{k >= p} W[k + m p] T[k + ldt v], v < NV, one wave per column
+// p; written as Z[p + ldz v], or (wt given) through the deflated solve's last
+// step, Out[v + ldo (p + 1)] = (z - a[v] wt[p] - 2 b[v] w1[p]) / (c d[p + 1]).
+template <int NV>
+__global__ void __launch_bounds__(256) k_wtmv(const double* __restrict__ W, int m, const double* __restrict__ T, int ldt,
+                                              double* __restrict__ Z, int ldz, const double* __restrict__ a,
+                                              const double* __restrict__ b, const double* __restrict__ wt,
+                                              const double* __restrict__ w1, const double* __restrict__ d, double c)
 {
-    hipStream_t st = pl->ctx->stream;
-    if (n <= 0 || nrhs <= 0) return;
-    dgemm(st, 0, 0, n, nrhs, n, 1.0, W, n, X, ldx, 0.0, T, n, false, TRI_A_LOWER);
-    dgemm(st, 1, 0, n, nrhs, n, 1.0, W, n, T, n, 0.0, X, ldx, false, TRI_A_UPPER);
+    const int p = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (p >= m) return;
+    const double* col = W + (size_t)m * p;
+    double acc[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) acc[v] = 0.0;
+#pragma unroll 8
+    for (int k = p + lane; k < m; k += 64) {
+        const double w = col[k];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) acc[v] = __builtin_fma(w, T[k + (size_t)ldt * v], acc[v]);
+    }
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        for (int off = 32; off > 0; off >>= 1) acc[v] += __shfl_xor(acc[v], off, 64);
+        if (lane == 0) {
+            if (wt) Z[v + (size_t)ldz * (p + 1)] = (acc[v] - a[v] * wt[p] - 2.0 * b[v] * w1[p]) / (c * d[p + 1]);
+            else Z[p + (size_t)ldz * v] = acc[v];
+        }
+    }
 }
 
 // --------------------------------------------------- deflated symmetric solve
 // w: the Householder vector of H = I - 2 w w^T with H (1/sqrt(n)) = e_1
-__global__ void k_house_vec(double* __restrict__ w, int n)
+// (and clears the pivot flag of the factorisation that follows)
+__global__ void k_house_vec(double* __restrict__ w, int n, int* __restrict__ info)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) *info = 0;
     if (i >= n) return;
     if (n == 1) {   // H = I
         w[0] = 0.0;
@@ -435,129 +696,167 @@ __global__ void k_rank2(double* __restrict__ A, int n, int lda, const double* __
     A[i + (size_t)lda * j] -= w[i] * p[j] + p[i] * w[j];
 }
 
-// r[j] = sum_{i < m} v[i] X[i + ldx j], one wave per column j
-__global__ void k_coldot(const double* __restrict__ v, const double* __restrict__ X, int m, int ldx, int ncols,
-                         double* __restrict__ r)
+// xt[0..m) = w1, xt[m..2m) = beta (columns of the products with W)
+__global__ void k_defl_vecs(const double* __restrict__ w, const double* __restrict__ A, int m, double* __restrict__ xt)
 {
-    const int j = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (j >= ncols) return;
-    const double* col = X + (size_t)ldx * j;
-    double s = 0.0;
-    for (int i = lane; i < m; i += 64) s += v[i] * col[i];
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if (lane == 0) r[j] = s;
-}
-
-// X[i + ldx j] += c a[i] b[j]  (i < m)
-__global__ void k_rank1(double* __restrict__ X, int m, int ldx, double c, const double* __restrict__ a,
-                        const double* __restrict__ b)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= m) return;
-    X[i + (size_t)ldx * j] += c * a[i] * b[j];
+    xt[i] = w[1 + i];
+    xt[m + i] = A[1 + i];
 }
 
-// rows 1..m of X -= wt y1^T, y1 = row 0 of X (not written here)
-__global__ void k_rank1_row(double* __restrict__ X, int ldx, int m, const double* __restrict__ wt)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
-    if (i >= m) return;
-    X[1 + i + (size_t)ldx * j] -= wt[i] * X[(size_t)ldx * j];
-}
-
-// first row of the deflated solve: X[0, j] = (X[0, j] - r[j]) / sigma
-__global__ void k_first_row(double* __restrict__ X, int ldx, int ncols, const double* __restrict__ r,
-                            const double* __restrict__ sig)
-{
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= ncols) return;
-    X[(size_t)ldx * j] = (X[(size_t)ldx * j] - r[j]) / sig[0];
-}
-
-// sigma = alpha - beta . wt  (alpha = A[0,0], beta = A[1:, 0], wt = Mt^-1 beta)
-__global__ void __launch_bounds__(1024) k_sigma(const double* __restrict__ A, const double* __restrict__ wt, int m,
+// sig = {alpha - beta . wt, w1 . wt, w1 . ut}
+__global__ void __launch_bounds__(1024) k_sigma(const double* __restrict__ A, const double* __restrict__ xt,
+                                                const double* __restrict__ ut, const double* __restrict__ wt, int m,
                                                 double* __restrict__ sig)
 {
-    __shared__ double red[1024];
-    double s = 0.0;
-    for (int i = threadIdx.x; i < m; i += 1024) s += A[1 + i] * wt[i];
-    red[threadIdx.x] = s;
+    __shared__ double red[3][1024];
+    double s[3] = {0.0, 0.0, 0.0};
+    for (int i = threadIdx.x; i < m; i += 1024) {
+        s[0] += xt[m + i] * wt[i];
+        s[1] += xt[i] * wt[i];
+        s[2] += xt[i] * ut[i];
+    }
+    for (int v = 0; v < 3; ++v) red[v][threadIdx.x] = s[v];
     __syncthreads();
     for (int off = 512; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
+        if ((int)threadIdx.x < off)
+            for (int v = 0; v < 3; ++v) red[v][threadIdx.x] += red[v][threadIdx.x + off];
         __syncthreads();
     }
-    if (threadIdx.x == 0) sig[0] = A[0] - red[0];
+    if (threadIdx.x == 0) {
+        sig[0] = A[0] - red[0][0];
+        sig[1] = red[1][0];
+        sig[2] = red[2][0];
+    }
 }
 
-bool sym_factor(ilh_plan* pl, SymFactor& F, int n)
+bool sym_factor(ilh_plan* pl, SymFactor& F, int n, double* scratch)
 {
     hipStream_t st = pl->ctx->stream;
     F.n = n;
-    const int m = n - 1;
+    F.ok = false;
+    const int m = n - 1, mc = std::max(m, 1);
     F.w.ensure(sizeof(double) * (size_t)n);
-    F.vec.ensure(sizeof(double) * (size_t)2 * n + 8);
-    F.W.ensure(sizeof(double) * (size_t)std::max(m, 1) * std::max(m, 1));
-    F.T.ensure(sizeof(double) * ((size_t)std::max(m, 2) / 2 + CB) * ((size_t)std::max(m, 2) / 2 + CB));
-    F.info.ensure(sizeof(int));
+    F.vec.ensure(sizeof(double) * (size_t)(2 * n + 6 * mc));
+    F.W.ensure(sizeof(double) * (size_t)mc * mc);
+    F.T.ensure(sizeof(double) * (size_t)mc * n);   // also the product W B of a full solve
+    F.info.ensure(4 * sizeof(double));   // {sigma, w1.wt, w1.ut}, then the pivot flag
     double* A = F.A.as<double>();
     double* w = F.w.as<double>();
     double* y = F.vec.as<double>();
     double* p = y + n;
-    k_house_vec<<<(n + 255) / 256, 256, 0, st>>>(w, n);
+    double *xt = F.xt(), *wx = F.ww(), *zt = F.ut();
+    double* sig = F.info.as<double>();
+    int* info = (int*)(sig + 3);
+    k_house_vec<<<(n + 255) / 256, 256, 0, st>>>(w, n, info);
     k_symv<<<(n + 3) / 4, 256, 0, st>>>(A, n, n, w, y);
     k_house_p<<<1, 1024, 0, st>>>(w, y, n, p);
     k_rank2<<<dim3((n + 255) / 256, n), 256, 0, st>>>(A, n, n, w, p);
     ILH_HIP(hipGetLastError());
     if (m > 0) {
-        const int bad = chol_factor(pl, A + 1 + (size_t)n, m, n, F.W.as<double>(), F.T.as<double>(), F.info.as<int>());
-        if (bad) return false;
+        chol_factor(st, A + 1 + (size_t)n, n, m, F.W.as<double>(), scratch, F.T.as<double>(), info);
+        k_defl_vecs<<<(m + 255) / 256, 256, 0, st>>>(w, A, m, xt);
+        k_wmv<2><<<(m + 15) / 16, 1024, 0, st>>>(F.W.as<double>(), m, xt, m, nullptr, nullptr, wx, m);
+        k_wtmv<2><<<(m + 3) / 4, 256, 0, st>>>(F.W.as<double>(), m, wx, m, zt, m, nullptr, nullptr, nullptr, nullptr,
+                                               nullptr, 1.0);
     }
-    // wt = Mt^-1 beta, sigma = alpha - beta . wt
-    F.wt.ensure(sizeof(double) * (size_t)std::max(m, 1));
-    if (m > 0) {
-        ILH_HIP(hipMemcpyAsync(F.wt.p, A + 1, sizeof(double) * m, hipMemcpyDeviceToDevice, st));
-        chol_solve(pl, F.W.as<double>(), m, F.wt.as<double>(), m, 1, F.T.as<double>());
-    }
-    F.sig.ensure(sizeof(double));
-    k_sigma<<<1, 1024, 0, st>>>(A, F.wt.as<double>(), m, F.sig.as<double>());
+    k_sigma<<<1, 1024, 0, st>>>(A, xt, F.ut(), F.wt(), m, sig);
     ILH_HIP(hipGetLastError());
-    double sig = 0.0;
-    ILH_HIP(hipMemcpyAsync(&sig, F.sig.p, sizeof(double), hipMemcpyDeviceToHost, st));
+    double h[4];
+    ILH_HIP(hipMemcpyAsync(h, sig, sizeof(h), hipMemcpyDeviceToHost, st));
     ILH_HIP(hipStreamSynchronize(st));
-    if (!(sig != 0.0) || !std::isfinite(sig)) return false;
+    int bad;
+    std::memcpy(&bad, h + 3, sizeof(bad));
+    if (bad || !(h[0] != 0.0) || !std::isfinite(h[0])) return false;
     F.ok = true;
     return true;
 }
 
-// Minv[q + ld p] = X[q + n p] / (c d[p]) for q < n, 0 for n <= q < ld: the
-// row-major inverse (M diag(c d))^-1 = diag(1 / (c d)) M^-1 from X = M^-1
-// (symmetric, so its row p is read along its column p, coalesced)
-__global__ void k_rows_scaled(const double* __restrict__ X, int n, const double* __restrict__ d, double c,
-                              double* __restrict__ Minv, int ld)
+// The scalars of each column j of the deflated solve M^-1 B (B n x ncols), one
+// wave per column:  r = w . B, y1 = (X'0 - wt . X'1) / sigma and
+// t = w . [y1; Z - wt y1] with X' = B - 2 w r, Z = Mt^-1 X'1 (w1 . Z = ut . X'1),
+// and the solution's first row, Out[j] = (y1 - 2 w0 t) / (c d0).
+__global__ void __launch_bounds__(256) k_defl_cols(const double* __restrict__ w, const double* __restrict__ wt,
+                                                   const double* __restrict__ ut, const double* __restrict__ sig,
+                                                   const double* B, int n, int ncols, double* __restrict__ rv,
+                                                   double* __restrict__ y1v, double* __restrict__ tv, double* Out,
+                                                   const double* __restrict__ d, double c)
 {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x, p = blockIdx.y;
-    if (q >= ld) return;
-    Minv[q + (size_t)ld * p] = q < n ? X[q + (size_t)n * p] / (c * d[p]) : 0.0;
+    const int j = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (j >= ncols) return;
+    const double* col = B + (size_t)n * j;
+    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+#pragma unroll 4
+    for (int i = 1 + lane; i < n; i += 64) {
+        const double b = col[i];
+        s0 = __builtin_fma(w[i], b, s0);
+        s1 = __builtin_fma(wt[i - 1], b, s1);
+        s2 = __builtin_fma(ut[i - 1], b, s2);
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        s0 += __shfl_xor(s0, off, 64);
+        s1 += __shfl_xor(s1, off, 64);
+        s2 += __shfl_xor(s2, off, 64);
+    }
+    if (lane == 0) {
+        const double w0 = w[0], b0 = col[0];
+        const double r = s0 + w0 * b0;
+        const double y1 = ((b0 - 2.0 * w0 * r) - (s1 - 2.0 * sig[1] * r)) / sig[0];
+        const double t = w0 * y1 + (s2 - 2.0 * sig[2] * r) - sig[1] * y1;
+        rv[j] = r;
+        y1v[j] = y1;
+        tv[j] = t;
+        Out[j] = (y1 - 2.0 * w0 * t) / (c * d[0]);
+    }
 }
 
-// X[i + n j] /= c d[i]  (rows scaled: diag(1 / (c d)) X)
-__global__ void k_scale_rows(double* __restrict__ X, int n, int ncols, const double* __restrict__ d, double c)
+// Out[j + ldo p] = (M^-1 B)[p, j] / (c d[p]) for B (n x ncols, leading
+// dimension n): the rows of diag(1 / (c d)) M^-1 B, each contiguous.  The two
+// reflections and the first coordinate's elimination are rank-one and rank-two
+// corrections of the products with W, applied as these are written, so the
+// columns are read once for their scalars and once by W B.  A single column
+// goes through the vector products instead of 64-wide tiles.  Out may be B
+// when ncols = ldo = 1.
+void sym_solve_rows(ilh_plan* pl, SymFactor& F, const double* B, int ncols, const double* d, double c, double* Out,
+                    int ldo)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
-    if (i >= n || j >= ncols) return;
-    X[i + (size_t)n * j] /= c * d[i];
-}
-
-void scale_rows_inv(hipStream_t st, double* X, int n, int ncols, const double* d, double c)
-{
-    if (n <= 0 || ncols <= 0) return;
-    k_scale_rows<<<dim3((n + 255) / 256, ncols), 256, 0, st>>>(X, n, ncols, d, c);
+    if (!F.ok) fail(ILH_ERR_STATE, "symmetric factor not built");
+    if (ncols <= 0) return;
+    hipStream_t st = pl->ctx->stream;
+    const int n = F.n, m = n - 1;
+    F.r.ensure(sizeof(double) * (size_t)3 * ncols);
+    double *r = F.r.as<double>(), *y1 = r + ncols, *t = y1 + ncols;
+    const double* w = F.w.as<double>();
+    k_defl_cols<<<(ncols + 3) / 4, 256, 0, st>>>(w, F.wt(), F.ut(), F.info.as<double>(), B, n, ncols, r, y1, t, Out, d, c);
+    ILH_HIP(hipGetLastError());
+    if (m <= 0) return;
+    const double* W = F.W.as<double>();
+    F.T.ensure(sizeof(double) * (size_t)m * std::max(ncols, 1));
+    double* T = F.T.as<double>();
+    if (ncols == 1) {
+        k_wmv<1><<<(m + 15) / 16, 1024, 0, st>>>(W, m, B + 1, n, F.ww(), r, T, m);
+        k_wtmv<1><<<(m + 3) / 4, 256, 0, st>>>(W, m, T, m, Out, ldo, y1, t, F.wt(), w + 1, d, c);
+    } else {
+        GemmEpi e1, e2;
+        e1.u = F.ww();
+        e1.v = r;
+        k_dgemm<0, 0, true, EPI_RANK1><<<dim3((m + GT - 1) / GT, (ncols + GT - 1) / GT), 256, 0, st>>>(
+            m, ncols, m, 1.0, W, m, B + 1, n, T, m, TRI_A_LOWER, GemmBatch(), e1);
+        e2.a = y1;
+        e2.b = t;
+        e2.wt = F.wt();
+        e2.w1 = w + 1;
+        e2.d = d + 1;
+        e2.c = c;
+        k_dgemm<1, 0, true, EPI_DEFLATE><<<dim3((ncols + GT - 1) / GT, (m + GT - 1) / GT), 256, 0, st>>>(
+            ncols, m, m, 1.0, T, m, W, m, Out + ldo, ldo, TRI_B_LOWER, GemmBatch(), e2);
+    }
     ILH_HIP(hipGetLastError());
 }
 
-// Minv (row-major, leading dimension solve_ld(n)) = (M diag(c d))^-1 for the
-// factor of sym_factor
+// Minv (row-major, leading dimension solve_ld(n), the padding columns zero) =
+// (M diag(c d))^-1 for the factor of sym_factor
 __global__ void k_identity_cm(double* __restrict__ A, int n)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
@@ -565,49 +864,29 @@ __global__ void k_identity_cm(double* __restrict__ A, int n)
     A[i + (size_t)n * j] = i == j ? 1.0 : 0.0;
 }
 
+__global__ void k_zero_pad(double* __restrict__ A, int n, int ld)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, pad = ld - n;
+    if (i < n * pad) A[n + i % pad + (size_t)ld * (i / pad)] = 0.0;
+}
+
+void zero_pad_columns(hipStream_t st, double* A, int n, int ld)
+{
+    if (ld <= n || n <= 0) return;
+    k_zero_pad<<<((unsigned)n * (ld - n) + 255) / 256, 256, 0, st>>>(A, n, ld);
+    ILH_HIP(hipGetLastError());
+}
+
 void sym_inverse_rowmajor(ilh_plan* pl, SymFactor& F, const double* d, double c, double* Minv)
 {
     hipStream_t st = pl->ctx->stream;
     const int n = F.n, ld = solve_ld(n);
-    DevBuf X;
-    X.ensure(sizeof(double) * (size_t)n * n);
-    k_identity_cm<<<dim3((n + 255) / 256, n), 256, 0, st>>>(X.as<double>(), n);
+    // A's storage holds the identity
+    k_identity_cm<<<dim3((n + 255) / 256, n), 256, 0, st>>>(F.A.as<double>(), n);
     ILH_HIP(hipGetLastError());
-    sym_solve(pl, F, X.as<double>(), n);
-    k_rows_scaled<<<dim3((ld + 255) / 256, n), 256, 0, st>>>(X.as<double>(), n, d, c, Minv, ld);
-    ILH_HIP(hipGetLastError());
-    ILH_HIP(hipStreamSynchronize(st));   // X is released on return
-}
-
-// X <- M^-1 X (n x nrhs, leading dimension n) for the factor of sym_factor
-void sym_solve(ilh_plan* pl, SymFactor& F, double* X, int nrhs)
-{
-    if (!F.ok) fail(ILH_ERR_STATE, "symmetric factor not built");
-    hipStream_t st = pl->ctx->stream;
-    const int n = F.n, m = n - 1;
-    F.r.ensure(sizeof(double) * (size_t)std::max(nrhs, 1));
-    double* r = F.r.as<double>();
-    const double* w = F.w.as<double>();
-    const dim3 g1((n + 255) / 256, nrhs);
-    // X' = H X
-    k_coldot<<<(nrhs + 3) / 4, 256, 0, st>>>(w, X, n, n, nrhs, r);
-    k_rank1<<<g1, 256, 0, st>>>(X, n, n, -2.0, w, r);
-    ILH_HIP(hipGetLastError());
-    const double* A = F.A.as<double>();
-    // rows 1.. : Mt^-1 X'[1:, :]
-    if (m > 0) {
-        F.T2.ensure(sizeof(double) * (size_t)m * nrhs);
-        chol_solve(pl, F.W.as<double>(), m, X + 1, n, nrhs, F.T2.as<double>());
-    }
-    // first row: y1 = (X'[0, :] - beta^T Mt^-1 X'[1:, :]) / sigma
-    k_coldot<<<(nrhs + 3) / 4, 256, 0, st>>>(A + 1, X + 1, m, n, nrhs, r);
-    k_first_row<<<(nrhs + 255) / 256, 256, 0, st>>>(X, n, nrhs, r, F.sig.as<double>());
-    // rows 1.. -= wt y1^T  (the first row of X now holds y1)
-    if (m > 0) k_rank1_row<<<dim3((m + 255) / 256, nrhs), 256, 0, st>>>(X, n, m, F.wt.as<double>());
-    // X = H X'
-    k_coldot<<<(nrhs + 3) / 4, 256, 0, st>>>(w, X, n, n, nrhs, r);
-    k_rank1<<<g1, 256, 0, st>>>(X, n, n, -2.0, w, r);
-    ILH_HIP(hipGetLastError());
+    sym_solve_rows(pl, F, F.A.as<double>(), n, d, c, Minv, ld);
+    zero_pad_columns(st, Minv, n, ld);
+    ILH_HIP(hipStreamSynchronize(st));   // F may be released on return
 }
 
 }  // namespace ilh

@@ -186,6 +186,130 @@ __global__ void __launch_bounds__(AT * AT) k_assemble(const Term* __restrict__ T
     }
 }
 
+// K[p + ldk q] = factor * (E . kernel . D_s)[p, q]: an interpolation window
+// (one term, four taps a side) against surface_divergence!'s two terms, whose
+// windows nearly coincide.  With b the corner one cell before the point's
+// plain DDF window, the first term's windows are five taps from b_x + 0 or 1
+// on and the plain four in y, the second's the plain four in x and five taps
+// from b_y + 0 or 1 on; so both correlations with the point p live in one
+// 9 x 9 window of the kernel, the plain axes in its middle 7.  One pass over
+// that window serves both terms: 77 table reads and 142 multiply-adds per
+// entry instead of the general form's 162 and 180, LDS reads being what bounds
+// it (N = 1885: 137 us, 167 us in the general form).  Tiles and staging as in k_assemble.
+__global__ void __launch_bounds__(AT * AT) k_assemble_ds(const Term* __restrict__ TA, const Term* __restrict__ TB, int N,
+                                                         const double* __restrict__ G, int Tn, double factor,
+                                                         double* __restrict__ K, int ldk)
+{
+    __shared__ Term sa[AT], sb[AT * 2];
+    __shared__ double sG[GBOX];
+    __shared__ int sbox[5];
+    const int p0 = blockIdx.x * AT, q0 = blockIdx.y * AT;
+    const int tid = threadIdx.x + AT * threadIdx.y;
+    if (tid < AT) {
+        if (p0 + tid < N) sa[tid] = TA[p0 + tid];
+    } else if (tid >= 64 && tid < 64 + 2 * AT) {
+        const int k = tid - 64;
+        if (q0 + k / 2 < N) sb[k] = TB[2 * (size_t)q0 + k];
+    }
+    __syncthreads();
+    if (tid < 64) {
+        // extents of the window bases: lanes < 16 the A terms, lanes 32..47 the corners b
+        int lo[4] = {1 << 30, 1 << 30, 1 << 30, 1 << 30}, hi[4] = {-(1 << 30), -(1 << 30), -(1 << 30), -(1 << 30)};
+        if (tid < AT) {
+            if (p0 + tid < N) { lo[0] = hi[0] = sa[tid].bx; lo[1] = hi[1] = sa[tid].by; }
+        } else if (tid >= 32 && tid < 32 + AT) {
+            const int k = tid - 32;
+            if (q0 + k < N) { lo[2] = hi[2] = sb[2 * k + 1].bx - 1; lo[3] = hi[3] = sb[2 * k].by - 1; }
+        }
+        for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                lo[c] = min(lo[c], __shfl_xor(lo[c], off, 64));
+                hi[c] = max(hi[c], __shfl_xor(hi[c], off, 64));
+            }
+        if (tid == 0) {
+            // offsets a - b - 5 ... a - b + 3
+            const int x0 = lo[0] - hi[2] - 5, x1 = hi[0] - lo[2] + 3, y0 = lo[1] - hi[3] - 5, y1 = hi[1] - lo[3] + 3;
+            const int bw = x1 - x0 + 1, bh = y1 - y0 + 1;
+            sbox[0] = bw > 0 && bh > 0 && (long)bw * bh <= GBOX ? 1 : -1;
+            sbox[1] = x0;
+            sbox[2] = y0;
+            sbox[3] = bw;
+            sbox[4] = bh;
+        }
+    }
+    __syncthreads();
+    const bool boxed = sbox[0] > 0;
+    const int bx0 = sbox[1], by0 = sbox[2], bw = sbox[3], bh = sbox[4];
+    if (boxed) {
+        for (int e = tid; e < bw * bh; e += AT * AT) {
+            const int ix = abs(bx0 + e % bw), iy = abs(by0 + e / bw);
+            sG[e] = (ix < Tn && iy < Tn) ? G[(size_t)Tn * iy + ix] : 0.0;
+        }
+    }
+    __syncthreads();
+    const int p = p0 + threadIdx.x, q = q0 + threadIdx.y;
+    if (p >= N || q >= N) return;
+    const Term &a = sa[threadIdx.x], &t1 = sb[2 * threadIdx.y], &t2 = sb[2 * threadIdx.y + 1];
+    // the correlations along x are kept, those along y formed row by row
+    double cx1[9], cx2[9];   // cx2: entries 1..7
+    const bool s1 = t1.bx == t2.bx, s2 = t2.by == t1.by;   // five-tap windows from b + 1 on (else b)
+    {
+        double ex[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) ex[u] = 0.0;
+#pragma unroll
+        for (int u = 0; u < 9; ++u) cx2[u] = 0.0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+#pragma unroll
+            for (int k = 0; k < 5; ++k) ex[i - k + 4] = __builtin_fma(a.wx[i], t1.wx[k], ex[i - k + 4]);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) cx2[i - k + 4] = __builtin_fma(a.wx[i], t2.wx[k], cx2[i - k + 4]);
+        }
+#pragma unroll
+        for (int u = 0; u < 9; ++u) cx1[u] = s1 ? (u < 8 ? ex[u] : 0.0) : (u > 0 ? ex[u - 1] : 0.0);
+    }
+    const int dx = a.bx - (t2.bx - 1) - 5, dy = a.by - (t1.by - 1) - 5;
+    double sum1 = 0.0, sum2 = 0.0;
+    auto row = [&](double c1, double c2, const double* g) {
+        double r1 = 0.0, r2 = 0.0;
+#pragma unroll
+        for (int u = 0; u < 9; ++u) r1 = __builtin_fma(cx1[u], g[u], r1);
+#pragma unroll
+        for (int u = 1; u < 8; ++u) r2 = __builtin_fma(cx2[u], g[u], r2);
+        sum1 = __builtin_fma(c1, r1, sum1);
+        sum2 = __builtin_fma(c2, r2, sum2);
+    };
+    const int sy = s2 ? 1 : 0;
+    const int at = bw * (dy - by0) + (dx - bx0);
+#pragma unroll 1
+    for (int v = 0; v < 9; ++v) {
+        // tap pairs i - k = v - 4 of the plain windows, i - k = v - 5 + sy with the five taps
+        double c1 = 0.0, c2 = 0.0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int k1 = i - v + 4, k2 = i - v + 5 - sy;
+            if (k1 >= 0 && k1 < 4) c1 = __builtin_fma(a.wy[i], t1.wy[k1], c1);
+            if (k2 >= 0 && k2 < 5) c2 = __builtin_fma(a.wy[i], t2.wy[k2], c2);
+        }
+        double g[9];
+        if (boxed) {
+#pragma unroll
+            for (int u = 0; u < 9; ++u) g[u] = sG[at + bw * v + u];
+        } else {
+            const int jj = abs(dy + v);
+#pragma unroll
+            for (int u = 0; u < 9; ++u) {
+                const int ii = abs(dx + u);
+                g[u] = ii < Tn && jj < Tn ? G[(size_t)Tn * jj + ii] : 0.0;
+            }
+        }
+        row(c1, c2, g);
+    }
+    K[p + (size_t)ldk * q] = factor * (a.coef * (t1.coef * sum1 + t2.coef * sum2));
+}
+
 static void launch_assemble(ilh_plan* pl, int opA, int opB, const double* tab, int Tn, double factor, bool delta,
                             double* K, int ldk, bool rowmajor)
 {
@@ -202,7 +326,9 @@ static void launch_assemble(ilh_plan* pl, int opA, int opB, const double* tab, i
                      (opA == OP_E_PRIMAL && opB == OP_E_PRIMAL) || (opA == OP_E_DUAL && opB == OP_E_DUAL);
     const int dl = delta ? 1 : 0;
     hipStream_t st = pl->ctx->stream;
-    if (rowmajor && sym)
+    if (!rowmajor && !delta && opA == OP_E_PRIMAL && opB == OP_DS)
+        k_assemble_ds<<<grid, dim3(AT, AT), 0, st>>>(A, B, N, tab, Tn, factor, K, ldk);
+    else if (rowmajor && sym)
         k_assemble<true, true><<<grid, dim3(AT, AT), 0, st>>>(A, ta, B, tb, N, tab, Tn, factor, dl, K, ldk);
     else if (rowmajor)
         k_assemble<true, false><<<grid, dim3(AT, AT), 0, st>>>(A, ta, B, tb, N, tab, Tn, factor, dl, K, ldk);
@@ -297,15 +423,6 @@ __global__ void __launch_bounds__(1024) k_panel(double* __restrict__ A, int n, i
         }
         __syncthreads();
     }
-}
-
-// Work-group barrier ordering LDS accesses only: outstanding global stores of
-// the calling waves need not complete (a plain __syncthreads waits for them).
-__device__ __forceinline__ void lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // max |value| over the work-group with the smallest row index among ties

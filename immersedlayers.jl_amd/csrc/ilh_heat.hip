@@ -313,7 +313,7 @@ static void schur_inverse(ilh_plan* pl, const std::vector<double>& K, bool ident
     SymFactor F;
     F.A.ensure(sizeof(double) * (size_t)N * N);
     build(OP_E_PRIMAL, F.A.as<double>());
-    if (sym_factor(pl, F, N)) {
+    if (sym_factor(pl, F, N, inv.as<double>())) {
         sym_inverse_rowmajor(pl, F, pl->ds.as<double>(), 1.0 / (pl->g.dx * pl->g.dx), inv.as<double>());
         return;
     }

@@ -205,6 +205,7 @@ struct ilh_plan {
     ilh::DevBuf scratch_a, scratch_b;         // grid scratch
     ilh::DevBuf lu_tinv, lu_perm, lu_tmp, lu_pmap;   // LU scratch (block inverses, row permutations)
     SolveCache* dir = nullptr;                // Dirichlet
+    SolveCache* dir_spare = nullptr;          // the previous geometry's, its buffers kept for the next
     SolveCache* neu = nullptr;                // Neumann
     SolveCache* fac[6] = {};                  // ilh_schur_factor caches per kind
     StokesCache* sto = nullptr;               // Stokes flow (vector cache) solve matrices
@@ -393,36 +394,52 @@ void assemble_table(ilh_plan* pl, int opA, int opB, const double* tab, int Tn, d
                     double* K /* N x N col-major */);
 int  lu_factor(ilh_plan* pl, double* A, int n, int* piv_dev, int* info_dev);
 // C (M x Nc) = beta C + alpha opA(A) opB(B) on the FP64 matrix cores (ilh_chol.hip),
-// column-major, ta/tb = 1 for a transposed operand, beta 0 or 1; lower: only
-// the lower triangle of a square C is needed (ta = 0, tb = 1, beta = 1)
+// column-major, ta/tb = 1 for a transposed operand, beta 0 or 1;
 // tri: the K range of each tile restricted to a triangular operand's nonzero half
 enum { TRI_NONE = 0, TRI_A_LOWER = 1, TRI_A_UPPER = 2, TRI_B_LOWER = 3, TRI_B_UPPER = 4 };
 void dgemm(hipStream_t st, int ta, int tb, int M, int Nc, int K, double alpha, const double* A, int lda,
-           const double* B, int ldb, double beta, double* C, int ldc, bool lower = false, int tri = TRI_NONE);
-// Recursive Cholesky (ilh_chol.hip): W (n x n) = L^-1 for A = L L^T; 0 or the
-// first non-positive pivot.  chol_solve: X <- W^T W X.
-int  chol_factor(ilh_plan* pl, double* A, int n, int lda, double* W, double* T, int* info_dev);
-void chol_solve(ilh_plan* pl, const double* W, int n, double* X, int ldx, int nrhs, double* T);
+           const double* B, int ldb, double beta, double* C, int ldc, int tri = TRI_NONE);
 // A symmetric matrix M that is positive definite on the vectors orthogonal to
 // the constant one (the symmetrised Schur matrices E K E^T), factored as a
 // Householder-deflated Cholesky (ilh_chol.hip).  The caller fills A (n x n,
 // both triangles) and calls sym_factor; false: a non-positive pivot (the
-// caller falls back to LU).  sym_solve: X <- M^-1 X (n x nrhs, leading dim n).
+// caller falls back to LU).
 struct SymFactor {
     int n = 0;
     bool ok = false;
-    DevBuf A, W, T, T2, w, wt, vec, sig, r, info;
+    DevBuf A, W, T, w, vec, r, info;
+    // vec: n-vectors y, p (scratch), then of m = n - 1 entries each w1, beta,
+    // W w1, W beta, Mt^-1 w1, Mt^-1 beta
+    double* xt() const { return vec.as<double>() + 2 * n; }
+    double* ww() const { return xt() + 2 * (n - 1); }
+    double* ut() const { return xt() + 4 * (n - 1); }
+    double* wt() const { return xt() + 5 * (n - 1); }
 };
-bool sym_factor(ilh_plan* pl, SymFactor& F, int n);
-void sym_solve(ilh_plan* pl, SymFactor& F, double* X, int nrhs);
-// with S = M diag(c d): Minv = S^-1 row-major (leading dimension solve_ld(n)),
-// and X <- diag(1 / (c d)) X (n x ncols)
+// A is free for other use after it; scratch: n x n entries (the factor's
+// blocks below the diagonal ones while W = L^-1 is formed)
+bool sym_factor(ilh_plan* pl, SymFactor& F, int n, double* scratch);
+// with S = M diag(c d): the rows of S^-1 B (B n x ncols), row p at Out + ldo p
+// (Out may be B for one column and ldo = 1), and Minv = S^-1 row-major
+// (leading dimension solve_ld(n), padding columns zero)
+void sym_solve_rows(ilh_plan* pl, SymFactor& F, const double* B, int ncols, const double* d, double c, double* Out,
+                    int ldo);
 void sym_inverse_rowmajor(ilh_plan* pl, SymFactor& F, const double* d, double c, double* Minv);
-void scale_rows_inv(hipStream_t st, double* X, int n, int ncols, const double* d, double c);
+// columns [n, ld) of the n rows of a row-major matrix = 0
+void zero_pad_columns(hipStream_t st, double* A, int n, int ld);
 void lu_solve_multi(ilh_plan* pl, const double* LU, const int* piv, int n, double* B, int nrhs);
 // row-major solve matrices use a leading dimension padded to a multiple of 32
 inline int solve_ld(int n) { return (n + 31) / 32 * 32; }
 void transpose(hipStream_t st, const double* A, double* At, int rows, int cols, int ldt);
+// Work-group barrier ordering LDS accesses only: outstanding global stores
+// and loads of the calling waves need not complete (a plain __syncthreads
+// waits for them).
+__device__ __forceinline__ void lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // a.x b.x + a.y b.y with one explicit fused multiply-add, so that the rounding
 // is the same wherever the compiler places it
 __device__ __forceinline__ double dot2(double2 a, double2 b) { return __builtin_fma(a.x, b.x, a.y * b.y); }

@@ -1,0 +1,66 @@
+"""The deflated Cholesky of the symmetrised Schur matrix and the solve matrices
+made from it, at the edges of its 64-wide blocks and 16-wide sub-blocks, and
+again on the same plan after the points moved (its workspaces are kept).
+
+Bars: f 1e-10 and s 1e-10 (relative L2) against the oracle; the residual of
+S x = b within 1e-11 (a backward-stable solve leaves about cond(M)^(1/2) eps
+per block product, cond(M) < 1e6 here: 1e3 x 2.2e-16 x a few tens of products).
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+from conftest import rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def ring(N, spacing, dx, shift=0.003):
+    """N points on a circle `spacing` dx apart (at least 4 dx across), the grid around it."""
+    from ilhip import geometry as G
+    r = max(N * spacing * dx / (2 * np.pi), 2 * dx)
+    n = int(2 * r / dx) + 24
+    th = 2 * np.pi * np.arange(N) / N
+    s = G.Surface(r * np.cos(th) + shift, r * np.sin(th), np.cos(th), np.sin(th), np.full(N, 2 * np.pi * r / N),
+                  np.zeros(N, int))
+    return G.GridSpec(n + 1, n + 1, n // 2 + 1, n // 2 + 1, dx), s, th
+
+
+@pytest.mark.parametrize("N", [1, 2, 16, 17, 64, 65, 66, 128, 129, 130, 193, 321, 450])
+def test_factor_block_edges(ctx, N):
+    import ilhip
+    g, s, th = ring(N, 1.4, 0.02)
+    print("factor N", N, "grid", g.NX, flush=True)
+    c = ilhip.SurfaceScalarCache(s, g, ctx=ctx)
+    b = np.random.default_rng(N).standard_normal(N)
+    x = ilhip.SchurFactor(c).solve(b)
+    S = ilhip.create_RTLinvR(c)
+    assert rel_err(S @ x, b) < 1e-11
+    fp, fm = 0.3 + np.cos(th), np.sin(2 * th)
+    prob = ilhip.DirichletPoisson(c)
+    og = O.grid(g.NX, g.NY, g.I0x, g.I0y, g.dx)
+    for shift in (0.003, 0.011):
+        t = ring(N, 1.4, 0.02, shift)[1]
+        c.update_points(t)
+        f, sv = prob.solve(fp, fm, filter_power=0)
+        fr, sr = O.dirichlet_solve(og, O.Geometry(t.X, t.Y, t.nx, t.ny, t.ds), fp, fm)
+        assert rel_err(f.flat(), fr) < 1e-10
+        assert rel_err(sv.flat(), sr) < 1e-10
+
+
+@pytest.mark.parametrize("N,spacing,ddf", [(33, 1.4, "Roma"), (40, 6.0, "Yang3"), (50, 3.1, "Witchhat"),
+                                           (31, 2.0, "M4prime")])
+def test_double_layer_assembly(ctx, N, spacing, ddf):
+    """E L^-1 D_s for every DDF's window alignment, and for points so far
+    apart that a tile's kernel box does not fit in LDS (6 dx)."""
+    import ilhip
+    g, s, th = ring(N, spacing, 0.02)
+    kind = getattr(ilhip, ddf)
+    print("double layer N", N, "spacing", spacing, ddf, flush=True)
+    c = ilhip.SurfaceScalarCache(s, g, ctx=ctx, ddftype=kind)
+    fp = 0.3 + np.cos(th)
+    f, sv = ilhip.DirichletPoisson(c).solve(fp, filter_power=0)
+    og = O.grid(g.NX, g.NY, g.I0x, g.I0y, g.dx)
+    fr, sr = O.dirichlet_solve(og, O.Geometry(s.X, s.Y, s.nx, s.ny, s.ds), fp, ddf_kind=kind)
+    assert rel_err(f.flat(), fr) < 1e-10
+    assert rel_err(sv.flat(), sr) < 1e-10
