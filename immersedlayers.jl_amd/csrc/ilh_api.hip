@@ -437,9 +437,7 @@ int op_components(int op, int* gks)
     }
 }
 
-template <class T>
-static void scatter_op_t(ilh_plan* pl, int op, const T* amp, size_t amp_stride, int nb, T* out, size_t out_stride,
-                         const T* base = nullptr, double cb = 1.0)
+const RowBins* scatter_bins(ilh_plan* pl, int op)
 {
     const Term* t = get_terms(pl, op);
     int gks[4];
@@ -448,9 +446,18 @@ static void scatter_op_t(ilh_plan* pl, int op, const T* amp, size_t amp_stride, 
         for (int c = 0; c < nc; ++c) build_bins(pl, t, pl->N * op_terms_per_point(op), gks[c], pl->bins[op][c]);
         pl->bins_ok[op] = true;
     }
+    return pl->bins[op];
+}
+
+template <class T>
+static void scatter_op_t(ilh_plan* pl, int op, const T* amp, size_t amp_stride, int nb, T* out, size_t out_stride)
+{
+    const RowBins* bins = scatter_bins(pl, op);
+    int gks[4];
+    const int nc = op_components(op, gks);
     size_t off = 0;
     for (int c = 0; c < nc; ++c) {
-        scatter(pl, pl->bins[op][c], amp, amp_stride, nb, out + off, out_stride, base ? base + off : nullptr, cb);
+        scatter(pl, bins[c], amp, amp_stride, nb, out + off, out_stride);
         off += pl->g.n(gks[c]);
     }
 }
@@ -462,10 +469,6 @@ void scatter_op_multi(ilh_plan* pl, int op, const double* amp, size_t amp_stride
 }
 
 void scatter_op(ilh_plan* pl, int op, const double* amp, double* out) { scatter_op_t(pl, op, amp, 0, 1, out, 0); }
-void scatter_op_add(ilh_plan* pl, int op, const double* amp, const double* base, double c, double* out)
-{
-    scatter_op_t(pl, op, amp, 0, 1, out, 0, base, c);
-}
 void scatter_op(ilh_plan* pl, int op, const float* amp, float* out) { scatter_op_t(pl, op, amp, 0, 1, out, 0); }
 
 void gather_op_multi(ilh_plan* pl, int op, const double* field, size_t field_stride, int nb, double* out,

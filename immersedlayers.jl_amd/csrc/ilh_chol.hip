@@ -641,14 +641,15 @@ __global__ void __launch_bounds__(256) k_wtmv(const double* __restrict__ W, int 
 
 // --------------------------------------------------- deflated symmetric solve
 // w: the Householder vector of H = I - 2 w w^T with H (1/sqrt(n)) = e_1
-// (and clears the pivot flag of the factorisation that follows)
-__global__ void k_house_vec(double* __restrict__ w, int n, int* __restrict__ info)
+// (w = 0, H = I without deflation); clears the pivot flag of the factorisation
+// that follows
+__global__ void k_house_vec(double* __restrict__ w, int n, bool deflate, int* __restrict__ info)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i == 0) *info = 0;
     if (i >= n) return;
-    if (n == 1) {   // H = I
-        w[0] = 0.0;
+    if (n == 1 || !deflate) {
+        w[i] = 0.0;
         return;
     }
     const double u = 1.0 / sqrt((double)n);
@@ -731,7 +732,7 @@ __global__ void __launch_bounds__(1024) k_sigma(const double* __restrict__ A, co
     }
 }
 
-bool sym_factor(ilh_plan* pl, SymFactor& F, int n, double* scratch)
+bool sym_factor(ilh_plan* pl, SymFactor& F, int n, double* scratch, bool deflate)
 {
     hipStream_t st = pl->ctx->stream;
     F.n = n;
@@ -749,10 +750,12 @@ bool sym_factor(ilh_plan* pl, SymFactor& F, int n, double* scratch)
     double *xt = F.xt(), *wx = F.ww(), *zt = F.ut();
     double* sig = F.info.as<double>();
     int* info = (int*)(sig + 3);
-    k_house_vec<<<(n + 255) / 256, 256, 0, st>>>(w, n, info);
-    k_symv<<<(n + 3) / 4, 256, 0, st>>>(A, n, n, w, y);
-    k_house_p<<<1, 1024, 0, st>>>(w, y, n, p);
-    k_rank2<<<dim3((n + 255) / 256, n), 256, 0, st>>>(A, n, n, w, p);
+    k_house_vec<<<(n + 255) / 256, 256, 0, st>>>(w, n, deflate, info);
+    if (deflate) {
+        k_symv<<<(n + 3) / 4, 256, 0, st>>>(A, n, n, w, y);
+        k_house_p<<<1, 1024, 0, st>>>(w, y, n, p);
+        k_rank2<<<dim3((n + 255) / 256, n), 256, 0, st>>>(A, n, n, w, p);
+    }
     ILH_HIP(hipGetLastError());
     if (m > 0) {
         chol_factor(st, A + 1 + (size_t)n, n, m, F.W.as<double>(), scratch, F.T.as<double>(), info);

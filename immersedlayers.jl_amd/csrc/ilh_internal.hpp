@@ -243,8 +243,7 @@ void free_bins(RowBins& b);
 // batched over nb operands (grid.y): operand k reads amp + k amp_stride /
 // field + k field_stride and writes out + k out_stride
 template <class T>
-void scatter(ilh_plan* pl, const RowBins& bins, const T* amp, size_t amp_stride, int nb, T* out, size_t out_stride,
-             const T* base = nullptr, double c = 1.0);
+void scatter(ilh_plan* pl, const RowBins& bins, const T* amp, size_t amp_stride, int nb, T* out, size_t out_stride);
 // field: the operator's whole input (Nodes, Edges or EdgeGradient); each term
 // reads its component grid at Grid::offset(gk)
 template <class T>
@@ -372,8 +371,8 @@ const std::vector<BatchProb>& fused_probs(const FusedBatch* fb);
 // grid, gather E-type ops to the surface; inverse of a dense N x N matrix
 // (overwritten) into row-major Minv with leading dimension solve_ld(N)
 void scatter_op(ilh_plan* pl, int op, const double* amp, double* out);
-// out = base + c (op amp), one pass (base and out grid-sized, distinct)
-void scatter_op_add(ilh_plan* pl, int op, const double* amp, const double* base, double c, double* out);
+// the row bins of a scatter op, one per component grid (built on first use)
+const RowBins* scatter_bins(ilh_plan* pl, int op);
 void gather_op(ilh_plan* pl, int op, const double* field, double* out);
 // nb operands at once: amplitudes / fields k at a stride, outputs k at a stride
 void scatter_op_multi(ilh_plan* pl, int op, const double* amp, size_t amp_stride, int nb, double* out,
@@ -416,8 +415,9 @@ struct SymFactor {
     double* wt() const { return xt() + 5 * (n - 1); }
 };
 // A is free for other use after it; scratch: n x n entries (the factor's
-// blocks below the diagonal ones while W = L^-1 is formed)
-bool sym_factor(ilh_plan* pl, SymFactor& F, int n, double* scratch);
+// blocks below the diagonal ones while W = L^-1 is formed).  deflate = false:
+// M is positive definite outright and is factored without the reflection.
+bool sym_factor(ilh_plan* pl, SymFactor& F, int n, double* scratch, bool deflate = true);
 // with S = M diag(c d): the rows of S^-1 B (B n x ncols), row p at Out + ldo p
 // (Out may be B for one column and ldo = 1), and Minv = S^-1 row-major
 // (leading dimension solve_ld(n), padding columns zero)

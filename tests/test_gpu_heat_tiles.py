@@ -1,0 +1,52 @@
+"""Heat conduction on the tiled one-kernel filter and the packed stage inverses,
+at the edges of the 64 x 64 tiles and of the filter widths (8 to 16 taps a
+side, then the two-pass form), with a body 5 cells from the grid's edge, new
+boundary values between calls, and without bodies.
+
+Bar: 1e-11 (relative L2) against the oracle: stage matrices of condition < 50
+at these points and Fourier numbers, three solves and six filters a step, at
+most 5 steps: a few hundred roundings of 1e-16.
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+from conftest import rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,m,fo,N", [(63, 64, 0.02, 40), (64, 65, 0.1, 60), (129, 70, 0.25, 70), (100, 140, 0.45, 90),
+                                      (193, 128, 0.62, 120), (90, 91, 0.9, 64), (70, 129, 0.25, 0)])
+def test_heat_tiles(ctx, n, m, fo, N):
+    import ilhip
+    from ilhip import geometry as G
+    dx = 0.02
+    g = G.GridSpec(n + 1, m + 1, n // 2 + 1, m // 2 + 1, dx)
+    r = N * 1.4 * dx / (2 * np.pi)
+    th = 2 * np.pi * np.arange(N) / max(N, 1)
+    # leftmost point 5.3 cells from the grid's left edge, centre a little off the cells
+    cx, cy = g.x_primal()[0] + 5.3 * dx + r, 0.4 * dx
+    s = G.Surface(cx + r * np.cos(th), cy + r * np.sin(th), np.cos(th), np.sin(th), np.full(N, 1.4 * dx),
+                  np.zeros(N, int))
+    rng = np.random.default_rng(n)
+    T0 = rng.standard_normal((n, m))
+    print("heat tiles", n, m, "Fo", fo, "N", N, flush=True)
+    og = O.grid(g.NX, g.NY, g.I0x, g.I0y, dx)
+    geo = O.Geometry(s.X, s.Y, s.nx, s.ny, s.ds)
+    tp, tm = 1.0 + 0.3 * np.cos(th), 0.2 * np.sin(3 * th)
+    c = ilhip.SurfaceScalarCache(s, g, ctx=ctx)
+    heat = ilhip.DirichletHeatConduction(c, 1.0, fo * dx * dx, tp, tm)
+    T = ilhip.Nodes(ilhip.Primal, g, T0.copy())
+    ref = T0.ravel(order="F").copy()
+    for k, (a, b, steps) in enumerate(((tp, tm, 2), (tm, None, 1), (tp - tm, tp, 2))):
+        if k:
+            heat.set_boundary(a, b)
+        heat.advance(T, steps)
+        ref = O.heat_advance(og, geo, 1.0, fo * dx * dx, steps, ref, a, b if b is not None else np.zeros(N))
+        assert rel_err(T.flat(), ref) < 1e-11
+        if N:
+            Eb = ilhip.ScalarData(N)
+            ilhip.interpolate(Eb, T, c)
+            assert np.abs(Eb.flat() - 0.5 * (a + (0 if b is None else b))).max() < 1e-12
+    heat.close()
