@@ -313,13 +313,19 @@ static void load_points(ilh_plan* pl, const double* X, const double* Y, const do
     const int N = pl->N;
     if (N > 0 && (!X || !Y || !nx || !ny || !ds)) fail(ILH_ERR_ARG, "null geometry array");
     double mm = 1e300;
+    double ext[4] = {1e300, -1e300, 1e300, -1e300};
     for (int p = 0; p < N; ++p) {
         if (!std::isfinite(X[p]) || !std::isfinite(Y[p]) || !std::isfinite(nx[p]) || !std::isfinite(ny[p]) ||
             !std::isfinite(ds[p]))
             fail(ILH_ERR_NONFINITE, "non-finite surface geometry");
         const double xp = X[p] / pl->g.dx - (1.0 - pl->g.I0x), yp = Y[p] / pl->g.dx - (1.0 - pl->g.I0y);
         mm = std::min({mm, xp, (pl->g.NX - 2) - xp, yp, (pl->g.NY - 2) - yp});
+        ext[0] = std::min(ext[0], xp);
+        ext[1] = std::max(ext[1], xp);
+        ext[2] = std::min(ext[2], yp);
+        ext[3] = std::max(ext[3], yp);
     }
+    std::copy(ext, ext + 4, pl->ext);
     pl->min_margin = N > 0 ? (int)std::floor(mm) : 1 << 20;
     const size_t b = sizeof(double) * (size_t)std::max(1, N);
     pl->X.ensure(b);
@@ -1271,8 +1277,9 @@ extern "C" int ilh_dirichlet_solve_noalloc(ilh_plan* pl, const double* fp, const
             return;
         }
         unsigned char* base = (unsigned char*)scratch_ptr(pl->ctx->device);
-        if (!pl->conv_ok[GK_PRIMAL]) fail(ILH_ERR_STATE, "the plan's LGF spectrum is not built yet");
-        const ConvPlan& C = pl->conv[GK_PRIMAL];
+        const ConvPlan* conv = find_conv_sources(pl, GK_PRIMAL);
+        if (!conv) fail(ILH_ERR_STATE, "the plan's LGF spectrum is not built yet");
+        const ConvPlan& C = *conv;
         auto up = [](size_t b) { return (b + 255) / 256 * 256; };
         const size_t b_amp = up(sizeof(double) * 2 * (size_t)N);
         const size_t b_t1 = up(sizeof(double2) * (size_t)conv_ext_rows1(sc->src1) * C.H);
@@ -1966,7 +1973,7 @@ bool batch_fusable(int nprob, ilh_plan* const* plans)
 {
     for (int i = 0; i < nprob; ++i) {
         if (plans[i]->N == 0) continue;
-        const ConvPlan& C = get_conv(plans[i], GK_PRIMAL);
+        const ConvPlan& C = get_conv_sources(plans[i], GK_PRIMAL);
         if (!fused_supported(C.Px, C.Py)) return false;
     }
     return true;
@@ -1989,7 +1996,7 @@ void batch_probs(ilh_ctx* ctx, int nprob, ilh_plan* const* plans, SolveCache* co
         }
         const SourceSet& src = sc[i]->src1;
         if (src.npairs_dev) fail(ILH_ERR_STATE, "the source pairs are not pinned");
-        ConvPlan& C = get_conv(pl, GK_PRIMAL);
+        ConvPlan& C = get_conv_sources(pl, GK_PRIMAL);
         BatchProb b;
         std::memset(&b, 0, sizeof(b));   // padding too: batches are compared bytewise
         b.Mp = sc[i]->M[0].as<double>();
@@ -3236,7 +3243,7 @@ static bool moving_conv_fused(ilh_ctx* ctx, int slot, const std::vector<ilh_plan
     std::vector<BatchProb> probs;
     for (size_t k = 0; k < pls.size(); ++k) {
         ilh_plan* pl = pls[k];
-        const ConvPlan& C = get_conv(pl, GK_PRIMAL);
+        const ConvPlan& C = get_conv_sources(pl, GK_PRIMAL);
         if (!fused_supported(C.Px, C.Py)) return false;
         const SourceSet& src = mcs[k]->src1;
         BatchProb b;
@@ -3418,7 +3425,7 @@ extern "C" int ilh_dirichlet_solve_moving_batched(int nprob, ilh_plan* const* pl
         // streams' assemblies read the table, and the first convolution runs
         // on the context stream beside them
         for (int i = 0; i < nprob; ++i)
-            if (mc[i]) (void)get_conv(plans[i], GK_PRIMAL);
+            if (mc[i]) (void)get_conv_sources(plans[i], GK_PRIMAL);
         fork();
         auto on = [&](int i) { ctx->stream = ctx->pool[i % ilh_ctx::POOL]; };
         std::vector<int> state(nprob, 0), it(nprob, 0);

@@ -4,7 +4,8 @@
 // inverse_laplacian!(w, cache) = L \ w = dx^2 (G * w) over the field's own
 // index set (src/grid_operators.jl:144-179, LGF plan of src/cache.jl:321-324),
 // G(0,0) = 0, L G = delta.  G is even, so a circular period P >= 2n-2 per axis
-// reproduces the linear convolution exactly; P is a power of two >= 16.
+// reproduces the linear convolution exactly (less where the sources' extent is
+// known: source_period); P is a power of two >= 16.
 //
 // Transforms are Stockham radix-8 stages (plus one radix-2 or -4 stage when P
 // is not a power of 8), with each thread holding V = 8 complex values in
@@ -398,44 +399,93 @@ void ensure_lgf(ilh_plan* pl)
 
 
 // -------------------------------------------------------------- plans
-static int period(int n)
+static int period(int need)
 {
     int P = 16;
-    while (P < 2 * n - 2) P <<= 1;
+    while (P < need) P <<= 1;
     return P;
+}
+
+// A circular convolution of period P (the kernel even, its table out to P/2)
+// gives out(o) = sum_s G(|o - s|) in(s) exactly where |o - s| <= P/2: for any
+// field of n values P >= 2n - 2, and for sources between s0 and s1 alone
+// P >= 2 max(s1, n - 1 - s0), down to n for sources in the middle (a period
+// must also hold the n outputs).  Bodies rarely reach both ends of an axis, so
+// the solves' convolutions run on the periods their points need: half the
+// period for a body in the middle third.
+static int source_period(int n, double lo, double hi, double shift)
+{
+    // the terms' windows span floor(x) - 2 ... floor(x) + 3 about a point at x
+    const int s0 = std::max(0, (int)std::floor(lo + shift) - 2), s1 = std::min(n - 1, (int)std::floor(hi + shift) + 3);
+    return period(std::max(n, 2 * std::max(s1, n - 1 - s0)));
+}
+
+static void source_periods(const ilh_plan* pl, int gk, int& Px, int& Py)
+{
+    const Grid& g = pl->g;
+    const double sx = gk == GK_DUAL || gk == GK_EDGE_U ? 0.5 : 0.0, sy = gk == GK_DUAL || gk == GK_EDGE_V ? 0.5 : 0.0;
+    Px = source_period(g.nx(gk), pl->ext[0], pl->ext[1], sx);
+    Py = source_period(g.ny(gk), pl->ext[2], pl->ext[3], sy);
+}
+
+static ConvPlan& conv_of(ilh_plan* pl, int gk, int Px, int Py)
+{
+    for (ConvPlan& C : pl->conv[gk])
+        if (C.Px == Px && C.Py == Py) return C;
+    ilh_ctx* ctx = pl->ctx;
+    ensure_lgf(pl);
+    const Grid& g = pl->g;
+    if (Px > MAXP || Py > MAXP) fail(ILH_ERR_ARG, "grid too large for the FFT convolution (period > 8192)");
+    pl->conv[gk].emplace_back();
+    ConvPlan& C = pl->conv[gk].back();
+    try {
+        C.gk = gk;
+        C.nx = g.nx(gk);
+        C.ny = g.ny(gk);
+        C.Px = Px;
+        C.Py = Py;
+        C.H = C.Px / 2;
+        const int rows = (std::max(C.Py, C.ny + 1) + 7) / 8 * 8;   // tiled layout: whole 8-row tiles
+        C.T1.ensure(sizeof(double2) * (size_t)rows * C.H);
+        C.T2.ensure(sizeof(double2) * (size_t)((C.ny + 1 + 7) / 8 * 8) * C.H);
+        C.spec.ensure(sizeof(double) * (size_t)(C.H + 1) * (C.Py / 2 + 1));
+        // spectrum of the circular kernel: rows of G_circ, then forward columns
+        RowSrc S{};
+        S.mode = ROW_LGF;
+        S.tab = pl->lgf.as<double>();
+        S.tmx = pl->lgf_mx;
+        S.Px = C.Px;
+        S.Py = C.Py;
+        launch_rows_fwd(ctx, S, C.Px, C.Py / 2, C.Py, C.T1.as<double2>());
+        const double scale = g.dx * g.dx / ((double)C.Px * C.Py);
+        launch_cols<1, double2, double2>(ctx, C.T1.as<double2>(), nullptr, C.Px, C.Py, C.Py, C.Py, nullptr, scale,
+                                         (double2*)nullptr, C.spec.as<double>());
+    } catch (...) {
+        pl->conv[gk].pop_back();
+        throw;
+    }
+    return C;
 }
 
 ConvPlan& get_conv(ilh_plan* pl, int gk)
 {
-    ConvPlan& C = pl->conv[gk];
-    if (pl->conv_ok[gk]) return C;
-    ilh_ctx* ctx = pl->ctx;
-    ensure_lgf(pl);
-    const Grid& g = pl->g;
-    C.gk = gk;
-    C.nx = g.nx(gk);
-    C.ny = g.ny(gk);
-    C.Px = period(C.nx);
-    C.Py = period(C.ny);
-    if (C.Px > MAXP || C.Py > MAXP) fail(ILH_ERR_ARG, "grid too large for the FFT convolution (period > 8192)");
-    C.H = C.Px / 2;
-    const int rows = (std::max(C.Py, C.ny + 1) + 7) / 8 * 8;   // tiled layout: whole 8-row tiles
-    C.T1.ensure(sizeof(double2) * (size_t)rows * C.H);
-    C.T2.ensure(sizeof(double2) * (size_t)((C.ny + 1 + 7) / 8 * 8) * C.H);
-    C.spec.ensure(sizeof(double) * (size_t)(C.H + 1) * (C.Py / 2 + 1));
-    // spectrum of the circular kernel: rows of G_circ, then forward columns
-    RowSrc S{};
-    S.mode = ROW_LGF;
-    S.tab = pl->lgf.as<double>();
-    S.tmx = pl->lgf_mx;
-    S.Px = C.Px;
-    S.Py = C.Py;
-    launch_rows_fwd(ctx, S, C.Px, C.Py / 2, C.Py, C.T1.as<double2>());
-    const double scale = g.dx * g.dx / ((double)C.Px * C.Py);
-    launch_cols<1, double2, double2>(ctx, C.T1.as<double2>(), nullptr, C.Px, C.Py, C.Py, C.Py, nullptr, scale,
-                                     (double2*)nullptr, C.spec.as<double>());
-    pl->conv_ok[gk] = true;
-    return C;
+    return conv_of(pl, gk, period(2 * pl->g.nx(gk) - 2), period(2 * pl->g.ny(gk) - 2));
+}
+
+ConvPlan& get_conv_sources(ilh_plan* pl, int gk)
+{
+    int Px, Py;
+    source_periods(pl, gk, Px, Py);
+    return conv_of(pl, gk, Px, Py);
+}
+
+const ConvPlan* find_conv_sources(const ilh_plan* pl, int gk)
+{
+    int Px, Py;
+    source_periods(pl, gk, Px, Py);
+    for (const ConvPlan& C : pl->conv[gk])
+        if (C.Px == Px && C.Py == Py) return &C;
+    return nullptr;
 }
 
 void conv_dense(ilh_plan* pl, int gk, const double* in, double* out)
@@ -531,7 +581,7 @@ static RowSrc terms_source(const ConvPlan& C, const SourceSet& src, const double
 // one pass of conv_sources alone (0 = rows, 1 = columns, 2 = inverse rows), for timing
 void conv_stage(ilh_plan* pl, int gk, const SourceSet& src, const double* amp, double* out, int stage)
 {
-    ConvPlan& C = get_conv(pl, gk);
+    ConvPlan& C = get_conv_sources(pl, gk);
     if (stage == 0) {
         launch_rows_fwd(pl->ctx, terms_source(C, src, amp), C.Px, src.npairs, C.ny, C.T1.as<double2>());
     } else if (stage == 1) {
@@ -547,7 +597,7 @@ void conv_stage(ilh_plan* pl, int gk, const SourceSet& src, const double* amp, d
 void conv_sources_multi(ilh_plan* pl, int gk, const SourceSet& src, const double* amp, size_t amp_stride, int nb,
                         double* out)
 {
-    ConvPlan& C = get_conv(pl, gk);
+    ConvPlan& C = get_conv_sources(pl, gk);
     const size_t s1 = C.T1.bytes / sizeof(double2), s2 = C.T2.bytes / sizeof(double2);
     C.T1m.ensure(C.T1.bytes * (size_t)nb);
     C.T2m.ensure(C.T2.bytes * (size_t)nb);
@@ -569,10 +619,11 @@ int conv_ext_rows2(const ConvPlan& C) { return (C.ny + 1 + 7) / 8 * 8; }
 void conv_sources_ext(ilh_plan* pl, int gk, const SourceSet& src, const double* amp, double* out, double2* T1,
                       double2* T2)
 {
-    if (!pl->conv_ok[gk]) fail(ILH_ERR_STATE, "the plan's LGF spectrum is not built yet");
     if (src.npairs_dev) fail(ILH_ERR_STATE, "the source pairs are not pinned");
     LookupOnly guard;
-    const ConvPlan& C = pl->conv[gk];
+    const ConvPlan* conv = find_conv_sources(pl, gk);
+    if (!conv) fail(ILH_ERR_STATE, "the plan's LGF spectrum is not built yet");
+    const ConvPlan& C = *conv;
     launch_rows_fwd(pl->ctx, terms_source(C, src, amp), C.Px, src.npairs, C.ny, T1);
     launch_cols<0>(pl->ctx, T1, src.slot_of_row, C.Px, C.Py, C.ny, 0, C.spec.as<double>(), 1.0, T2, nullptr);
     launch_rows_inv(pl->ctx, (const double2*)T2, C.Px, C.nx, C.ny, out);
@@ -586,7 +637,7 @@ void conv_sources_ext(ilh_plan* pl, int gk, const SourceSet& src, const double* 
 // after the product the spectrum is smooth and FP32 keeps ~1e-7.)
 void conv_sources_f32(ilh_plan* pl, int gk, const SourceSet& src, const double* amp, double* out)
 {
-    ConvPlan& C = get_conv(pl, gk);
+    ConvPlan& C = get_conv_sources(pl, gk);
     launch_rows_fwd(pl->ctx, terms_source(C, src, amp), C.Px, src.npairs, C.ny, C.T1.as<double2>());
     launch_cols<0>(pl->ctx, (const double2*)C.T1.as<double2>(), src.slot_of_row, C.Px, C.Py, C.ny, 0,
                    C.spec.as<double>(), 1.0, C.T2.as<float2>(), nullptr);
@@ -595,7 +646,7 @@ void conv_sources_f32(ilh_plan* pl, int gk, const SourceSet& src, const double* 
 
 void conv_sources(ilh_plan* pl, int gk, const SourceSet& src, const double* amp, double* out, hipEvent_t* ev)
 {
-    ConvPlan& C = get_conv(pl, gk);
+    ConvPlan& C = get_conv_sources(pl, gk);
     hipStream_t st = pl->ctx->stream;
     launch_rows_fwd(pl->ctx, terms_source(C, src, amp), C.Px, src.npairs, C.ny, C.T1.as<double2>());
     if (ev) ILH_HIP(hipEventRecord(ev[0], st));

@@ -4,6 +4,7 @@
 #include <atomic>
 #include <cstddef>
 #include <cstdint>
+#include <list>
 #include <new>
 #include <string>
 #include <vector>
@@ -197,8 +198,8 @@ struct ilh_plan {
     bool wins_ok = false;
     ilh::RowBins bins[ilh::OP_COUNT][4];     // row bins of scatter ops per component grid
     bool bins_ok[ilh::OP_COUNT] = {};
-    ilh::ConvPlan conv[4];                    // primal, dual, u edges, v edges
-    bool conv_ok[4] = {};
+    std::list<ilh::ConvPlan> conv[4];         // primal, dual, u edges, v edges: one per pair of periods in use
+    double ext[4] = {};                       // the points' extent in primal grid units, 0-based: x, x, y, y
     ilh::DevBuf lgf;                          // LGF table tmx x tmy (covers both kinds)
     int lgf_mx = 0, lgf_my = 0;
     ilh::DevBuf io_a, io_b, io_c, io_d;       // staging for host-memory calls
@@ -268,7 +269,11 @@ void axpby(hipStream_t st, double* y, const double* x, double a, double b, size_
 
 // FFT convolution (ilh_fft.hip)
 void ensure_lgf(ilh_plan* pl);
-ConvPlan& get_conv(ilh_plan* pl, int gk);
+ConvPlan& get_conv(ilh_plan* pl, int gk);       // periods for any field on the grid
+// Periods for sources on the plan's points alone (the windows of their terms),
+// and the result on the whole grid: what the points' extent needs.
+ConvPlan& get_conv_sources(ilh_plan* pl, int gk);
+const ConvPlan* find_conv_sources(const ilh_plan* pl, int gk);   // null: not built yet
 // field -> field:  out = dx^2 (G * in)
 void conv_dense(ilh_plan* pl, int gk, const double* in, double* out);
 void conv_dense(ilh_plan* pl, int gk, const float* in, float* out);   // FP32 fields, FP32 transforms
