@@ -1361,8 +1361,8 @@ extern "C" int ilh_neumann_solve(ilh_plan* pl, const double* vp, const double* v
         } else {
             neumann_amp(st, sc->M[0].as<double>(), sc->M[1].as<double>(), sc->M[2].as<double>(), sc->M[3].as<double>(),
                         solve_ld(N), d_vp, d_vm, sc->amp1.as<double>(), sc->amp2.as<double>(), d_df, d_ds, N);
-            conv_sources(pl, GK_PRIMAL, sc->src1, sc->amp1.as<double>(), d_f);
-            conv_sources(pl, GK_DUAL, sc->src2, sc->amp2.as<double>(), d_s);
+            conv_sources_pair(pl, GK_PRIMAL, sc->src1, sc->amp1.as<double>(), d_f, GK_DUAL, sc->src2,
+                              sc->amp2.as<double>(), d_s);
         }
         io.back(f, d_f, ng);
         io.back(df, d_df, N);

@@ -174,6 +174,57 @@ __global__ void __launch_bounds__(tpb_of(P)) k_rows_inv(const typename Cplx<R>::
     rows_inv_body<P, tpb_of(P) / (P / V), TO, R, TR>(T2, tw, nx, ny, out, xcd_block(), (C2*)lds_raw, threadIdx.x);
 }
 
+// Two convolutions with the same periods and their own sources, spectra and
+// outputs (a solve's primal and dual fields), blockIdx.y choosing between them.
+// At a few hundred points a side a pass of one convolution is a few dozen
+// work-groups and its time is latency: two of them on one launch take little
+// more than the time of one (periods 1024: rows 9.1, columns 8.8, inverse rows
+// 6.1 us for two against 7.2 + 7.7 + 5.1 us for each).  Every transform is the
+// single launches' own code.
+struct ConvPairArgs {
+    RowSrc S[2];
+    int npairs[2];
+    double2* T1[2];
+    double2* T2[2];
+    const int* slot[2];
+    const double* spec[2];
+    double* out[2];
+    int nx[2], ny[2];
+};
+
+template <int P>
+__global__ void __launch_bounds__(tpb_of(P)) k_rows_fwd_pair(ConvPairArgs A, const double2* __restrict__ tw)
+{
+    extern __shared__ double2 lds_raw[];
+    constexpr int NB = tpb_of(P) / (P / V);
+    const int y = blockIdx.y;
+    const RowSrc S = A.S[y];
+    const int npairs = S.npairs_dev ? *S.npairs_dev : A.npairs[y];
+    const int nblk = (npairs + NB - 1) / NB;
+    if ((int)blockIdx.x >= nblk) return;
+    rows_fwd_body<P, NB, double, true>(S, tw, npairs, A.ny[y], A.T1[y], xcd_block_of(blockIdx.x, nblk), lds_raw,
+                                       threadIdx.x);
+}
+
+template <int P>
+__global__ void __launch_bounds__(tpb_of(P)) __attribute__((amdgpu_waves_per_eu(4)))
+k_cols_pair(ConvPairArgs A, const double2* __restrict__ tw, int H)
+{
+    extern __shared__ double2 lds_raw[];
+    const int y = blockIdx.y;
+    cols_body<P, tpb_of(P) / (P / V), 0, double, double, 4>(A.T1[y], A.slot[y], tw, tw, H, A.ny[y], 0, A.spec[y], 1.0,
+                                                           A.T2[y], nullptr, xcd_block(), lds_raw, threadIdx.x);
+}
+
+template <int P>
+__global__ void __launch_bounds__(tpb_of(P)) k_rows_inv_pair(ConvPairArgs A, const double2* __restrict__ tw)
+{
+    extern __shared__ double2 lds_raw[];
+    const int y = blockIdx.y;
+    rows_inv_body<P, tpb_of(P) / (P / V), double, double, 4>(A.T2[y], tw, A.nx[y], A.ny[y], A.out[y], xcd_block(),
+                                                            lds_raw, threadIdx.x);
+}
+
 // ------------------------------------------------------------- launches
 static void set_lds(const void* fn, size_t bytes)
 {
@@ -654,6 +705,95 @@ void conv_sources(ilh_plan* pl, int gk, const SourceSet& src, const double* amp,
                    C.T2.as<double2>(), nullptr);
     if (ev) ILH_HIP(hipEventRecord(ev[1], st));
     launch_rows_inv(pl->ctx, C.T2.as<double2>(), C.Px, C.nx, C.ny, out);
+}
+
+template <int P>
+static void launch_rows_fwd_pair(ilh_ctx* ctx, const ConvPairArgs& A)
+{
+    constexpr int NB = tpb_of(P) / (P / V);
+    ConvPairArgs B = A;
+    size_t amps = 0;
+    for (int y = 0; y < 2; ++y) {
+        B.S[y].amp_lds = B.S[y].amp_len <= amp_lds_cap(P);
+        if (B.S[y].amp_lds) amps = std::max(amps, sizeof(double) * (size_t)B.S[y].amp_len);
+    }
+    const size_t lds = sizeof(double2) * (size_t)NB * lds_len(P) + amps;
+    set_lds((const void*)k_rows_fwd_pair<P>, lds);
+    k_rows_fwd_pair<P><<<dim3((std::max(A.npairs[0], A.npairs[1]) + NB - 1) / NB, 2), tpb_of(P), lds, ctx->stream>>>(
+        B, twiddles<double>(ctx, P));
+    ILH_HIP(hipGetLastError());
+}
+
+template <int P>
+static void launch_cols_pair(ilh_ctx* ctx, const ConvPairArgs& A, int H)
+{
+    constexpr int NB = tpb_of(P) / (P / V);
+    const size_t lds = sizeof(double2) * (size_t)NB * lds_len(P);
+    set_lds((const void*)k_cols_pair<P>, lds);
+    k_cols_pair<P><<<dim3((H + NB - 1) / NB, 2), tpb_of(P), lds, ctx->stream>>>(A, twiddles<double>(ctx, P), H);
+    ILH_HIP(hipGetLastError());
+}
+
+template <int P>
+static void launch_rows_inv_pair(ilh_ctx* ctx, const ConvPairArgs& A)
+{
+    constexpr int NB = tpb_of(P) / (P / V);
+    const size_t lds = sizeof(double2) * (size_t)NB * lds_len(P);
+    set_lds((const void*)k_rows_inv_pair<P>, lds);
+    k_rows_inv_pair<P><<<dim3(((std::max(A.ny[0], A.ny[1]) + 1) / 2 + NB - 1) / NB, 2), tpb_of(P), lds, ctx->stream>>>(
+        A, twiddles<double>(ctx, P));
+    ILH_HIP(hipGetLastError());
+}
+
+// Periods up to here run as pairs.  A Neumann solve, two by two and as pairs
+// (with the surface step's change): 38 -> 20 us at 256^2, 48 -> 29 at 406^2,
+// 70 -> 55 at 700^2, 76 -> 65 at 1000^2; from 4096 on one convolution's pass
+// is many times the chip's work-groups and there is nothing left to hide.
+constexpr int PAIR_MAX_P = 2048;
+
+#define ILH_FOR_PAIR_P(P, BODY)                          \
+    switch (P) {                                         \
+    case 16: { constexpr int PP = 16; BODY; } break;     \
+    case 32: { constexpr int PP = 32; BODY; } break;     \
+    case 64: { constexpr int PP = 64; BODY; } break;     \
+    case 128: { constexpr int PP = 128; BODY; } break;   \
+    case 256: { constexpr int PP = 256; BODY; } break;   \
+    case 512: { constexpr int PP = 512; BODY; } break;   \
+    case 1024: { constexpr int PP = 1024; BODY; } break; \
+    case 2048: { constexpr int PP = 2048; BODY; } break; \
+    default: fail(ILH_ERR_ARG, "FFT length of a pair");  \
+    }
+
+void conv_sources_pair(ilh_plan* pl, int gk0, const SourceSet& src0, const double* amp0, double* out0, int gk1,
+                       const SourceSet& src1, const double* amp1, double* out1)
+{
+    ConvPlan& C0 = get_conv_sources(pl, gk0);
+    ConvPlan& C1 = get_conv_sources(pl, gk1);
+    if (gk0 == gk1 || C0.Px != C1.Px || C0.Py != C1.Py || std::max(C0.Px, C0.Py) > PAIR_MAX_P || src0.npairs <= 0 ||
+        src1.npairs <= 0) {
+        conv_sources(pl, gk0, src0, amp0, out0);
+        conv_sources(pl, gk1, src1, amp1, out1);
+        return;
+    }
+    ConvPairArgs A{};
+    const ConvPlan* C[2] = {&C0, &C1};
+    const SourceSet* src[2] = {&src0, &src1};
+    const double* amp[2] = {amp0, amp1};
+    double* out[2] = {out0, out1};
+    for (int y = 0; y < 2; ++y) {
+        A.S[y] = terms_source(*C[y], *src[y], amp[y]);
+        A.npairs[y] = src[y]->npairs;
+        A.T1[y] = C[y]->T1.as<double2>();
+        A.T2[y] = C[y]->T2.as<double2>();
+        A.slot[y] = src[y]->slot_of_row;
+        A.spec[y] = C[y]->spec.as<double>();
+        A.out[y] = out[y];
+        A.nx[y] = C[y]->nx;
+        A.ny[y] = C[y]->ny;
+    }
+    ILH_FOR_PAIR_P(C0.Px, (launch_rows_fwd_pair<PP>(pl->ctx, A)));
+    ILH_FOR_PAIR_P(C0.Py, (launch_cols_pair<PP>(pl->ctx, A, C0.H)));
+    ILH_FOR_PAIR_P(C0.Px, (launch_rows_inv_pair<PP>(pl->ctx, A)));
 }
 
 }  // namespace ilh

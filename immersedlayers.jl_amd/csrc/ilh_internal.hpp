@@ -317,6 +317,10 @@ void conv_stage(ilh_plan* pl, int gk, const SourceSet& src, const double* amp, d
 // the same convolution in split precision: forward transforms and the spectrum
 // product in FP64, the inverse transforms in FP32 (FP64 output)
 void conv_sources_f32(ilh_plan* pl, int gk, const SourceSet& src, const double* amp, double* out);
+// two source convolutions at once (different fields; one launch per pass where
+// their periods agree)
+void conv_sources_pair(ilh_plan* pl, int gk0, const SourceSet& src0, const double* amp0, double* out0, int gk1,
+                       const SourceSet& src1, const double* amp1, double* out1);
 // conv_sources into caller-supplied spectra buffers, allocating nothing
 int conv_ext_rows1(const SourceSet& src);
 int conv_ext_rows2(const ConvPlan& C);

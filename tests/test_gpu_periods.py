@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("n,m,cx,cy,r", [(64, 64, 0.5, 0.5, 8), (65, 33, 0.5, 0.5, 8), (100, 140, 0.0, 0.5, 12),
                                          (129, 70, 1.0, 1.0, 9), (200, 97, 0.0, 0.0, 20), (260, 60, 0.3, 0.5, 14),
-                                         (150, 600, 0.5, 0.9, 30)])
+                                         (150, 600, 0.5, 0.9, 30),
+                                         (140, 64, 0.9172, 0.5, 20)])   # last: the primal and dual periods differ
 def test_source_periods(ctx, n, m, cx, cy, r):
     """A circle of r cells, its centre at the fraction (cx, cy) between the
     positions that keep it 6 cells inside the grid."""
