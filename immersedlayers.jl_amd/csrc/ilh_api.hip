@@ -115,9 +115,15 @@ struct StokesCache {
     DevBuf Cf;                    // the vector surface filter's two diagonal blocks (N x N each, row-major,
                                   // leading dimension solve_ld(N)), built on the first filtered solve
     bool cf_ok = false;
-    DevBuf sv;                    // surface work: dv, vb, e_phi, w, vprime, sigma (2N each); dvn, dsv, ds (N each)
-    DevBuf gE, gE2, gP;           // grid work: edges (2), primal
-    DevBuf gDD;                   // two Nodes{Dual} fields back to back (one batched convolution)
+    DevBuf sv;                    // surface work (SW_* below)
+    DevBuf gP;                    // phi
+    DevBuf gDD;                   // two Nodes{Dual} fields back to back (y, then t; c)
+    DevBuf terms[3];              // merged source terms of src
+    SourceSet src[3];             // R (phi); [C^T D_s^symm, C_s^T] (y); C^x_s^T (c)
+    ~StokesCache()
+    {
+        for (SourceSet& q : src) free_sources(q);
+    }
 };
 
 // Moving bodies: the inverse Schur matrix of a reference geometry (row-major,
@@ -437,7 +443,7 @@ int op_components(int op, int* gks)
 {
     switch (op) {
     case OP_R_PRIMAL: case OP_DS: gks[0] = GK_PRIMAL; return 1;
-    case OP_R_DUAL: case OP_CST: case OP_CXT: case OP_CVT: gks[0] = GK_DUAL; return 1;
+    case OP_R_DUAL: case OP_CST: case OP_CXT: case OP_CVT: case OP_CDSYM: gks[0] = GK_DUAL; return 1;
     case OP_RNSYM: gks[0] = GK_T_XX; gks[1] = GK_T_XY; gks[2] = GK_T_YX; gks[3] = GK_T_YY; return 4;
     default: gks[0] = GK_EDGE_U; gks[1] = GK_EDGE_V; return 2;
     }
@@ -1008,19 +1014,20 @@ void factor_into(ilh_plan* pl, SolveCache* sc, int kind)
     if (info) fail(ILH_ERR_SINGULAR, "Schur complement is singular (zero pivot at column " + std::to_string(info) + ")");
 }
 
-// merged source terms: first op with amplitude slot 0, second with slot 1
+// merged source terms: op0's amplitudes first, op1's (op1 < 0: none) behind them
 void merge_sources(ilh_plan* pl, int op0, int op1, int gk, DevBuf& tbuf, SourceSet& src)
 {
     const int N = pl->N;
-    const int n0 = N * op_terms_per_point(op0), n1 = N * op_terms_per_point(op1);
+    const int n0 = N * op_terms_per_point(op0), n1 = op1 < 0 ? 0 : N * op_terms_per_point(op1);
+    const int a0 = N * op_amps_per_point(op0), a1 = op1 < 0 ? 0 : N * op_amps_per_point(op1);
     tbuf.ensure(sizeof(Term) * (size_t)std::max(1, n0 + n1));
     hipStream_t st = pl->ctx->stream;
     Term* t = tbuf.as<Term>();
     if (n0) k_term_shift<<<(n0 + 255) / 256, 256, 0, st>>>(get_terms(pl, op0), n0, 0, t);
-    if (n1) k_term_shift<<<(n1 + 255) / 256, 256, 0, st>>>(get_terms(pl, op1), n1, N, t + n0);
+    if (n1) k_term_shift<<<(n1 + 255) / 256, 256, 0, st>>>(get_terms(pl, op1), n1, a0, t + n0);
     ILH_HIP(hipGetLastError());
     src.terms = t;
-    src.amp_len = 2 * N;
+    src.amp_len = a0 + a1;
     build_bins(pl, t, n0 + n1, gk, src.bins);
     build_source_pairs(pl, src);
 }
@@ -1728,13 +1735,20 @@ extern "C" int ilh_surface_filter_apply_vector(ilh_plan* pl, int power, const do
 //   sigma = S^-1 (v_bar - E v_phi + Ka [v]),   b = L^-2 C_s^T sigma,
 //   t = a + b = L^-1 (L^-1 (C^T D_s^symm [v] + C_s^T sigma)),
 //   v = v_phi - C t,   s = -(t + L^-1 C^x_s^T Ss^-1 G^x_s phi).
-// The reference's six convolutions per solve become three passes: phi on
-// Nodes{Primal}, L^-1 of the summed sources on Nodes{Dual}, then L^-1 of
-// that field and of the potential's sources together as one batched pass.
+// The reference's six convolutions per solve become four: phi on
+// Nodes{Primal}; y = L^-1 (C^T D_s^symm [v] + C_s^T sigma) and the potential's
+// streamfunction c = L^-1 C^x_s^T Ss^-1 G^x_s phi as one pair, both straight
+// from the points' terms; t = L^-1 y.  At the sizes this runs at (a few hundred
+// cells a side) every launch is 3-9 us of latency whatever it does, so the
+// solve is arranged for few launches: 16 and one per filter power, where
+// operator by operator they were 28 and two (406^2, 214 points, power 2:
+// 134 -> 94 us).
 namespace {
+// surface quantities of the prescribed velocities: [v], v_bar, n . [v] and the
+// symmetric surface tensor's T_xx, T_xy (OP_CDSYM's amplitudes)
 __global__ void k_stokes_rhs(int N, const double* __restrict__ vp, const double* __restrict__ vm,
                              const double* __restrict__ nx, const double* __restrict__ ny, double* __restrict__ dv,
-                             double* __restrict__ vb, double* __restrict__ dvn)
+                             double* __restrict__ vb, double* __restrict__ dvn, double* __restrict__ tt)
 {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= N) return;
@@ -1747,14 +1761,28 @@ __global__ void k_stokes_rhs(int N, const double* __restrict__ vp, const double*
         vb[k] = 0.5 * a + 0.5 * b;    // prescribed_surface_average!
     }
     dvn[p] = nx[p] * d[0] + ny[p] * d[1];   // pointwise_dot!(dvn, nrm, dv)
+    tt[p] = nx[p] * d[0] - ny[p] * d[1];
+    tt[N + p] = ny[p] * d[0] + nx[p] * d[1];
 }
 
-// vprime = (vb - e_phi) + w
-__global__ void k_stokes_vprime(int n, const double* __restrict__ vb, const double* __restrict__ ephi,
-                                const double* __restrict__ w, double* __restrict__ out)
+// One wave per row: rows [0, 2N) vprime = (vb - e_phi) + Ka [v] (w = Ka [v] =
+// E C a, the reference's -E C psi*), rows [2N, 3N) ds = Ss^-1 G^x_s phi
+__global__ void __launch_bounds__(256) k_stokes_vprime(int N, const double* __restrict__ Ka, int ld2,
+                                                       const double* __restrict__ dv, const double* __restrict__ vb,
+                                                       const double* __restrict__ ephi, double* __restrict__ vpr,
+                                                       const double* __restrict__ Ssinv, int ld1,
+                                                       const double* __restrict__ dsv, double* __restrict__ dsn)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) out[k] = (vb[k] - ephi[k]) + w[k];
+    const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int n2 = 2 * N;
+    if (i >= 3 * N) return;
+    const bool first = i < n2;
+    const double s = wave_dot(first ? Ka + (size_t)ld2 * i : Ssinv + (size_t)ld1 * (i - n2), first ? dv : dsv,
+                              first ? n2 : N, lane);
+    if (lane == 0) {
+        if (first) vpr[i] = (vb[i] - ephi[i]) + s;
+        else dsn[i - n2] = s;
+    }
 }
 
 // the vector filter's diagonal blocks (C is block-diagonal: u and v
@@ -1774,6 +1802,30 @@ void stokes_filter(ilh_plan* pl, StokesCache* sc)
     sc->cf_ok = true;
 }
 
+// the solve's surface vectors, every one at an even offset (16-byte loads).
+// [T_xx, T_xy] and sigma are y's amplitudes, one behind the other.
+struct StokesWork {
+    int tt, sig, sig2, dv, vb, ephi, vpr, r, dvn, dsv, dsn, len;
+};
+StokesWork stokes_work(int N)
+{
+    const int n2 = 2 * N, n1 = N + (N & 1);
+    StokesWork w;
+    w.tt = 0;
+    w.sig = w.tt + n2;
+    w.sig2 = w.sig + n2;
+    w.dv = w.sig2 + n2;
+    w.vb = w.dv + n2;
+    w.ephi = w.vb + n2;
+    w.vpr = w.ephi + n2;
+    w.r = w.vpr + n2;
+    w.dvn = w.r + n2;
+    w.dsv = w.dvn + n1;
+    w.dsn = w.dsv + n1;
+    w.len = std::max(1, w.dsn + n1);
+    return w;
+}
+
 StokesCache* prepare_stokes(ilh_plan* pl)
 {
     if (pl->sto) return pl->sto;
@@ -1782,9 +1834,7 @@ StokesCache* prepare_stokes(ilh_plan* pl)
     try {
         const int N = pl->N, n2 = 2 * N;
         const Grid& g = pl->g;
-        sc->sv.ensure(sizeof(double) * (size_t)std::max(1, 6 * n2 + 3 * N));
-        sc->gE.ensure(sizeof(double) * std::max(g.n_edges(), (size_t)n2));   // also the filter's second iterate
-        sc->gE2.ensure(sizeof(double) * g.n_edges());
+        sc->sv.ensure(sizeof(double) * (size_t)stokes_work(N).len);
         sc->gDD.ensure(2 * sizeof(double) * g.n(GK_DUAL));
         sc->gP.ensure(sizeof(double) * g.n(GK_PRIMAL));
         if (N > 0) {
@@ -1801,6 +1851,10 @@ StokesCache* prepare_stokes(ilh_plan* pl)
             build_stokes_ka(pl, K.as<double>());
             sc->Ka.ensure(sizeof(double) * (size_t)n2 * solve_ld(n2));
             transpose(pl->ctx->stream, K.as<double>(), sc->Ka.as<double>(), n2, n2, solve_ld(n2));
+            merge_sources(pl, OP_R_PRIMAL, -1, GK_PRIMAL, sc->terms[0], sc->src[0]);
+            merge_sources(pl, OP_CDSYM, OP_CVT, GK_DUAL, sc->terms[1], sc->src[1]);
+            merge_sources(pl, OP_CXT, -1, GK_DUAL, sc->terms[2], sc->src[2]);
+            for (SourceSet& q : sc->src) pin_source_pairs(pl, q);
             ILH_HIP(hipStreamSynchronize(pl->ctx->stream));
         }
     } catch (...) {
@@ -1829,69 +1883,55 @@ extern "C" int ilh_stokes_solve(ilh_plan* pl, const double* v_plus, const double
         double* d_v = io.out(v, ne, pl->io_b);
         double* d_s = io.out(s, nd, pl->io_d);
         if (n2 > 0 && !sigma) fail(ILH_ERR_ARG, "null output array");
-        // sigma is staged in the surface work area when it lives on the host
+        const StokesWork W = stokes_work(N);
         double* sv = sc->sv.as<double>();
-        double *dv = sv, *vb = sv + n2, *ephi = sv + 2 * n2, *w = sv + 3 * n2, *vpr = sv + 4 * n2;
-        double* sig = mem == ILH_MEM_DEVICE ? sigma : sv + 5 * n2;
-        double *dvn = sv + 6 * n2, *dsv = dvn + N, *dsn = dsv + N;
-        double *gE = sc->gE.as<double>(), *gE2 = sc->gE2.as<double>(), *gP = sc->gP.as<double>();
-        double *gD = sc->gDD.as<double>(), *gD2 = gD + nd;
+        double *dv = sv + W.dv, *vb = sv + W.vb, *ephi = sv + W.ephi, *vpr = sv + W.vpr, *r = sv + W.r;
+        double *tt = sv + W.tt, *sig = sv + W.sig, *dvn = sv + W.dvn, *dsv = sv + W.dsv, *dsn = sv + W.dsn;
+        // the filtered sigma, staged in the work area when it lives on the host
+        double* sig_out = mem == ILH_MEM_DEVICE ? sigma : sv + W.sig2;
+        double *gP = sc->gP.as<double>(), *gD = sc->gDD.as<double>(), *gD2 = gD + nd;
         if (N == 0) {
             fill_zero(st, d_v, ne);
             fill_zero(st, d_s, nd);
         } else {
-            const unsigned bN = (unsigned)((N + 127) / 128), b2 = (unsigned)((n2 + 127) / 128);
-            const int ld2 = solve_ld(n2);
-            k_stokes_rhs<<<bN, 128, 0, st>>>(N, d_vp, d_vm, pl->nx.as<double>(), pl->ny.as<double>(), dv, vb, dvn);
-            // phi = L^-1 R (n . [v]),  v_phi = G phi
-            scatter_op(pl, OP_R_PRIMAL, dvn, gP);
-            conv_dense(pl, GK_PRIMAL, gP, gP);
-            k_grad(pl, gE2, gP);
-            gather_op(pl, OP_E_EDGES, gE2, ephi);
-            // w = Ka [v] = E C a (the reference's -E C psi*)
-            matvec_rows(st, sc->Ka.as<double>(), ld2, dv, w, n2, n2, 1.0, 0);
-            k_stokes_vprime<<<b2, 128, 0, st>>>(n2, vb, ephi, w, vpr);
+            const int ld2 = solve_ld(n2), ld1 = solve_ld(N);
+            k_stokes_rhs<<<(N + 127) / 128, 128, 0, st>>>(N, d_vp, d_vm, pl->nx.as<double>(), pl->ny.as<double>(), dv,
+                                                          vb, dvn, tt);
+            ILH_HIP(hipGetLastError());
+            // phi = L^-1 R (n . [v]);  E v_phi = E G phi and G^x_s phi on the points
+            conv_sources(pl, GK_PRIMAL, sc->src[0], dvn, gP);
+            gather_grad(pl, gP, get_terms(pl, OP_E_EDGES), op_terms_per_point(OP_E_EDGES), ephi,
+                        get_terms(pl, OP_GXS), op_terms_per_point(OP_GXS), dsv);
+            k_stokes_vprime<<<(3 * N + 3) / 4, 256, 0, st>>>(N, sc->Ka.as<double>(), ld2, dv, vb, ephi, vpr,
+                                                             sc->Ssinv.as<double>(), ld1, dsv, dsn);
             ILH_HIP(hipGetLastError());
             // sigma = S^-1 vprime with one refinement step, so that the residual
             // (the constraint E v = v_bar) is at roundoff as with the
             // reference's LU solve, not at cond(S) eps
-            matvec_rows(st, sc->S2inv.as<double>(), ld2, vpr, sig, n2, n2, 1.0, 0);
-            axpby(st, ephi, vpr, 1.0, 0.0, n2);
-            matvec_rows(st, sc->S2.as<double>(), ld2, sig, ephi, n2, n2, -1.0, 1);
-            matvec_rows(st, sc->S2inv.as<double>(), ld2, ephi, sig, n2, n2, 1.0, 1);
-            // y = L^-1 (C^T D_s^symm [v] + C_s^T sigma)
-            scatter_op(pl, OP_DSYM, dv, gE);
-            k_curl_e2n(pl, gD, gE);
-            scatter_op(pl, OP_CVT, sig, gD2);
-            axpby(st, gD, gD2, 1.0, 1.0, nd);
+            matvec_rows(st, sc->S2inv.as<double>(), ld2, vpr, sig, n2, n2);
+            matvec_rows(st, sc->S2.as<double>(), ld2, sig, r, n2, n2, -1.0, vpr);
+            matvec_rows(st, sc->S2inv.as<double>(), ld2, r, sig, n2, n2, 1.0, sig,
+                        filter_power == 0 ? sig_out : nullptr);
+            // y = L^-1 (C^T D_s^symm [v] + C_s^T sigma) and c = L^-1 C^x_s^T ds,
+            // the streamfunction of the potential's sources
+            conv_sources_pair(pl, GK_DUAL, sc->src[1], tt, gD, GK_DUAL, sc->src[2], dsn, gD2);
+            // t = L^-1 y;  v = G phi - C t,  s = -(t + c)
             conv_dense(pl, GK_DUAL, gD, gD);
-            // the potential's streamfunction sources C^x_s^T Ss^-1 G^x_s phi
-            gather_op(pl, OP_GXS, gP, dsv);
-            matvec_rows(st, sc->Ssinv.as<double>(), solve_ld(N), dsv, dsn, N, N, 1.0, 0);
-            scatter_op(pl, OP_CXT, dsn, gD2);
-            // [t, c] = L^-1 [y, C^x_s^T ds] in one batched pass
-            conv_dense_multi(pl, GK_DUAL, gD, 2, gD);
-            // v = v_phi - C t,  s = -(t + c)
-            k_curl_n2e(pl, d_v, gD);
-            axpby(st, d_v, gE2, 1.0, -1.0, ne);
-            axpby(st, gD2, gD, -1.0, -1.0, nd);
-            ILH_HIP(hipMemcpyAsync(d_s, gD2, sizeof(double) * nd, hipMemcpyDeviceToDevice, st));
+            k_stokes_fields(pl, gP, gD, gD2, d_v, d_s);
             // sigma <- C^k sigma with the stored diagonal blocks of the filter
-            // (gE holds the other iterate)
             if (filter_power > 0) stokes_filter(pl, sc);
-            double *fa = sig, *fb = gE;
-            const int ld1 = solve_ld(N);
+            const double* fa = sig;
             for (int k = 0; k < filter_power; ++k) {
-                matvec_rows(st, sc->Cf.as<double>(), ld1, fa, fb, N, N, 1.0, 0);
-                matvec_rows(st, sc->Cf.as<double>() + (size_t)N * ld1, ld1, fa + N, fb + N, N, N, 1.0, 0);
-                std::swap(fa, fb);
+                // iterates alternate between vpr and r; the last one is the result
+                double* fb = k == filter_power - 1 ? sig_out : (k & 1 ? r : vpr);
+                matvec_rows(st, sc->Cf.as<double>(), ld1, fa, fb, n2, N, 1.0, nullptr, nullptr, N);
+                fa = fb;
             }
-            if (fa != sig) ILH_HIP(hipMemcpyAsync(sig, fa, sizeof(double) * n2, hipMemcpyDeviceToDevice, st));
         }
         io.back(v, d_v, ne);
         io.back(s, d_s, nd);
         if (mem != ILH_MEM_DEVICE && n2 > 0)
-            ILH_HIP(hipMemcpyAsync(sigma, sig, sizeof(double) * n2, hipMemcpyDeviceToHost, st));
+            ILH_HIP(hipMemcpyAsync(sigma, sig_out, sizeof(double) * n2, hipMemcpyDeviceToHost, st));
         io.done();
     });
 }
@@ -3005,7 +3045,7 @@ __global__ void k_identity(double* __restrict__ A, int n)   // A (zeroed) += I, 
 // the current geometry, assembled row-major from the LGF table
 static void schur_apply(ilh_plan* pl, MovingCache* mc, const double* v, double* out)
 {
-    matvec_rows(pl->ctx->stream, mc->S.as<double>(), solve_ld(pl->N), v, out, pl->N, pl->N, 1.0, 0);
+    matvec_rows(pl->ctx->stream, mc->S.as<double>(), solve_ld(pl->N), v, out, pl->N, pl->N);
 }
 
 // K (N x N column-major, overwritten by its LU factors; N = n, or the point

@@ -942,22 +942,27 @@ void transpose(hipStream_t st, const double* A, double* At, int rows, int cols, 
     ILH_HIP(hipGetLastError());
 }
 
-// One wave per row: y[i] = alpha * dot(M[i, :], x) (+ y[i]).  M row-major n x m
+// One wave per row: y[i] = alpha * dot(M[i, :], x) (+ add[i]).  M row-major n x m
 // with leading dimension ld (a multiple of 2, rows 16-byte aligned).
-__global__ void __launch_bounds__(256) k_matvec_rows(const double* __restrict__ M, int ld, const double* __restrict__ x, double* __restrict__ y,
-                              int n, int m, double alpha, int accumulate)
+__global__ void __launch_bounds__(256) k_matvec_rows(const double* __restrict__ M, int ld, const double* __restrict__ x,
+                              double* y, int n, int m, double alpha, const double* add /* may be y */,
+                              double* __restrict__ y2, int block)
 {
     const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (i >= n) return;
-    const double s = wave_dot(M + (size_t)ld * i, x, m, lane);
-    if (lane == 0) y[i] = alpha * s + (accumulate ? y[i] : 0.0);
+    const double s = wave_dot(M + (size_t)ld * i, block ? x + (size_t)(i / block) * block : x, m, lane);
+    if (lane == 0) {
+        const double t = alpha * s + (add ? add[i] : 0.0);
+        y[i] = t;
+        if (y2) y2[i] = t;
+    }
 }
 
 void matvec_rows(hipStream_t st, const double* M, int ld, const double* x, double* y, int n, int m, double alpha,
-                 int acc)
+                 const double* add, double* y2, int block)
 {
     if (n <= 0) return;
-    k_matvec_rows<<<(n + 3) / 4, 256, 0, st>>>(M, ld, x, y, n, m, alpha, acc);
+    k_matvec_rows<<<(n + 3) / 4, 256, 0, st>>>(M, ld, x, y, n, m, alpha, add, y2, block);
     ILH_HIP(hipGetLastError());
 }
 

@@ -769,7 +769,7 @@ void conv_sources_pair(ilh_plan* pl, int gk0, const SourceSet& src0, const doubl
 {
     ConvPlan& C0 = get_conv_sources(pl, gk0);
     ConvPlan& C1 = get_conv_sources(pl, gk1);
-    if (gk0 == gk1 || C0.Px != C1.Px || C0.Py != C1.Py || std::max(C0.Px, C0.Py) > PAIR_MAX_P || src0.npairs <= 0 ||
+    if (C0.Px != C1.Px || C0.Py != C1.Py || std::max(C0.Px, C0.Py) > PAIR_MAX_P || src0.npairs <= 0 ||
         src1.npairs <= 0) {
         conv_sources(pl, gk0, src0, amp0, out0);
         conv_sources(pl, gk1, src1, amp1, out1);
@@ -777,14 +777,21 @@ void conv_sources_pair(ilh_plan* pl, int gk0, const SourceSet& src0, const doubl
     }
     ConvPairArgs A{};
     const ConvPlan* C[2] = {&C0, &C1};
+    double2 *T1[2] = {C0.T1.as<double2>(), C1.T1.as<double2>()}, *T2[2] = {C0.T2.as<double2>(), C1.T2.as<double2>()};
+    if (&C0 == &C1) {   // two fields of one kind: the second one's spectra in the batches' buffers
+        C1.T1m.ensure(C1.T1.bytes);
+        C1.T2m.ensure(C1.T2.bytes);
+        T1[1] = C1.T1m.as<double2>();
+        T2[1] = C1.T2m.as<double2>();
+    }
     const SourceSet* src[2] = {&src0, &src1};
     const double* amp[2] = {amp0, amp1};
     double* out[2] = {out0, out1};
     for (int y = 0; y < 2; ++y) {
         A.S[y] = terms_source(*C[y], *src[y], amp[y]);
         A.npairs[y] = src[y]->npairs;
-        A.T1[y] = C[y]->T1.as<double2>();
-        A.T2[y] = C[y]->T2.as<double2>();
+        A.T1[y] = T1[y];
+        A.T2[y] = T2[y];
         A.slot[y] = src[y]->slot_of_row;
         A.spec[y] = C[y]->spec.as<double>();
         A.out[y] = out[y];

@@ -95,9 +95,11 @@ enum OpKind {
     OP_GSYM,           // surface_grad_symm!       Edges{Primal} -> VectorData
     OP_RNSYM,          // regularize_normal_symm!  VectorData -> EdgeGradient
     OP_NISYM,          // normal_interpolate_symm! EdgeGradient -> VectorData
+    OP_CDSYM,          // curl! of surface_divergence_symm!, from the points' (T_xx, T_xy) -> Nodes{Dual}
     OP_COUNT
 };
 int op_terms_per_point(int op);
+int op_amps_per_point(int op);   // amplitudes a point carries (2: VectorData, or two tensor components)
 bool op_is_scatter(int op);
 
 // Row-binned index of scatter terms on one component grid:
@@ -251,7 +253,14 @@ template <class T>
 void gather(ilh_plan* pl, const Term* terms, int nterms_per_point, const T* field, size_t field_stride, int nb,
             T* out, size_t out_stride);
 
+// e = E G phi and x = G^x_s phi of one Nodes{Primal} field in one launch, the
+// gradient's edge values taken from phi where the windows read them
+void gather_grad(ilh_plan* pl, const double* phi, const Term* termsE, int TE, double* e, const Term* termsX, int TX,
+                 double* x);
+
 // stencils (ilh_stencil.hip)
+// v = G phi - C t (edges), s = -(t + c) (Nodes{Dual})
+void k_stokes_fields(ilh_plan* pl, const double* phi, const double* t, const double* c, double* v, double* s);
 void k_divergence(ilh_plan* pl, double* p, const double* q);
 void k_grad(ilh_plan* pl, double* q, const double* p);
 void k_curl_n2e(ilh_plan* pl, double* q, const double* s);
@@ -317,8 +326,7 @@ void conv_stage(ilh_plan* pl, int gk, const SourceSet& src, const double* amp, d
 // the same convolution in split precision: forward transforms and the spectrum
 // product in FP64, the inverse transforms in FP32 (FP64 output)
 void conv_sources_f32(ilh_plan* pl, int gk, const SourceSet& src, const double* amp, double* out);
-// two source convolutions at once (different fields; one launch per pass where
-// their periods agree)
+// two source convolutions at once (one launch per pass where their periods agree)
 void conv_sources_pair(ilh_plan* pl, int gk0, const SourceSet& src0, const double* amp0, double* out0, int gk1,
                        const SourceSet& src1, const double* amp1, double* out1);
 // conv_sources into caller-supplied spectra buffers, allocating nothing
@@ -521,8 +529,11 @@ __device__ __forceinline__ double wave_dot(const double* __restrict__ row, const
     return s;
 }
 
+// y = alpha M x (+ add), row-major M of n rows and m columns; y2 (or null): a
+// second copy of y; block > 0: M is n / block blocks of `block` rows, block k
+// applied to x + k block
 void matvec_rows(hipStream_t st, const double* Mrow, int ld, const double* x, double* y, int n, int m,
-                 double alpha, int accumulate);
+                 double alpha = 1.0, const double* add = nullptr, double* y2 = nullptr, int block = 0);
 void dirichlet_amp(hipStream_t st, const double* Mp, const double* Mm, int ld, const double* fp,
                    const double* fm, double* amp, double* s_out, int n);
 void dirichlet_amp_multi(hipStream_t st, const double* Mp, const double* Mm, int ld, const double* fp,

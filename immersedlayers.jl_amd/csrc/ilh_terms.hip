@@ -244,6 +244,25 @@ __device__ __forceinline__ void k_build_terms_body(int op, int N, Grid g, const 
         }
         return;
     }
+    case OP_CDSYM: {
+        // C^T D_s^symm of the point's tensor (T_xx = -T_yy at p, T_xy = T_yx at
+        // N + p): with u = d_x T_xx + d_y T_xy and v = d_x T_yx + d_y T_yy as in
+        // OP_DSYM, w = d_x v - d_y u = -2 d_x d_y T_xx + (d_x d_x - d_y d_y) T_xy.
+        // A second difference of a 4-tap window has 6 taps, one more than a
+        // term holds: two terms, the first difference and its neighbour.
+        Term* o = out + 5 * (size_t)p;
+        const double r4 = r3 * i1;
+        const Win dPx = diff_win(Px, 0), dPy = diff_win(Py, 0);
+        Win dDx = diff_win(Dx, -1), dDy = diff_win(Dy, -1);
+        put(o[0], p, GK_DUAL, dPx, dPy, -2.0 * r4);
+        put(o[1], N + p, GK_DUAL, dDx, Dy, r4);
+        put(o[2], N + p, GK_DUAL, Dx, dDy, -r4);
+        dDx.b += 1;
+        dDy.b += 1;
+        put(o[3], N + p, GK_DUAL, dDx, Dy, -r4);
+        put(o[4], N + p, GK_DUAL, Dx, dDy, r4);
+        return;
+    }
     default: return;
     }
     out[2 * p] = a;
@@ -261,7 +280,17 @@ int op_terms_per_point(int op)
     switch (op) {
     case OP_R_PRIMAL: case OP_R_DUAL: case OP_E_PRIMAL: case OP_E_DUAL: return 1;
     case OP_DSYM: case OP_GSYM: case OP_RNSYM: case OP_NISYM: return 8;
+    case OP_CDSYM: return 5;
     default: return 2;
+    }
+}
+
+int op_amps_per_point(int op)
+{
+    switch (op) {
+    case OP_R_EDGES: case OP_E_EDGES: case OP_CVT: case OP_CVS: case OP_DSYM: case OP_GSYM: case OP_RNSYM:
+    case OP_NISYM: case OP_CDSYM: return 2;
+    default: return 1;
     }
 }
 
@@ -269,7 +298,7 @@ bool op_is_scatter(int op)
 {
     switch (op) {
     case OP_R_PRIMAL: case OP_R_DUAL: case OP_R_EDGES: case OP_RN: case OP_RNX:
-    case OP_DS: case OP_CST: case OP_CXT: case OP_CVT: case OP_DSYM: case OP_RNSYM: return true;
+    case OP_DS: case OP_CST: case OP_CXT: case OP_CVT: case OP_DSYM: case OP_RNSYM: case OP_CDSYM: return true;
     default: return false;
     }
 }
@@ -1257,19 +1286,13 @@ struct GatherFields {
 };
 
 // One wave per point: lane l takes the (term, row, column) triples l, l + 64,
-// ... of the point's T terms (T x 5 x 5), each the field value times coef wy
-// wx, into the partial sum of its term's amplitude slot; the wave then sums
-// the two slots' partials in a fixed butterfly order (bitwise reproducible).
-template <class D>
-__global__ void __launch_bounds__(256) k_gather(const Term* __restrict__ t, int T, int N, GatherFields<D> F,
-                                                size_t field_stride, D* __restrict__ out, size_t out_stride)
+// ... of the point's T terms (T x 5 x 5), each the field value (value(grid,
+// row, column), 0 off the grid) times coef wy wx, into the partial sum of its
+// term's amplitude slot; the wave then sums the two slots' partials in a fixed
+// butterfly order (bitwise reproducible).
+template <class D, class F>
+__device__ __forceinline__ void gather_point(const Term* __restrict__ tp, int T, int lane, F value, D* __restrict__ out)
 {
-    const int lane = threadIdx.x & 63;
-    const int p = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (p >= N) return;   // uniform over the wave
-    out += out_stride * blockIdx.y;
-    const size_t foff = field_stride * blockIdx.y;
-    const Term* tp = t + (size_t)p * T;
     // the point's amplitude indices, term k on lane k (T <= 64, checked by the
     // launcher): ai0 of term 0 and the first that differs from it, in one load
     // round trip
@@ -1281,12 +1304,9 @@ __global__ void __launch_bounds__(256) k_gather(const Term* __restrict__ t, int 
     for (int e = lane; e < T * 25; e += 64) {
         const int k = e / 25, r = e - 25 * k, b = r / 5, a = r - 5 * b;
         const Term& tt = tp[k];
-        const int gk = tt.gk, row = tt.by + b, col = tt.bx + a;
-        const int nx = F.nx[gk], ny = F.ny[gk];
         double v = 0.0;
         const double w = tt.wy[b] * tt.wx[a];
-        if (w != 0.0 && row >= 0 && row < ny && col >= 0 && col < nx)
-            v = tt.coef * w * (double)F.f[gk][foff + col + (size_t)nx * row];
+        if (w != 0.0) v = tt.coef * w * value(tt.gk, tt.by + b, tt.bx + a);
         if (tt.ai == ai0) acc0 += v;
         else acc1 += v;
     }
@@ -1298,6 +1318,67 @@ __global__ void __launch_bounds__(256) k_gather(const Term* __restrict__ t, int 
         out[ai0] = (D)acc0;
         if (ai1 >= 0) out[ai1] = (D)acc1;
     }
+}
+
+template <class D>
+__global__ void __launch_bounds__(256) k_gather(const Term* __restrict__ t, int T, int N, GatherFields<D> F,
+                                                size_t field_stride, D* __restrict__ out, size_t out_stride)
+{
+    const int p = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (p >= N) return;   // uniform over the wave
+    const size_t foff = field_stride * blockIdx.y;
+    gather_point<D>(t + (size_t)p * T, T, threadIdx.x & 63,
+                    [&](int gk, int row, int col) {
+                        const int nx = F.nx[gk], ny = F.ny[gk];
+                        if (row < 0 || row >= ny || col < 0 || col >= nx) return 0.0;
+                        return (double)F.f[gk][foff + col + (size_t)nx * row];
+                    },
+                    out + out_stride * blockIdx.y);
+}
+
+// The Stokes potential's two surface values, blockIdx.y = 0: E G phi (a wave
+// reads each edge value as the difference k_grad would have stored), 1: G^x_s
+// phi.  One launch on phi instead of a gradient over the grid and two gathers.
+__global__ void __launch_bounds__(256) k_gather_grad(const Term* __restrict__ tE, int TE, const Term* __restrict__ tX,
+                                                     int TX, int N, int NX, int NY, double dx,
+                                                     const double* __restrict__ phi, double* __restrict__ e,
+                                                     double* __restrict__ x)
+{
+    const int p = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (p >= N) return;   // uniform over the wave
+    const int np = NX - 1;
+    if (blockIdx.y == 0)
+        gather_point<double>(tE + (size_t)p * TE, TE, lane,
+                             [&](int gk, int row, int col) {
+                                 // the gradient is 0 on the outer faces
+                                 if (gk == GK_EDGE_U) {
+                                     if (row < 0 || row > NY - 2 || col < 1 || col > NX - 2) return 0.0;
+                                     const double* q = phi + col + (size_t)np * row;
+                                     return (q[0] - q[-1]) / dx;
+                                 }
+                                 if (row < 1 || row > NY - 2 || col < 0 || col > NX - 2) return 0.0;
+                                 const double* q = phi + col + (size_t)np * row;
+                                 return (q[0] - q[-np]) / dx;
+                             },
+                             e);
+    else
+        gather_point<double>(tX + (size_t)p * TX, TX, lane,
+                             [&](int, int row, int col) {
+                                 if (row < 0 || row > NY - 2 || col < 0 || col > NX - 2) return 0.0;
+                                 return phi[col + (size_t)np * row];
+                             },
+                             x);
+}
+
+void gather_grad(ilh_plan* pl, const double* phi, const Term* termsE, int TE, double* e, const Term* termsX, int TX,
+                 double* x)
+{
+    if (pl->N == 0) return;
+    if (TE < 1 || TE > 64 || TX < 1 || TX > 64) fail(ILH_ERR_ARG, "gather: terms per point must fit one wave");
+    const Grid& g = pl->g;
+    k_gather_grad<<<dim3((pl->N + 3) / 4, 2), 256, 0, pl->ctx->stream>>>(termsE, TE, termsX, TX, pl->N, g.NX, g.NY,
+                                                                         g.dx, phi, e, x);
+    ILH_HIP(hipGetLastError());
 }
 
 template <class D>
