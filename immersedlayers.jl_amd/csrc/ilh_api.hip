@@ -2549,6 +2549,16 @@ struct ArnLayout {
 };
 __host__ __device__ inline int arn_slices(int n) { return (n + 63) / 64; }
 
+// One work-group does step j on n points alone (k_arn_one) while its registers
+// hold the whole basis: 16 vectors of 2 entries a thread, 8 of 4.  One launch
+// takes 5.5-7 us to j = 7 and 9-10 us to j = 15 (1885 points; 421 points: 5.5
+// and 9), the three slice launches 15.4 us and two more launch gaps (about 18.5
+// us) whatever j; with vectors read again from memory at each use the one
+// work-group needed 20-28 us from j = 16, and 19-24 us for 2241 points from
+// j = 8.
+constexpr int ARN_T = 1024;
+__host__ __device__ inline bool arn_one_wg(int n, int j) { return j < (n <= 2 * ARN_T ? 16 : n <= 4 * ARN_T ? 8 : 0); }
+
 // one plan's Arnoldi operands (device pointers)
 struct ArnOp {
     double* V;
@@ -2625,7 +2635,7 @@ __global__ void __launch_bounds__(256) k_arn_dots(ArnOp one, const BGm* __restri
     const ArnOp A = arn_block<BAT>(one, g);
     const ArnLayout L{arn_slices(A.n), m};
     const int b = blockIdx.x;
-    if (b >= L.G) return;
+    if (b >= L.G || (BAT && arn_one_wg(A.n, j))) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nv = j + 1;
     const int k = 64 * b + lane;
     const bool in = k < A.n;
@@ -2696,7 +2706,7 @@ __global__ void __launch_bounds__(256) k_arn_update(ArnOp one, const BGm* __rest
     const ArnOp A = arn_block<BAT>(one, g);
     const ArnLayout L{arn_slices(A.n), m};
     const int b = blockIdx.x;
-    if (b >= L.G) return;
+    if (b >= L.G || (BAT && arn_one_wg(A.n, j))) return;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nv = j + 1;
     const int k = 64 * b + lane;
     const bool in = k < A.n;
@@ -2732,8 +2742,50 @@ __global__ void __launch_bounds__(256) k_arn_update(ArnOp one, const BGm* __rest
     arn_slice_dots(A, A.part + L.dots(1) + (size_t)(m + 2) * b, nv, nv, k, in, sw[lane], wave, lane);
 }
 
+// column j of H (col[0..j], |w| = hn below it): the rotations so far, a new one,
+// the residual norm and its test; one wave.  The rotations are a serial chain
+// along the column: each lane holds one rotation and one entry, and the chain
+// takes them by v_readlane (through memory every link waits for its loads).
+__device__ __forceinline__ void arn_column(double* __restrict__ st, const GmLayout& G, int* __restrict__ flags,
+                                           const double* __restrict__ col, const double* __restrict__ rc,
+                                           const double* __restrict__ rs, int j, int m, double hn, double gj, double tl,
+                                           double bn, int lane)
+{
+    double* H = st + G.H() + (size_t)(m + 1) * j;
+    double a = col[0];   // entry i of the column, rotated by rotations < i
+    for (int i0 = 0; i0 < j; i0 += 64) {
+        const bool in = i0 + lane < j;
+        const double c = in ? rc[i0 + lane] : 0.0, s = in ? rs[i0 + lane] : 0.0, x = in ? col[i0 + lane + 1] : 0.0;
+        const int cnt = min(64, j - i0);
+        double mine = 0.0;
+        for (int i = 0; i < cnt; ++i) {
+            const double ci = readlane_f64(c, i), si = readlane_f64(s, i), xi = readlane_f64(x, i);
+            const double y = ci * a + si * xi;
+            a = -si * a + ci * xi;
+            if (lane == i) mine = y;
+        }
+        if (in) H[i0 + lane] = mine;
+    }
+    if (lane != 0) return;
+    const double rr = hypot(a, hn);
+    const double cj = rr == 0.0 ? 1.0 : a / rr, sj = rr == 0.0 ? 0.0 : hn / rr;
+    H[j] = rr;
+    H[j + 1] = 0.0;
+    st[G.cs() + j] = cj;
+    st[G.sn() + j] = sj;
+    st[G.g() + j + 1] = -sj * gj;
+    st[G.g() + j] = cj * gj;
+    if (fabs(-sj * gj) <= tl * bn || hn == 0.0) {
+        flags[0] = 1;
+        flags[1] = j + 1;
+    } else if (j + 1 == m) {
+        flags[0] = 2;
+        flags[1] = m;
+    }
+}
+
 // the second pass if the test asks for it, |w|, v_{j+1} on the slice; slice 0
-// (one thread for the serial part, the column and rotations staged in LDS)
+// (one wave for the serial part, the column and rotations staged in LDS)
 // finishes column j of H.  Slices that start after slice 0 has set the flags
 // skip v_{j+1}, which a stopped iteration never reads.
 template <bool BAT>
@@ -2746,7 +2798,7 @@ __global__ void __launch_bounds__(256) k_arn_final(ArnOp one, const BGm* __restr
     const ArnOp A = arn_block<BAT>(one, g);
     const ArnLayout L{arn_slices(A.n), m};
     const int b = blockIdx.x;
-    if (b >= L.G) return;
+    if (b >= L.G || (BAT && arn_one_wg(A.n, j))) return;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nv = j + 1;
     const int k = 64 * b + lane;
     const bool in = k < A.n;
@@ -2770,7 +2822,7 @@ __global__ void __launch_bounds__(256) k_arn_final(ArnOp one, const BGm* __restr
             rc[t] = st[G.cs() + t];
             rs[t] = st[G.sn() + t];
         }
-        if (t == 0) {
+        if (wave == 0) {
             gj = st[G.g() + j];
             tl = st[G.tol()];
             bn = st[G.bnorm()];
@@ -2799,40 +2851,212 @@ __global__ void __launch_bounds__(256) k_arn_final(ArnOp one, const BGm* __restr
     if (b != 0) return;
     if (ht) col[t] = c0 + (again ? h[t] : 0.0);
     __syncthreads();
-    if (t == 0) {
-        col[j + 1] = hn;
-        double a = col[0];   // entry i of the column, rotated by rotations < i
-        for (int i = 0; i < j; ++i) {
-            const double c = col[i + 1];
-            col[i] = rc[i] * a + rs[i] * c;
-            a = -rs[i] * a + rc[i] * c;
+    if (wave == 0) arn_column(st, G, A.flags, col, rc, rs, j, m, hn, gj, tl, bn, lane);
+}
+
+// ---- The same step in one work-group of 1024 threads, one launch, for the
+// first steps (arn_one_wg).  Bound by latency: the basis is read once (200 KB
+// at most) and kept in registers through its four uses, the dots and the
+// subtraction of both passes; thread t holds entries t + 1024 e of w and of CH
+// vectors (those past v_j are zeros).  The CH dots are reduced together: each
+// halving step pairs two vectors' partials, so CH sums over a wave take CH + 1
+// exchanges (CH = 16: 17) instead of 6 CH; the 16 waves' sums are added in wave
+// order.  Every sum has a fixed order.
+// The exchanges stay in the vector ALU (row swaps and DPP moves): through the
+// LDS the 16 waves of the work-group queue up for it.
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double x)
+{
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E;              // quad_perm [1,0,3,2], [2,3,0,1]
+constexpr int DPP_MIRROR8 = 0x141, DPP_ROR8 = 0x128;         // lane ^ 7, lane ^ 8 of a row of 16
+
+// a + (the value of a in the lane's partner half), for a in the lower halves
+// and b in the upper ones: halves of 64 (SPAN 32) or of each 32 (SPAN 16)
+template <int SPAN>
+__device__ __forceinline__ double swap_add(double a, double b)
+{
+    auto sw = [](unsigned x, unsigned y) {
+        if constexpr (SPAN == 32) return __builtin_amdgcn_permlane32_swap(x, y, false, false);
+        else return __builtin_amdgcn_permlane16_swap(x, y, false, false);
+    };
+    const auto lo = sw((unsigned)__double2loint(a), (unsigned)__double2loint(b));
+    const auto hi = sw((unsigned)__double2hiint(a), (unsigned)__double2hiint(b));
+    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+
+// the sum over the wave's 64 lanes, in every lane
+__device__ __forceinline__ double wave_sum_alu(double a)
+{
+    a += dpp_f64<DPP_XOR1>(a);
+    a += dpp_f64<DPP_XOR2>(a);
+    a += dpp_f64<DPP_MIRROR8>(a);
+    a += dpp_f64<DPP_ROR8>(a);
+    a = swap_add<16>(a, a);
+    return swap_add<32>(a, a);
+}
+
+// p[v] summed over the wave; lane l gets the sum of vector l / (64 / CH)
+template <int CH>
+__device__ __forceinline__ double wave_sums(double (&p)[CH], int lane)
+{
+    static_assert(CH == 4 || CH == 8 || CH == 16, "vectors per chunk");
+#pragma unroll
+    for (int u = 0; u < CH / 2; ++u) p[u] = swap_add<32>(p[u], p[u + CH / 2]);
+#pragma unroll
+    for (int u = 0; u < CH / 4; ++u) p[u] = swap_add<16>(p[u], p[u + CH / 4]);
+    if constexpr (CH >= 8) {
+        const bool up = (lane & 8) != 0;
+#pragma unroll
+        for (int u = 0; u < CH / 8; ++u) {
+            const double keep = up ? p[u + CH / 8] : p[u], send = up ? p[u] : p[u + CH / 8];
+            p[u] = keep + dpp_f64<DPP_ROR8>(send);
         }
-        col[j] = a;
-        const double rr = hypot(col[j], col[j + 1]);
-        const double cj = rr == 0.0 ? 1.0 : col[j] / rr, sj = rr == 0.0 ? 0.0 : col[j + 1] / rr;
-        col[j] = rr;
-        col[j + 1] = 0.0;
-        double* H = st + G.H() + (size_t)(m + 1) * j;
-        for (int i = 0; i <= j + 1; ++i) H[i] = col[i];
-        st[G.cs() + j] = cj;
-        st[G.sn() + j] = sj;
-        st[G.g() + j + 1] = -sj * gj;
-        st[G.g() + j] = cj * gj;
-        int* flags = A.flags;
-        if (fabs(-sj * gj) <= tl * bn || hn == 0.0) {
-            flags[0] = 1;
-            flags[1] = j + 1;
-        } else if (j + 1 == m) {
-            flags[0] = 2;
-            flags[1] = m;
+    } else {
+        p[0] += dpp_f64<DPP_ROR8>(p[0]);
+    }
+    if constexpr (CH >= 16) {
+        const bool up = (lane & 4) != 0;
+        const double keep = up ? p[1] : p[0], send = up ? p[0] : p[1];
+        p[0] = keep + dpp_f64<DPP_MIRROR8>(send);
+    } else {
+        p[0] += dpp_f64<DPP_MIRROR8>(p[0]);
+    }
+    p[0] += dpp_f64<DPP_XOR2>(p[0]);
+    p[0] += dpp_f64<DPP_XOR1>(p[0]);
+    return p[0];
+}
+
+struct ArnOneLds {
+    double red[16][16];    // each wave's dots
+    double nrm[2][16];     // each wave's w . w, |w1|^2
+    double h[2][16];       // the passes' coefficients
+    double rc[16], rs[16];
+    double col[16];
+};
+
+template <int E, int CH>
+__device__ __forceinline__ void arn_one_body(const ArnOp& A, int j, int m, ArnOneLds& S)
+{
+    auto& red = S.red;
+    auto& nrm = S.nrm;
+    auto& h = S.h;
+    auto &rc = S.rc, &rs = S.rs;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, nv = j + 1, n = A.n;
+    const GmLayout G{m};
+    double* st = A.st;
+    // every load that depends on nothing, before the flags' test
+    double w[E], x[CH][E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) w[e] = t + ARN_T * e < n ? A.w[t + ARN_T * e] : 0.0;
+#pragma unroll
+    for (int u = 0; u < CH; ++u)
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int k = t + ARN_T * e;
+            x[u][e] = k < n && u < nv ? A.V[(size_t)A.ld * u + k] : 0.0;
         }
+    if (t < j) {
+        rc[t] = st[G.cs() + t];
+        rs[t] = st[G.sn() + t];
+    }
+    double gj = 0.0, tl = 0.0, bn = 0.0;
+    if (wave == 0) {
+        gj = st[G.g() + j];
+        tl = st[G.tol()];
+        bn = st[G.bnorm()];
+    }
+    if (A.flags[0]) return;
+    // hp = V^T w summed over the work-group, |w|^2 beside it
+    auto dots = [&](double* hp, double* np) {
+        double p[CH], q = 0.0;
+#pragma unroll
+        for (int u = 0; u < CH; ++u) {
+            p[u] = 0.0;
+#pragma unroll
+            for (int e = 0; e < E; ++e) p[u] = __builtin_fma(x[u][e], w[e], p[u]);
+        }
+        const double d = wave_sums<CH>(p, lane);
+        if (lane % (64 / CH) == 0) red[wave][lane / (64 / CH)] = d;
+#pragma unroll
+        for (int e = 0; e < E; ++e) q = __builtin_fma(w[e], w[e], q);
+        q = wave_sum_alu(q);
+        if (lane == 0) np[wave] = q;
+        __syncthreads();
+        if (t < nv) {
+            double a = 0.0;
+#pragma unroll
+            for (int u = 0; u < 16; ++u) a += red[u][t];
+            hp[t] = a;
+        }
+        __syncthreads();
+    };
+    // w -= V hp, vectors in order
+    auto subtract = [&](const double* hp) {
+#pragma unroll
+        for (int u = 0; u < CH; ++u)
+            if (u < nv) {
+                const double hu = hp[u];
+#pragma unroll
+                for (int e = 0; e < E; ++e) w[e] = __builtin_fma(-hu, x[u][e], w[e]);
+            }
+    };
+    dots(h[0], nrm[0]);
+    subtract(h[0]);
+    dots(h[1], nrm[1]);
+    double ww = 0.0, q0 = 0.0;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        ww += nrm[0][u];
+        q0 += nrm[1][u];
+    }
+    const bool again = arn_again(ww, q0);
+    double hn = sqrt(q0);
+    if (again) {
+        const double hl = lane < nv ? h[1][lane] : 0.0;
+        const double hh = wave_sum_alu(hl * hl);   // |h'|^2
+        hn = sqrt(fmax(q0 - hh, 0.0));
+        subtract(h[1]);
+    }
+    if (hn > 0.0) {
+        const double inv = 1.0 / hn;
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            if (t + ARN_T * e < n) A.V[(size_t)A.ld * nv + t + ARN_T * e] = w[e] * inv;
+    }
+    if (wave == 0) {
+        if (lane < nv) S.col[lane] = h[0][lane] + (again ? h[1][lane] : 0.0);   // for this wave alone
+        arn_column(st, G, A.flags, S.col, rc, rs, j, m, hn, gj, tl, bn, lane);
     }
 }
 
-// the three launches of Arnoldi step j (grid: slices, plans)
 template <bool BAT>
-static void arn_step(hipStream_t st, const ArnOp& one, const BGm* g, dim3 grid, int j, int m)
+__global__ void __launch_bounds__(ARN_T) k_arn_one(ArnOp one, const BGm* __restrict__ g, int j, int m)
 {
+    const ArnOp A = arn_block<BAT>(one, g);
+    if (!arn_one_wg(A.n, j)) return;
+    __shared__ ArnOneLds S;
+    if (A.n <= 2 * ARN_T) {
+        if (j < 4) arn_one_body<2, 4>(A, j, m, S);
+        else if (j < 8) arn_one_body<2, 8>(A, j, m, S);
+        else arn_one_body<2, 16>(A, j, m, S);
+    } else {
+        if (j < 4) arn_one_body<4, 4>(A, j, m, S);
+        else arn_one_body<4, 8>(A, j, m, S);
+    }
+}
+
+// the launches of Arnoldi step j: the plans (np of them, nmin to nmax points)
+// that one work-group does, and those that take the slices
+template <bool BAT>
+static void arn_step(hipStream_t st, const ArnOp& one, const BGm* g, int np, int nmin, int nmax, int j, int m)
+{
+    if (arn_one_wg(nmin, j)) k_arn_one<BAT><<<dim3(1, (unsigned)np), ARN_T, 0, st>>>(one, g, j, m);
+    if (arn_one_wg(nmax, j)) return;
+    const dim3 grid((unsigned)arn_slices(nmax), (unsigned)np);
     k_arn_dots<BAT><<<grid, 256, 0, st>>>(one, g, j, m);
     k_arn_update<BAT><<<grid, 256, 0, st>>>(one, g, j, m);
     k_arn_final<BAT><<<grid, 256, 0, st>>>(one, g, j, m);
@@ -3145,7 +3369,7 @@ static void gm_issue(ilh_plan* pl, MovingCache* mc, int j0, int j1, int m)
     for (int j = j0; j < j1; ++j) {
         prec_apply(pl, mc, V + (size_t)ld * j, mc->z.as<double>(), flags, 0);
         k_gm_matvec<<<gR, 256, 0, st>>>(mc->S.as<double>(), ld, mc->z.as<double>(), mc->w.as<double>(), N, flags);
-        arn_step<false>(st, A, nullptr, dim3((unsigned)arn_slices(N)), j, m);
+        arn_step<false>(st, A, nullptr, 1, N, N, j, m);
     }
     ILH_HIP(hipGetLastError());
     ILH_HIP(hipMemcpyAsync(mc->pinned(1), flags, 2 * sizeof(int), hipMemcpyDeviceToHost, st));
@@ -3496,7 +3720,7 @@ extern "C" int ilh_dirichlet_solve_moving_batched(int nprob, ilh_plan* const* pl
         std::vector<BGm> hg;
         std::vector<int> gi;   // plan of each descriptor
         std::vector<unsigned> tiles;
-        int chunk = 1, maxn = 1;
+        int chunk = 1, maxn = 1, minn = 1 << 30;
         for (int i = 0; i < nprob; ++i) {
             if (!mc[i]) continue;
             ilh_plan* pl = plans[i];
@@ -3534,6 +3758,7 @@ extern "C" int ilh_dirichlet_solve_moving_batched(int nprob, ilh_plan* const* pl
             gi.push_back(i);
             chunk = std::max(chunk, std::min(m, c->last_iters));
             maxn = std::max(maxn, pl->N);
+            minn = std::min(minn, pl->N);
         }
         const int nd = (int)hg.size();
         if (nd > 0) {
@@ -3581,7 +3806,7 @@ extern "C" int ilh_dirichlet_solve_moving_batched(int nprob, ilh_plan* const* pl
                 for (int jj = j; jj < j1; ++jj) {
                     k_bgm_prec<<<nt, 128, 0, main>>>(dg, dt, jj);
                     k_bgm_matvec<<<nt, 256, 0, main>>>(dg, dt);
-                    arn_step<true>(main, ArnOp{}, dg, dim3((unsigned)arn_slices(maxn), (unsigned)nd), jj, m);
+                    arn_step<true>(main, ArnOp{}, dg, nd, minn, maxn, jj, m);
                 }
                 k_bgm_flags<<<(unsigned)((nd + 255) / 256), 256, 0, main>>>(dg, nd, df);
                 ILH_HIP(hipGetLastError());
