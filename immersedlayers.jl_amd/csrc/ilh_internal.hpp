@@ -141,6 +141,12 @@ struct DevBuf {
     ~DevBuf() { release(); }
 };
 
+// part of a DevBuf
+struct DevView {
+    void* p = nullptr;
+    template <class T> T* as() const { return (T*)p; }
+};
+
 // Zero-padded FFT convolution with the LGF on one grid kind.
 struct ConvPlan {
     int gk = 0;
@@ -193,7 +199,8 @@ struct ilh_plan {
     int N = 0;
     int ddf = 0;
     int min_margin = 0;       // cells between the point supports and the grid edge
-    ilh::DevBuf X, Y, nx, ny, ds;            // device geometry
+    ilh::DevBuf geo;                          // device geometry: the five arrays below, one behind the other
+    ilh::DevView X, Y, nx, ny, ds;
     ilh::DevBuf terms[ilh::OP_COUNT];        // per-op term arrays (built lazily)
     bool terms_ok[ilh::OP_COUNT] = {};
     ilh::DevBuf wins;                         // DDF windows of each point (primal x, y, dual x, y)
