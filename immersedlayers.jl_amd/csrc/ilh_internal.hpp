@@ -225,6 +225,11 @@ struct ilh_plan {
     unsigned mask_gen = ~0u;                  // generation the mask belongs to
     ilh::DevBuf filt_r1;                      // R 1 on Nodes{Primal} for the surface filter
     unsigned filt_gen = ~0u;
+    // the surface filter C as rows of at most FILT_CAP entries: weights and
+    // columns by slot ([slot][point]), row lengths; filt_len < 0: a row has more
+    ilh::DevBuf filt_w, filt_q;
+    int filt_len = -1;
+    unsigned filt_gen_rows = ~0u;
     ilh::DevBuf filt_r1e;                     // R 1 on Edges{Primal} for the vector surface filter
     unsigned filt_gen_e = ~0u;
     std::atomic<int> refs{1};                 // the caller's handle, batches and heat integrators using it
