@@ -118,8 +118,8 @@ struct StokesCache {
     DevBuf sv;                    // surface work (SW_* below)
     DevBuf gP;                    // phi
     DevBuf gDD;                   // two Nodes{Dual} fields back to back (y, then t; c)
-    DevBuf terms[3];              // merged source terms of src
-    SourceSet src[3];             // R (phi); [C^T D_s^symm, C_s^T] (y); C^x_s^T (c)
+    DevBuf terms[2];              // merged source terms of src
+    SourceSet src[2];             // [C^T D_s^symm, C_s^T] (y); C^x_s^T (c)
     ~StokesCache()
     {
         for (SourceSet& q : src) free_sources(q);
@@ -1926,9 +1926,9 @@ extern "C" int ilh_surface_filter_apply_vector(ilh_plan* pl, int power, const do
 // streamfunction c = L^-1 C^x_s^T Ss^-1 G^x_s phi as one pair, both straight
 // from the points' terms; t = L^-1 y.  At the sizes this runs at (a few hundred
 // cells a side) every launch is 3-9 us of latency whatever it does, so the
-// solve is arranged for few launches: 16 and one per filter power, where
+// solve is arranged for few launches: 17 and one per filter power, where
 // operator by operator they were 28 and two (406^2, 214 points, power 2:
-// 134 -> 94 us).
+// 136 -> 96 us).
 namespace {
 // surface quantities of the prescribed velocities: [v], v_bar, n . [v] and the
 // symmetric surface tensor's T_xx, T_xy (OP_CDSYM's amplitudes)
@@ -2037,9 +2037,8 @@ StokesCache* prepare_stokes(ilh_plan* pl)
             build_stokes_ka(pl, K.as<double>());
             sc->Ka.ensure(sizeof(double) * (size_t)n2 * solve_ld(n2));
             transpose(pl->ctx->stream, K.as<double>(), sc->Ka.as<double>(), n2, n2, solve_ld(n2));
-            merge_sources(pl, OP_R_PRIMAL, -1, GK_PRIMAL, sc->terms[0], sc->src[0]);
-            merge_sources(pl, OP_CDSYM, OP_CVT, GK_DUAL, sc->terms[1], sc->src[1]);
-            merge_sources(pl, OP_CXT, -1, GK_DUAL, sc->terms[2], sc->src[2]);
+            merge_sources(pl, OP_CDSYM, OP_CVT, GK_DUAL, sc->terms[0], sc->src[0]);
+            merge_sources(pl, OP_CXT, -1, GK_DUAL, sc->terms[1], sc->src[1]);
             for (SourceSet& q : sc->src) pin_source_pairs(pl, q);
             ILH_HIP(hipStreamSynchronize(pl->ctx->stream));
         }
@@ -2084,8 +2083,13 @@ extern "C" int ilh_stokes_solve(ilh_plan* pl, const double* v_plus, const double
             k_stokes_rhs<<<(N + 127) / 128, 128, 0, st>>>(N, d_vp, d_vm, pl->nx.as<double>(), pl->ny.as<double>(), dv,
                                                           vb, dvn, tt);
             ILH_HIP(hipGetLastError());
-            // phi = L^-1 R (n . [v]);  E v_phi = E G phi and G^x_s phi on the points
-            conv_sources(pl, GK_PRIMAL, sc->src[0], dvn, gP);
+            // phi = L^-1 R (n . [v]);  E v_phi = E G phi and G^x_s phi on the points.
+            // phi comes from the grid and the full period: S's smallest singular
+            // direction amplifies the rounding of E G phi 1e7-fold into s's
+            // constant, and from the points' terms (2.4 us less) its error
+            // against 64-bit results was up to twice as large
+            scatter_op(pl, OP_R_PRIMAL, dvn, gP);
+            conv_dense(pl, GK_PRIMAL, gP, gP);
             gather_grad(pl, gP, get_terms(pl, OP_E_EDGES), op_terms_per_point(OP_E_EDGES), ephi,
                         get_terms(pl, OP_GXS), op_terms_per_point(OP_GXS), dsv);
             k_stokes_vprime<<<(3 * N + 3) / 4, 256, 0, st>>>(N, sc->Ka.as<double>(), ld2, dv, vb, ephi, vpr,
@@ -2100,7 +2104,7 @@ extern "C" int ilh_stokes_solve(ilh_plan* pl, const double* v_plus, const double
                         filter_power == 0 ? sig_out : nullptr);
             // y = L^-1 (C^T D_s^symm [v] + C_s^T sigma) and c = L^-1 C^x_s^T ds,
             // the streamfunction of the potential's sources
-            conv_sources_pair(pl, GK_DUAL, sc->src[1], tt, gD, GK_DUAL, sc->src[2], dsn, gD2);
+            conv_sources_pair(pl, GK_DUAL, sc->src[0], tt, gD, GK_DUAL, sc->src[1], dsn, gD2);
             // t = L^-1 y;  v = G phi - C t,  s = -(t + c)
             conv_dense(pl, GK_DUAL, gD, gD);
             k_stokes_fields(pl, gP, gD, gD2, d_v, d_s);
