@@ -151,7 +151,7 @@ struct DevView {
 struct ConvPlan {
     int gk = 0;
     int nx = 0, ny = 0;       // field dims
-    int Px = 0, Py = 0;       // padded periods (powers of two, >= 2n-2)
+    int Px = 0, Py = 0;       // padded periods (powers of two: >= 2n-2, less for sources of known extent)
     int H = 0;                // Px/2: half-spectrum columns (column 0 packs DC and Nyquist)
     DevBuf spec;              // real spectrum * dx^2/(Px*Py): [kx][ky], kx <= H, ky <= Py/2 (even in ky)
     DevBuf spec32;            // the same rounded to FP32 (the FP32 passes), built on first use
