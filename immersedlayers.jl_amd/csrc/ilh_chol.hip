@@ -64,13 +64,13 @@ struct GemmBatch {
     int m_total = 0, m_step = 0;
     int k_is_m = 0;
 };
-// Epilogues: EPI_RANK1 C = alpha AB - 2 u[m] v[n]; EPI_DEFLATE
-// C = (AB - a[m] u[n] - 2 b[m] w[n]) / (c d[n]).
-enum { EPI_NONE = 0, EPI_RANK1 = 1, EPI_DEFLATE = 2 };
+// Epilogues: EPI_RANK1 C = alpha AB - 2 u[m] v[n]; EPI_DOT C = AB, and the sums
+// of C[m, n] v[n] over each 32 columns of a tile at dots + M (2 n-tile + half)
+// (for gridDim.z = 1).
+enum { EPI_NONE = 0, EPI_RANK1 = 1, EPI_DOT = 2 };
 struct GemmEpi {
-    const double *u = nullptr, *v = nullptr;                                         // EPI_RANK1
-    const double *a = nullptr, *b = nullptr, *wt = nullptr, *w1 = nullptr, *d = nullptr;   // EPI_DEFLATE
-    double c = 1.0;
+    const double *u = nullptr, *v = nullptr;
+    double* dots = nullptr;
 };
 
 template <int TA, int TB, bool BETA0, int EPI>
@@ -199,10 +199,21 @@ __global__ void __launch_bounds__(256) k_dgemm(int M, int Nc, int K, double alph
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int gm = m0 + wm + 16 * i + (lane & 15);
+        if (EPI == EPI_DOT) {
+            double q = 0.0;
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int gn = n0 + wn + 16 * j + (lane >> 4) + 4 * r;
+                    if (gn < Nc) q = __builtin_fma(acc[i][j][r], ep.v[gn], q);
+                }
+            q += __shfl_xor(q, 16, 64);
+            q += __shfl_xor(q, 32, 64);
+            if (lane < 16 && gm < M) ep.dots[gm + (size_t)M * (2 * by + (wave >> 1))] = q;
+        }
         if (gm >= M) continue;
-        double e0 = 0.0, e1 = 0.0;
-        if (EPI == EPI_RANK1) e0 = ep.u[gm];
-        if (EPI == EPI_DEFLATE) { e0 = ep.a[gm]; e1 = ep.b[gm]; }
+        const double e0 = EPI == EPI_RANK1 ? ep.u[gm] : 0.0;
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -211,8 +222,6 @@ __global__ void __launch_bounds__(256) k_dgemm(int M, int Nc, int K, double alph
                 if (gn >= Nc) continue;
                 double* p = C + gm + (size_t)ldc * gn;
                 if (EPI == EPI_RANK1) *p = alpha * acc[i][j][r] - 2.0 * e0 * ep.v[gn];
-                else if (EPI == EPI_DEFLATE)
-                    *p = (acc[i][j][r] - e0 * ep.wt[gn] - 2.0 * e1 * ep.w1[gn]) / (ep.c * ep.d[gn]);
                 else *p = BETA0 ? alpha * acc[i][j][r] : *p + alpha * acc[i][j][r];
             }
     }
@@ -608,35 +617,18 @@ __global__ void __launch_bounds__(1024) k_wmv(const double* __restrict__ W, int 
     }
 }
 
-// z_v[p] = sum_{k >= p} W[k + m p] T[k + ldt v], v < NV, one wave per column
-// p; written as Z[p + ldz v], or (wt given) through the deflated solve's last
-// step, Out[v + ldo (p + 1)] = (z - a[v] wt[p] - 2 b[v] w1[p]) / (c d[p + 1]).
-template <int NV>
-__global__ void __launch_bounds__(256) k_wtmv(const double* __restrict__ W, int m, const double* __restrict__ T, int ldt,
-                                              double* __restrict__ Z, int ldz, const double* __restrict__ a,
-                                              const double* __restrict__ b, const double* __restrict__ wt,
-                                              const double* __restrict__ w1, const double* __restrict__ d, double c)
+// Z[p] = sum_{k >= p} W[k + m p] T[k], one wave per column p
+__global__ void __launch_bounds__(256) k_wtmv(const double* __restrict__ W, int m, const double* __restrict__ T,
+                                              double* __restrict__ Z)
 {
     const int p = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (p >= m) return;
     const double* col = W + (size_t)m * p;
-    double acc[NV];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) acc[v] = 0.0;
+    double acc = 0.0;
 #pragma unroll 8
-    for (int k = p + lane; k < m; k += 64) {
-        const double w = col[k];
-#pragma unroll
-        for (int v = 0; v < NV; ++v) acc[v] = __builtin_fma(w, T[k + (size_t)ldt * v], acc[v]);
-    }
-#pragma unroll
-    for (int v = 0; v < NV; ++v) {
-        for (int off = 32; off > 0; off >>= 1) acc[v] += __shfl_xor(acc[v], off, 64);
-        if (lane == 0) {
-            if (wt) Z[v + (size_t)ldz * (p + 1)] = (acc[v] - a[v] * wt[p] - 2.0 * b[v] * w1[p]) / (c * d[p + 1]);
-            else Z[p + (size_t)ldz * v] = acc[v];
-        }
-    }
+    for (int k = p + lane; k < m; k += 64) acc = __builtin_fma(col[k], T[k], acc);
+    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+    if (lane == 0) Z[p] = acc;
 }
 
 // --------------------------------------------------- deflated symmetric solve
@@ -706,29 +698,26 @@ __global__ void k_defl_vecs(const double* __restrict__ w, const double* __restri
     xt[m + i] = A[1 + i];
 }
 
-// sig = {alpha - beta . wt, w1 . wt, w1 . ut}
+// sig = {alpha - beta . wt, w1 . wt}
 __global__ void __launch_bounds__(1024) k_sigma(const double* __restrict__ A, const double* __restrict__ xt,
-                                                const double* __restrict__ ut, const double* __restrict__ wt, int m,
-                                                double* __restrict__ sig)
+                                                const double* __restrict__ wt, int m, double* __restrict__ sig)
 {
-    __shared__ double red[3][1024];
-    double s[3] = {0.0, 0.0, 0.0};
+    __shared__ double red[2][1024];
+    double s[2] = {0.0, 0.0};
     for (int i = threadIdx.x; i < m; i += 1024) {
         s[0] += xt[m + i] * wt[i];
         s[1] += xt[i] * wt[i];
-        s[2] += xt[i] * ut[i];
     }
-    for (int v = 0; v < 3; ++v) red[v][threadIdx.x] = s[v];
+    for (int v = 0; v < 2; ++v) red[v][threadIdx.x] = s[v];
     __syncthreads();
     for (int off = 512; off > 0; off >>= 1) {
         if ((int)threadIdx.x < off)
-            for (int v = 0; v < 3; ++v) red[v][threadIdx.x] += red[v][threadIdx.x + off];
+            for (int v = 0; v < 2; ++v) red[v][threadIdx.x] += red[v][threadIdx.x + off];
         __syncthreads();
     }
     if (threadIdx.x == 0) {
         sig[0] = A[0] - red[0][0];
         sig[1] = red[1][0];
-        sig[2] = red[2][0];
     }
 }
 
@@ -739,17 +728,17 @@ bool sym_factor(ilh_plan* pl, SymFactor& F, int n, double* scratch, bool deflate
     F.ok = false;
     const int m = n - 1, mc = std::max(m, 1);
     F.w.ensure(sizeof(double) * (size_t)n);
-    F.vec.ensure(sizeof(double) * (size_t)(2 * n + 6 * mc));
+    F.vec.ensure(sizeof(double) * (size_t)(2 * n + 5 * mc));
     F.W.ensure(sizeof(double) * (size_t)mc * mc);
     F.T.ensure(sizeof(double) * (size_t)mc * n);   // also the product W B of a full solve
-    F.info.ensure(4 * sizeof(double));   // {sigma, w1.wt, w1.ut}, then the pivot flag
+    F.info.ensure(3 * sizeof(double));   // {sigma, w1.wt}, then the pivot flag
     double* A = F.A.as<double>();
     double* w = F.w.as<double>();
     double* y = F.vec.as<double>();
     double* p = y + n;
-    double *xt = F.xt(), *wx = F.ww(), *zt = F.ut();
+    double *xt = F.xt(), *wx = F.ww();
     double* sig = F.info.as<double>();
-    int* info = (int*)(sig + 3);
+    int* info = (int*)(sig + 2);
     k_house_vec<<<(n + 255) / 256, 256, 0, st>>>(w, n, deflate, info);
     if (deflate) {
         k_symv<<<(n + 3) / 4, 256, 0, st>>>(A, n, n, w, y);
@@ -761,66 +750,108 @@ bool sym_factor(ilh_plan* pl, SymFactor& F, int n, double* scratch, bool deflate
         chol_factor(st, A + 1 + (size_t)n, n, m, F.W.as<double>(), scratch, F.T.as<double>(), info);
         k_defl_vecs<<<(m + 255) / 256, 256, 0, st>>>(w, A, m, xt);
         k_wmv<2><<<(m + 15) / 16, 1024, 0, st>>>(F.W.as<double>(), m, xt, m, nullptr, nullptr, wx, m);
-        k_wtmv<2><<<(m + 3) / 4, 256, 0, st>>>(F.W.as<double>(), m, wx, m, zt, m, nullptr, nullptr, nullptr, nullptr,
-                                               nullptr, 1.0);
+        k_wtmv<<<(m + 3) / 4, 256, 0, st>>>(F.W.as<double>(), m, wx + m, F.wt());
     }
-    k_sigma<<<1, 1024, 0, st>>>(A, xt, F.ut(), F.wt(), m, sig);
+    k_sigma<<<1, 1024, 0, st>>>(A, xt, F.wt(), m, sig);
     ILH_HIP(hipGetLastError());
-    double h[4];
+    double h[3];
     ILH_HIP(hipMemcpyAsync(h, sig, sizeof(h), hipMemcpyDeviceToHost, st));
     ILH_HIP(hipStreamSynchronize(st));
     int bad;
-    std::memcpy(&bad, h + 3, sizeof(bad));
+    std::memcpy(&bad, h + 2, sizeof(bad));
     if (bad || !(h[0] != 0.0) || !std::isfinite(h[0])) return false;
     F.ok = true;
     return true;
 }
 
-// The scalars of each column j of the deflated solve M^-1 B (B n x ncols), one
-// wave per column:  r = w . B, y1 = (X'0 - wt . X'1) / sigma and
-// t = w . [y1; Z - wt y1] with X' = B - 2 w r, Z = Mt^-1 X'1 (w1 . Z = ut . X'1),
-// and the solution's first row, Out[j] = (y1 - 2 w0 t) / (c d0).
+// The first scalars of each column j of the deflated solve M^-1 B (B n x ncols),
+// one wave per column:  r = w . B and y1 = (X'0 - wt . X'1) / sigma with
+// X' = B - 2 w r.
 __global__ void __launch_bounds__(256) k_defl_cols(const double* __restrict__ w, const double* __restrict__ wt,
-                                                   const double* __restrict__ ut, const double* __restrict__ sig,
-                                                   const double* B, int n, int ncols, double* __restrict__ rv,
-                                                   double* __restrict__ y1v, double* __restrict__ tv, double* Out,
-                                                   const double* __restrict__ d, double c)
+                                                   const double* __restrict__ sig, const double* __restrict__ B, int n,
+                                                   int ncols, double* __restrict__ rv, double* __restrict__ y1v)
 {
     const int j = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (j >= ncols) return;
     const double* col = B + (size_t)n * j;
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+    double s0 = 0.0, s1 = 0.0;
 #pragma unroll 4
     for (int i = 1 + lane; i < n; i += 64) {
         const double b = col[i];
         s0 = __builtin_fma(w[i], b, s0);
         s1 = __builtin_fma(wt[i - 1], b, s1);
-        s2 = __builtin_fma(ut[i - 1], b, s2);
     }
     for (int off = 32; off > 0; off >>= 1) {
         s0 += __shfl_xor(s0, off, 64);
         s1 += __shfl_xor(s1, off, 64);
-        s2 += __shfl_xor(s2, off, 64);
     }
     if (lane == 0) {
         const double w0 = w[0], b0 = col[0];
         const double r = s0 + w0 * b0;
-        const double y1 = ((b0 - 2.0 * w0 * r) - (s1 - 2.0 * sig[1] * r)) / sig[0];
-        const double t = w0 * y1 + (s2 - 2.0 * sig[2] * r) - sig[1] * y1;
         rv[j] = r;
-        y1v[j] = y1;
-        tv[j] = t;
-        Out[j] = (y1 - 2.0 * w0 * t) / (c * d[0]);
+        y1v[j] = ((b0 - 2.0 * w0 * r) - (s1 - 2.0 * sig[1] * r)) / sig[0];
     }
 }
 
+// The last step of the deflated solve: the second reflection, of [y1; Z - wt y1],
+// with its scalar t = w . [y1; Z - wt y1] taken from the stored Z itself,
+//     t = w0 y1 + w1 . Z - (w1 . wt) y1:
+// the reflection then leaves the constant mode at y1 whatever Z's rounding is.
+// (From the right-hand side, w1 . Z = (Mt^-1 w1) . X'1, the error of Z in that
+// direction stays in the solution as net charge: 150 to 20000 eps |x| for
+// smooth data on 245 to 1885 points, against 1 to 75 eps |x|.)
+// Out[j + ldo p] = ([y1; Z - wt y1] - 2 w t) / (c d[p]), Z in Out's rows 1..m;
+// nd sums of w1 . Z at dots + ncols k.  A thread takes DR rows of a column j.
+constexpr int DR = 32;
+
+__global__ void __launch_bounds__(256) k_defl_rows(const double* __restrict__ w, const double* __restrict__ wt,
+                                                   const double* __restrict__ sig, const double* __restrict__ y1v,
+                                                   const double* __restrict__ dots, int nd, int n, int ncols,
+                                                   const double* __restrict__ d, double c, double* __restrict__ Out,
+                                                   int ldo)
+{
+    const int j = blockIdx.x * 256 + threadIdx.x, p0 = blockIdx.y * DR;
+    if (j >= ncols) return;
+    double q = 0.0;
+#pragma unroll 8
+    for (int k = 0; k < nd; ++k) q += dots[j + (size_t)ncols * k];
+    const double y1 = y1v[j], w0 = w[0];
+    const double t = w0 * y1 + q - sig[1] * y1;
+    if (p0 == 0) Out[j] = (y1 - 2.0 * w0 * t) / (c * d[0]);
+    const int p1 = min(p0 + DR, n);
+#pragma unroll 8
+    for (int p = max(p0, 1); p < p1; ++p) {
+        double* o = Out + j + (size_t)ldo * p;
+        *o = (*o - y1 * wt[p - 1] - 2.0 * t * w[p]) / (c * d[p]);
+    }
+}
+
+// the same for a single column, in one work-group
+__global__ void __launch_bounds__(1024) k_defl_vec(const double* __restrict__ w, const double* __restrict__ wt,
+                                                   const double* __restrict__ sig, const double* __restrict__ y1v, int n,
+                                                   const double* __restrict__ d, double c, double* __restrict__ Out)
+{
+    __shared__ double red[16];
+    double q = 0.0;
+    for (int p = 1 + threadIdx.x; p < n; p += 1024) q = __builtin_fma(w[p], Out[p], q);
+    for (int off = 32; off > 0; off >>= 1) q += __shfl_xor(q, off, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = q;
+    __syncthreads();
+    q = 0.0;
+    for (int k = 0; k < 16; ++k) q += red[k];
+    const double y1 = y1v[0], w0 = w[0];
+    const double t = w0 * y1 + q - sig[1] * y1;
+    if (threadIdx.x == 0) Out[0] = (y1 - 2.0 * w0 * t) / (c * d[0]);
+    for (int p = 1 + threadIdx.x; p < n; p += 1024) Out[p] = (Out[p] - y1 * wt[p - 1] - 2.0 * t * w[p]) / (c * d[p]);
+}
+
 // Out[j + ldo p] = (M^-1 B)[p, j] / (c d[p]) for B (n x ncols, leading
-// dimension n): the rows of diag(1 / (c d)) M^-1 B, each contiguous.  The two
-// reflections and the first coordinate's elimination are rank-one and rank-two
-// corrections of the products with W, applied as these are written, so the
-// columns are read once for their scalars and once by W B.  A single column
-// goes through the vector products instead of 64-wide tiles.  Out may be B
-// when ncols = ldo = 1.
+// dimension n): the rows of diag(1 / (c d)) M^-1 B, each contiguous.  The first
+// reflection is a rank-one correction of the product W B, applied as that is
+// written; the second one needs the whole of W^T W B (its dots come with the
+// product, 32 columns of a tile at a time) and is a pass over the result.  A
+// single column (ldo = 1) goes through the vector products instead of 64-wide
+// tiles, and Out may be B then.
 void sym_solve_rows(ilh_plan* pl, SymFactor& F, const double* B, int ncols, const double* d, double c, double* Out,
                     int ldo)
 {
@@ -828,33 +859,38 @@ void sym_solve_rows(ilh_plan* pl, SymFactor& F, const double* B, int ncols, cons
     if (ncols <= 0) return;
     hipStream_t st = pl->ctx->stream;
     const int n = F.n, m = n - 1;
-    F.r.ensure(sizeof(double) * (size_t)3 * ncols);
-    double *r = F.r.as<double>(), *y1 = r + ncols, *t = y1 + ncols;
+    const bool vec = ncols == 1 && ldo == 1;
+    const int nt = (m + GT - 1) / GT, nd = vec ? 0 : 2 * nt;
+    F.r.ensure(sizeof(double) * (size_t)(2 + nd) * ncols);
+    double *r = F.r.as<double>(), *y1 = r + ncols, *dots = y1 + ncols;
     const double* w = F.w.as<double>();
-    k_defl_cols<<<(ncols + 3) / 4, 256, 0, st>>>(w, F.wt(), F.ut(), F.info.as<double>(), B, n, ncols, r, y1, t, Out, d, c);
+    const double* sig = F.info.as<double>();
+    k_defl_cols<<<(ncols + 3) / 4, 256, 0, st>>>(w, F.wt(), sig, B, n, ncols, r, y1);
     ILH_HIP(hipGetLastError());
-    if (m <= 0) return;
     const double* W = F.W.as<double>();
-    F.T.ensure(sizeof(double) * (size_t)m * std::max(ncols, 1));
-    double* T = F.T.as<double>();
-    if (ncols == 1) {
-        k_wmv<1><<<(m + 15) / 16, 1024, 0, st>>>(W, m, B + 1, n, F.ww(), r, T, m);
-        k_wtmv<1><<<(m + 3) / 4, 256, 0, st>>>(W, m, T, m, Out, ldo, y1, t, F.wt(), w + 1, d, c);
-    } else {
-        GemmEpi e1, e2;
-        e1.u = F.ww();
-        e1.v = r;
-        k_dgemm<0, 0, true, EPI_RANK1><<<dim3((m + GT - 1) / GT, (ncols + GT - 1) / GT), 256, 0, st>>>(
-            m, ncols, m, 1.0, W, m, B + 1, n, T, m, TRI_A_LOWER, GemmBatch(), e1);
-        e2.a = y1;
-        e2.b = t;
-        e2.wt = F.wt();
-        e2.w1 = w + 1;
-        e2.d = d + 1;
-        e2.c = c;
-        k_dgemm<1, 0, true, EPI_DEFLATE><<<dim3((ncols + GT - 1) / GT, (m + GT - 1) / GT), 256, 0, st>>>(
-            ncols, m, m, 1.0, T, m, W, m, Out + ldo, ldo, TRI_B_LOWER, GemmBatch(), e2);
+    if (m > 0) {
+        F.T.ensure(sizeof(double) * (size_t)m * ncols);
+        double* T = F.T.as<double>();
+        if (vec) {
+            k_wmv<1><<<(m + 15) / 16, 1024, 0, st>>>(W, m, B + 1, n, F.ww(), r, T, m);
+            k_wtmv<<<(m + 3) / 4, 256, 0, st>>>(W, m, T, Out + 1);
+        } else {
+            GemmEpi e1, e2;
+            e1.u = F.ww();
+            e1.v = r;
+            k_dgemm<0, 0, true, EPI_RANK1><<<dim3(nt, (ncols + GT - 1) / GT), 256, 0, st>>>(
+                m, ncols, m, 1.0, W, m, B + 1, n, T, m, TRI_A_LOWER, GemmBatch(), e1);
+            e2.v = w + 1;
+            e2.dots = dots;
+            k_dgemm<1, 0, true, EPI_DOT><<<dim3((ncols + GT - 1) / GT, nt), 256, 0, st>>>(
+                ncols, m, m, 1.0, T, m, W, m, Out + ldo, ldo, TRI_B_LOWER, GemmBatch(), e2);
+        }
+        ILH_HIP(hipGetLastError());
     }
+    if (vec) k_defl_vec<<<1, 1024, 0, st>>>(w, F.wt(), sig, y1, n, d, c, Out);
+    else
+        k_defl_rows<<<dim3((ncols + 255) / 256, (n + DR - 1) / DR), 256, 0, st>>>(w, F.wt(), sig, y1, dots, nd, n, ncols,
+                                                                                d, c, Out, ldo);
     ILH_HIP(hipGetLastError());
 }
 

@@ -437,11 +437,10 @@ struct SymFactor {
     bool ok = false;
     DevBuf A, W, T, w, vec, r, info;
     // vec: n-vectors y, p (scratch), then of m = n - 1 entries each w1, beta,
-    // W w1, W beta, Mt^-1 w1, Mt^-1 beta
+    // W w1, W beta, Mt^-1 beta
     double* xt() const { return vec.as<double>() + 2 * n; }
     double* ww() const { return xt() + 2 * (n - 1); }
-    double* ut() const { return xt() + 4 * (n - 1); }
-    double* wt() const { return xt() + 5 * (n - 1); }
+    double* wt() const { return xt() + 4 * (n - 1); }
 };
 // A is free for other use after it; scratch: n x n entries (the factor's
 // blocks below the diagonal ones while W = L^-1 is formed).  deflate = false:

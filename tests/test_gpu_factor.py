@@ -64,3 +64,28 @@ def test_double_layer_assembly(ctx, N, spacing, ddf):
     fr, sr = O.dirichlet_solve(og, O.Geometry(s.X, s.Y, s.nx, s.ny, s.ds), fp, ddf_kind=kind)
     assert rel_err(f.flat(), fr) < 1e-10
     assert rel_err(sv.flat(), sr) < 1e-10
+
+
+@pytest.mark.parametrize("N", [245, 450, 900])
+def test_factor_net_charge(ctx, N):
+    """The constant mode of S^-1 b for smooth b: sum_p ds_p x_p = q . b with
+    S^T q = ds (q refined in extended precision).  The solve's last reflection
+    passes its length-N dot's rounding into it, at most N eps |ds x|; the
+    factor's own error (thousands of eps, its constant mode being the one that
+    f's far field sees) must not show."""
+    import ilhip
+    g, s, th = ring(N, 1.4, 0.02)
+    print("net charge N", N, flush=True)
+    c = ilhip.SurfaceScalarCache(s, g, ctx=ctx)
+    S = ilhip.create_RTLinvR(c)
+    Sl = S.T.astype(np.longdouble)
+    inv = np.linalg.inv(S.T)
+    q = (inv @ s.ds).astype(np.longdouble)
+    for _ in range(4):
+        q = q + inv @ (s.ds - Sl @ q).astype(float)
+    F = ilhip.SchurFactor(c)
+    for b in (0.3 + np.cos(th), np.sin(2 * th) + 0.1 * np.cos(7 * th), np.exp(np.cos(th)), 1 / (1.3 + np.cos(th))):
+        x = s.ds * F.solve(b)
+        err = abs(float(x.astype(np.longdouble).sum() - q @ b.astype(np.longdouble)))
+        print("  error / (eps |x|): %.1f" % (err / (np.finfo(float).eps * np.linalg.norm(x))), flush=True)
+        assert err <= N * np.finfo(float).eps * np.linalg.norm(x)
