@@ -228,7 +228,7 @@ struct FusedBatch {
 
 bool fused_supported(int Px, int Py)
 {
-    auto ok = [](int P) { return P >= 128 && P <= 2048 && (P & (P - 1)) == 0; };
+    auto ok = [](int P) { return P >= FUSED_MIN_P && P <= FUSED_MAX_P && (P & (P - 1)) == 0; };
     return ok(Px) && ok(Py);
 }
 

@@ -463,12 +463,14 @@ static int period(int need)
 // P >= 2 max(s1, n - 1 - s0), down to n for sources in the middle (a period
 // must also hold the n outputs).  Bodies rarely reach both ends of an axis, so
 // the solves' convolutions run on the periods their points need: half the
-// period for a body in the middle third.
+// period for a body in the middle third.  Never below the periods the fused
+// batch takes when the grid's own period is one of them: one problem outside
+// them would send its whole batch to single launches.
 static int source_period(int n, double lo, double hi, double shift)
 {
     // the terms' windows span floor(x) - 2 ... floor(x) + 3 about a point at x
     const int s0 = std::max(0, (int)std::floor(lo + shift) - 2), s1 = std::min(n - 1, (int)std::floor(hi + shift) + 3);
-    return period(std::max(n, 2 * std::max(s1, n - 1 - s0)));
+    return std::max(period(std::max(n, 2 * std::max(s1, n - 1 - s0))), std::min(FUSED_MIN_P, period(2 * n - 2)));
 }
 
 static void source_periods(const ilh_plan* pl, int gk, int& Px, int& Py)

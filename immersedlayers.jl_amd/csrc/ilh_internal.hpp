@@ -384,6 +384,7 @@ struct FusedCfg {
     int amp_cap;
 };
 struct FusedBatch;
+constexpr int FUSED_MIN_P = 128, FUSED_MAX_P = 2048;   // FFT periods of the fused passes
 bool fused_supported(int Px, int Py);
 FusedBatch* fused_create(ilh_ctx* ctx, const std::vector<BatchProb>& probs);
 void fused_destroy(FusedBatch* fb);

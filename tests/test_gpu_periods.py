@@ -39,3 +39,32 @@ def test_source_periods(ctx, n, m, cx, cy, r):
     f, df, st, ds = ilhip.NeumannPoisson(c).solve(fp, fm)
     for a, b in zip((f, df, st, ds), O.neumann_solve(og, geo, fp, fm)):
         assert rel_err(a.flat(), b) < 1e-10
+
+
+def test_batch_of_small_and_centred(ctx):
+    """A body in the middle of 48 cells needs a period of 64, below the fused
+    batch's 128, and one in the middle of 140 x 300 needs half the grid's: the
+    batch is fused all the same and equals the single solves bit for bit."""
+    import ilhip
+    from ilhip import geometry as G
+    dx = 0.02
+    caches, fbs = [], []
+    for n, m, r in ((48, 48, 6), (140, 300, 12), (60, 52, 7)):
+        g = G.GridSpec(n + 1, m + 1, n // 2 + 1, m // 2 + 1, dx)
+        s = G.circle(r * dx, 1.4 * dx, 0.3 * dx, -0.2 * dx)
+        caches.append(ilhip.SurfaceScalarCache(s, g, ctx=ctx))
+        fbs.append(np.cos(s.theta(0, 0)) + 0.2)
+    print("fused batch of small grids", flush=True)
+    out = ilhip.dirichlet_solve_batched(caches, fbs)
+    fp = [ilhip.DeviceArray.from_host(ctx, b) for b in fbs]
+    fd = [ilhip.DeviceArray(ctx, int(np.prod(c.g.primal_shape()))) for c in caches]
+    sd = [ilhip.DeviceArray(ctx, len(b)) for b in fbs]
+    batch = ilhip.DirichletBatch(caches, fp, fd, sd)
+    print("tuning", batch.tuning(), flush=True)   # an error for a batch of single launches
+    batch.launch()
+    ctx.synchronize()
+    for k, c in enumerate(caches):
+        f, s = ilhip.DirichletPoisson(c).solve(fbs[k], filter_power=0)
+        for a, b in ((out[k][0].flat(), f.flat()), (out[k][1].flat(), s.flat()), (fd[k].download(), f.flat()),
+                     (sd[k].download(), s.flat())):
+            assert np.array_equal(a, b)
