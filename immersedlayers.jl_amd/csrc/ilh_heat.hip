@@ -62,9 +62,9 @@ struct ilh_heat {
     ilh::StageInverse S13, S23, S0;       // inverse stage Schur matrices
     ilh::DevBuf F, A, Bt, Y, W1, W2;  // grid fields
     ilh::DevBuf e, sg, r2, r2s;           // surface vectors; r2s = r2 - dt a21 E H13 F
-    // filters of at most 16 taps a side: the 64 x 64 tiles near the bodies.
-    // near[t]: F or a W_i may be nonzero within 16 cells of tile t; the lists
-    // hold those tiles and the ones E reads (touch)
+    // the 64 x 64 tiles near the bodies.  near[t]: F or a W_i may be nonzero
+    // within 16 cells of tile t; the lists hold those tiles and the ones E reads
+    // (touch)
     ilh::DevBuf near, near_list, touch_list;
     int n_near = 0, n_touch = 0;
     bool have_bc = false;
@@ -226,8 +226,8 @@ __global__ void k_heat_y_long(const double* __restrict__ in, int nx, int ny, con
 }
 
 // One tile's pass of the whole 2-D filter: out = H(cin in + cb b) + g + cadd add
-// (b, g, add may be null; b and add are read in the tiles that near marks),
-// zero outside the grid.
+// (b, g, add may be null; b and add are read in the tiles that near marks, in
+// all of them without near), zero outside the grid.  out must not be in or b.
 struct TilePass {
     const double* in = nullptr;
     double cin = 1.0;
@@ -272,7 +272,7 @@ __global__ void __launch_bounds__(HTH, 4) k_heat_xy(TilePass P)
         if (tile >= ntiles) return;
     }
     const int x0 = tile % tiles_x * HT, y0 = tile / tiles_x * HT;
-    const bool near = P.near && P.near[tile];
+    const bool near = !P.near || P.near[tile];
     const bool use_b = P.b && near, use_add = P.add && near;
     // the whole stage's loads go out together: one memory round trip
     {
@@ -523,13 +523,29 @@ static void tile_pass(ilh_plan* pl, TilePass P, const int* list = nullptr, int n
     ILH_HIP(hipGetLastError());
 }
 
-// out = exp(tau kappa L) (a + ca b) + cp add in two passes   (b, add may be
-// null; tmp: one grid field of scratch; out may alias a, b or add)
+// out = exp(tau kappa L) (a + ca b) + cp add   (b, add may be null; tmp: one
+// grid field of scratch; out may be add, not a or b): in one pass for filters
+// of at most 16 taps a side, as the shorter one of a step is up to Fo = 1.6, an
+// x and a y pass for longer ones.  A step at 2048^2, N = 3000, Fo = 1.25:
+// 324 us (its three short passes in two each: 376).
 static void heat_apply(ilh_plan* pl, const double* K, int M, const double* a, double ca, const double* b,
                        double* tmp, double* out, double cp = 0.0, const double* add = nullptr)
 {
     const int nx = pl->g.nx(GK_PRIMAL), ny = pl->g.ny(GK_PRIMAL);
     hipStream_t st = pl->ctx->stream;
+    if (M <= YMB) {
+        TilePass P;
+        P.in = a;
+        P.b = b;
+        P.cb = ca;
+        P.add = add;
+        P.cadd = cp;
+        P.K = K;
+        P.M = M;
+        P.out = out;
+        tile_pass(pl, P);
+        return;
+    }
     if (M <= MX_LDS)
         k_heat_x<<<dim3((nx + XT - 1) / XT, (ny + XR - 1) / XR), XT, 0, st>>>(a, ca, b, nx, ny, K, M, tmp);
     else
@@ -654,32 +670,30 @@ extern "C" int ilh_heat_create(ilh_plan* pl, double kappa, double dt, ilh_heat**
                 schur_inverse(pl, K13, false, lng, F, inv, h->S13);
                 schur_inverse(pl, K23, false, lng, F, inv, h->S23);
                 schur_inverse(pl, {1.0}, true, lng, F, inv, h->S0);
-                if (h->M23 <= YMB) {
-                    const int nx = pl->g.nx(GK_PRIMAL), ny = pl->g.ny(GK_PRIMAL);
-                    const size_t nt = (size_t)((nx + HT - 1) / HT) * ((ny + HT - 1) / HT), pad = (nt + 7) / 8 * 8;
-                    h->near.ensure(2 * pad);
-                    unsigned char* near = h->near.as<unsigned char>();
-                    fill_zero(st, (double*)near, 2 * pad / 8);
-                    k_heat_mark<<<(N + 255) / 256, 256, 0, st>>>(get_terms(pl, OP_E_PRIMAL), N, nx, ny, near,
-                                                                near + pad);
-                    ILH_HIP(hipGetLastError());
-                    std::vector<unsigned char> f(2 * pad);
-                    ILH_HIP(hipMemcpyAsync(f.data(), near, 2 * pad, hipMemcpyDeviceToHost, st));
-                    ILH_HIP(hipStreamSynchronize(st));
-                    // F and the W_i are nonzero on near tiles only, and set there with the boundary values
-                    for (DevBuf* w : {&h->W1, &h->W2}) fill_zero(st, w->as<double>(), ng);
-                    auto list = [&](const unsigned char* on, DevBuf& buf) {
-                        std::vector<int> l;
-                        for (size_t k = 0; k < nt; ++k)
-                            if (on[k]) l.push_back((int)k);
-                        buf.ensure(sizeof(int) * std::max<size_t>(1, l.size()));
-                        ILH_HIP(hipMemcpyAsync(buf.p, l.data(), sizeof(int) * l.size(), hipMemcpyHostToDevice, st));
-                        ILH_HIP(hipStreamSynchronize(st));   // l is released on return
-                        return (int)l.size();
-                    };
-                    h->n_near = list(f.data(), h->near_list);
-                    h->n_touch = list(f.data() + pad, h->touch_list);
-                }
+                const int nx = pl->g.nx(GK_PRIMAL), ny = pl->g.ny(GK_PRIMAL);
+                const size_t nt = (size_t)((nx + HT - 1) / HT) * ((ny + HT - 1) / HT), pad = (nt + 7) / 8 * 8;
+                h->near.ensure(2 * pad);
+                unsigned char* near = h->near.as<unsigned char>();
+                fill_zero(st, (double*)near, 2 * pad / 8);
+                k_heat_mark<<<(N + 255) / 256, 256, 0, st>>>(get_terms(pl, OP_E_PRIMAL), N, nx, ny, near,
+                                                            near + pad);
+                ILH_HIP(hipGetLastError());
+                std::vector<unsigned char> f(2 * pad);
+                ILH_HIP(hipMemcpyAsync(f.data(), near, 2 * pad, hipMemcpyDeviceToHost, st));
+                ILH_HIP(hipStreamSynchronize(st));
+                // F and the W_i are nonzero on near tiles only, and set there with the boundary values
+                for (DevBuf* w : {&h->W1, &h->W2}) fill_zero(st, w->as<double>(), ng);
+                auto list = [&](const unsigned char* on, DevBuf& buf) {
+                    std::vector<int> l;
+                    for (size_t k = 0; k < nt; ++k)
+                        if (on[k]) l.push_back((int)k);
+                    buf.ensure(sizeof(int) * std::max<size_t>(1, l.size()));
+                    ILH_HIP(hipMemcpyAsync(buf.p, l.data(), sizeof(int) * l.size(), hipMemcpyHostToDevice, st));
+                    ILH_HIP(hipStreamSynchronize(st));   // l is released on return
+                    return (int)l.size();
+                };
+                h->n_near = list(f.data(), h->near_list);
+                h->n_touch = list(f.data() + pad, h->touch_list);
             }
             ILH_HIP(hipStreamSynchronize(st));
         } catch (...) {
@@ -709,14 +723,12 @@ extern "C" int ilh_heat_set_boundary(ilh_heat* h, const double* tb_plus, const d
             double* F = h->F.as<double>();
             scatter_op(pl, OP_DS, h->e.as<double>(), F);   // includes the 1/dx of GridScaling
             // a stage's W = F + R sigma differs from F only on R's cells, which every stage rewrites
-            const size_t ng = pl->g.n(GK_PRIMAL);
-            if (h->M23 > YMB) {
-                for (DevBuf* w : {&h->W1, &h->W2})
-                    ILH_HIP(hipMemcpyAsync(w->p, F, sizeof(double) * ng, hipMemcpyDeviceToDevice, st));
-            } else if (h->n_near > 0) {
+            if (h->n_near > 0) {
                 k_heat_copy_tiles<<<h->n_near, 256, 0, st>>>(F, h->near_list.as<int>(), pl->g.nx(GK_PRIMAL),
                                                             pl->g.ny(GK_PRIMAL), h->W1.as<double>(), h->W2.as<double>());
                 ILH_HIP(hipGetLastError());
+            }
+            if (h->M23 <= YMB && h->n_near > 0) {
                 // r2s = r2 - dt a21 E H13 F
                 TilePass P;
                 P.in = F;
