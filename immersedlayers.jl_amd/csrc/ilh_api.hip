@@ -9,6 +9,7 @@
 #include <memory>
 #include <mutex>
 #include <new>
+#include <numeric>
 
 using namespace ilh;
 
@@ -358,6 +359,7 @@ static void load_points(ilh_plan* pl, const double* X, const double* Y, const do
         mm = std::min({mm, ext[0], (pl->g.NX - 2) - ext[1], ext[2], (pl->g.NY - 2) - ext[3]});
     }
     std::copy(ext, ext + 4, pl->ext);
+    pl->sum_ds = std::accumulate(ds, ds + N, 0.0);
     pl->min_margin = N > 0 ? (int)std::floor(mm) : 1 << 20;
     const size_t stride = ((size_t)std::max(1, N) + 31) / 32 * 32;   // 256-byte aligned arrays
     pl->geo.ensure(sizeof(double) * 5 * stride);
@@ -1597,13 +1599,19 @@ const double* filter_r1(ilh_plan* pl, DevBuf& ones)
 
 // ---- C as sparse rows.  A point's row reaches the points whose windows overlap
 // its own: about ten along a curve at the usual spacing.  Built once per
-// geometry, C^k is k sparse products in ONE launch (up to FILT_ONE points: the
-// vector lives in one work-group's LDS, and a power is one gather from it),
-// where scattering onto the grid, weighting it and gathering back was three
-// launches a power over a whole grid field (power 6 at 206 x 206, 112 points:
-// 18 launches, 87 us of the host's wait, against 6.8 us).
+// geometry, C^k is k sparse products in one launch (up to FILT_ONE points: the
+// vector lives in one work-group's LDS, and a power is one gather from it) or
+// in one each, where scattering onto the grid, weighting it and gathering back
+// is three launches a power over a whole grid field (power 6 at 206 x 206, 112
+// points: 18 launches, 87 us of the host's wait, against 6.8 us).  The rows
+// form R 1 on their own windows' cells, so that a new geometry needs neither
+// the row bins nor R 1 on the grid for them.
 constexpr int FILT_CAP = 64;     // entries a row holds: denser samplings take the grid
-constexpr int FILT_ONE = 4096;   // points of one work-group: two vectors in 64 KB of LDS
+// Points up to which one work-group takes every power: power 6 in one launch
+// and in six, 1885 points 27 and 31 us, 3000 points 33 and 31, 4096 40 and 31
+// (power 2: 17.4 and 17.9, 19.7 and 17.5, 21.8 and 17.6).
+constexpr int FILT_ONE = 2048;
+constexpr int FILT_NEAR = 128;   // points whose five-tap windows overlap a row's
 
 __global__ void k_filter_bases(const Term* __restrict__ t, int N, int2* __restrict__ b)
 {
@@ -1611,53 +1619,83 @@ __global__ void k_filter_bases(const Term* __restrict__ t, int N, int2* __restri
     if (p < N) b[p] = make_int2(t[p].bx, t[p].by);
 }
 
-// One wave per point p: 64 candidates q at a time, the entry
-// sum over the common cells of E_p R_q / (R 1), kept when not 0, q ascending.
-// info[0] collects the longest row.
+// One wave per point p.  The points whose windows overlap its window are
+// listed, q ascending; R 1 on the window's 25 cells is summed over the list
+// (a lane a cell), and the entry of q is
+// sum over the common cells of E_p R_q / (R 1), kept when not 0.
+// info[0] collects the longest row (FILT_CAP + 1 for a list that is too long).
 __global__ void __launch_bounds__(256) k_filter_rows(const Term* __restrict__ TE, const Term* __restrict__ TR,
                                                      const int2* __restrict__ bases, int N, int nx, int ny,
-                                                     const double* __restrict__ r1, double* __restrict__ w,
-                                                     int* __restrict__ qi, int* __restrict__ len, int* __restrict__ info)
+                                                     double* __restrict__ w, int* __restrict__ qi,
+                                                     int* __restrict__ len, int* __restrict__ info)
 {
-    const int p = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (p >= N) return;   // uniform over the wave
+    __shared__ int list[4][FILT_NEAR];
+    __shared__ double cell[4][25];   // E_p / (R 1) on the window's cells
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int p = min((int)blockIdx.x * 4 + wave, N - 1);   // waves past the end repeat the last point's row
     const Term& t = TE[p];
     const int tx = t.bx, ty = t.by;
     int cnt = 0;
-    for (int q0 = 0; q0 < N; q0 += 64) {
-        const int q = q0 + lane;
+    for (int q0 = 0; q0 < N; q0 += 256) {
+        int2 b[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) b[u] = bases[min(q0 + 64 * u + lane, N - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int q = q0 + 64 * u + lane;
+            const bool on = q < N && abs(tx - b[u].x) <= 4 && abs(ty - b[u].y) <= 4;
+            const unsigned long long m = __ballot(on);
+            const int at = cnt + __popcll(m & ((1ull << lane) - 1));
+            if (on && at < FILT_NEAR) list[wave][at] = q;
+            cnt += __popcll(m);
+        }
+    }
+    const bool fits = cnt <= FILT_NEAR;
+    if (!fits) cnt = 0;
+    __syncthreads();
+    if (lane < 25) {
+        const int b = lane / 5, a = lane - 5 * b, row = ty + b, col = tx + a;
+        double one = 0.0, e = 0.0;
+        if (row >= 0 && row < ny && col >= 0 && col < nx) {
+#pragma unroll 4
+            for (int k = 0; k < cnt; ++k) {
+                const Term& r = TR[list[wave][k]];
+                const int ra = col - r.bx, rb = row - r.by;
+                if (ra >= 0 && ra < 5 && rb >= 0 && rb < 5) one += r.coef * (r.wy[rb] * r.wx[ra]);
+            }
+            if (one != 0.0) e = t.coef * (t.wx[a] * t.wy[b]) / one;
+        }
+        cell[wave][lane] = e;
+    }
+    __syncthreads();
+    int n = 0;
+    for (int k0 = 0; k0 < cnt; k0 += 64) {
+        const int q = k0 + lane < cnt ? list[wave][k0 + lane] : -1;
         double v = 0.0;
-        if (q < N) {
-            const int2 bq = bases[q];
-            const int sx = tx - bq.x, sy = ty - bq.y;   // tap a of p is tap a + sx of q
-            if (abs(sx) <= 4 && abs(sy) <= 4) {
-                const Term& r = TR[q];
-                for (int b = 0; b < 5; ++b) {
-                    const int row = ty + b, rb = b + sy;
-                    if (rb < 0 || rb > 4 || row < 0 || row >= ny) continue;
-                    const double wy = t.wy[b] * r.wy[rb];
-                    if (wy == 0.0) continue;
-                    for (int a = 0; a < 5; ++a) {
-                        const int col = tx + a, ra = a + sx;
-                        if (ra < 0 || ra > 4 || col < 0 || col >= nx) continue;
-                        const double wx = t.wx[a] * r.wx[ra];
-                        const double one = r1[col + (size_t)nx * row];
-                        if (wx != 0.0 && one != 0.0) v += t.coef * r.coef * (wx * wy / one);
-                    }
+        if (q >= 0) {
+            const Term& r = TR[q];
+            const int sx = tx - r.bx, sy = ty - r.by;   // tap a of p is tap a + sx of q
+            for (int b = 0; b < 5; ++b) {
+                const int rb = b + sy;
+                if (rb < 0 || rb > 4) continue;
+                const double wy = r.coef * r.wy[rb];
+                for (int a = 0; a < 5; ++a) {
+                    const int ra = a + sx;
+                    if (ra >= 0 && ra < 5) v += cell[wave][5 * b + a] * (wy * r.wx[ra]);
                 }
             }
         }
         const unsigned long long on = __ballot(v != 0.0);
-        const int at = cnt + __popcll(on & ((1ull << lane) - 1));
+        const int at = n + __popcll(on & ((1ull << lane) - 1));
         if (v != 0.0 && at < FILT_CAP) {
             w[(size_t)N * at + p] = v;
             qi[(size_t)N * at + p] = q;
         }
-        cnt += __popcll(on);
+        n += __popcll(on);
     }
     if (lane == 0) {
-        len[p] = min(cnt, FILT_CAP);
-        atomicMax(info, cnt);
+        len[p] = min(n, FILT_CAP);
+        atomicMax(info, fits ? n : FILT_CAP + 1);
     }
 }
 
@@ -1708,11 +1746,15 @@ __global__ void __launch_bounds__(256) k_filter_step(const double* __restrict__ 
     if (p < N) y[p] = filter_row(w, qi, N, p, len[p], x);
 }
 
-// the rows of the current geometry; false: a row is too long for them
-bool filter_rows(ilh_plan* pl, const double* r1)
+// the rows of the current geometry; false: a row is too long for them.  Where
+// the points' mean spacing along their curves says so (the points within reach
+// span 8 sqrt(2) dx where a curve runs diagonally) they are not tried, which
+// would cost 40 us and a wait for nothing (300 points, new geometry).
+bool filter_rows(ilh_plan* pl)
 {
     if (pl->filt_gen_rows == pl->gen) return pl->filt_len >= 0;
     const int N = pl->N;
+    if (!(FILT_CAP * pl->sum_ds >= 11.4 * pl->g.dx * N)) return false;
     hipStream_t st = pl->ctx->stream;
     pl->filt_w.ensure(sizeof(double) * (size_t)N * FILT_CAP);
     pl->filt_q.ensure(sizeof(int) * ((size_t)N * (FILT_CAP + 3) + 1));   // window bases, columns, lengths, the longest
@@ -1722,7 +1764,7 @@ bool filter_rows(ilh_plan* pl, const double* r1)
     fill_zero(st, (float*)info, 1);
     k_filter_bases<<<(N + 255) / 256, 256, 0, st>>>(tr, N, (int2*)bases);
     k_filter_rows<<<(N + 3) / 4, 256, 0, st>>>(te, tr, (const int2*)bases, N, pl->g.nx(GK_PRIMAL), pl->g.ny(GK_PRIMAL),
-                                               r1, pl->filt_w.as<double>(), q, len, info);
+                                               pl->filt_w.as<double>(), q, len, info);
     ILH_HIP(hipGetLastError());
     int longest = 0;
     ILH_HIP(hipMemcpyAsync(&longest, info, sizeof(int), hipMemcpyDeviceToHost, st));
@@ -1772,13 +1814,12 @@ extern "C" int ilh_surface_filter_apply(ilh_plan* pl, int power, const double* s
         hipStream_t st = pl->ctx->stream;
         const double* d_in = io.in(s_in, N, pl->io_a);
         double* d_out = io.out(s_out, N, pl->io_d);
+        DevBuf ones;   // in use until the wait below
         if (N > 0) {
-            DevBuf ones;
-            const double* r1 = filter_r1(pl, ones);
             if (power == 0) {
                 if (d_out != d_in)
                     ILH_HIP(hipMemcpyAsync(d_out, d_in, sizeof(double) * N, hipMemcpyDeviceToDevice, st));
-            } else if (filter_rows(pl, r1)) {
+            } else if (filter_rows(pl)) {
                 const double* w = pl->filt_w.as<double>();
                 const int *q = pl->filt_q.as<int>() + 2 * (size_t)N, *len = q + (size_t)N * FILT_CAP;
                 if (N <= FILT_ONE) {
@@ -1799,6 +1840,7 @@ extern "C" int ilh_surface_filter_apply(ilh_plan* pl, int power, const double* s
             } else {
                 if (d_out != d_in)
                     ILH_HIP(hipMemcpyAsync(d_out, d_in, sizeof(double) * N, hipMemcpyDeviceToDevice, st));
+                const double* r1 = filter_r1(pl, ones);
                 pl->scratch_a.ensure(sizeof(double) * ng);
                 double* g = pl->scratch_a.as<double>();
                 const unsigned gb = (unsigned)std::min<size_t>(4096, (ng + 255) / 256);

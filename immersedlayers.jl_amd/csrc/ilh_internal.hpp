@@ -209,6 +209,7 @@ struct ilh_plan {
     bool bins_ok[ilh::OP_COUNT] = {};
     std::list<ilh::ConvPlan> conv[4];         // primal, dual, u edges, v edges: one per pair of periods in use
     double ext[4] = {};                       // the points' extent in primal grid units, 0-based: x, x, y, y
+    double sum_ds = 0.0;                      // length of the bodies' curves
     ilh::DevBuf lgf;                          // LGF table tmx x tmy (covers both kinds)
     int lgf_mx = 0, lgf_my = 0;
     ilh::DevBuf io_a, io_b, io_c, io_d;       // staging for host-memory calls
