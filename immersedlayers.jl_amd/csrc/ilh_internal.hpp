@@ -4,6 +4,7 @@
 #include <atomic>
 #include <cstddef>
 #include <cstdint>
+#include <initializer_list>
 #include <list>
 #include <new>
 #include <string>
@@ -193,6 +194,7 @@ struct ilh_lpc;      // learned preconditioner model (ilh_learned.hip)
 
 struct MovingCache;
 struct StokesCache;
+struct StokesSources;
 struct ilh_plan {
     ilh_ctx* ctx = nullptr;
     ilh::Grid g{};
@@ -220,6 +222,7 @@ struct ilh_plan {
     SolveCache* neu = nullptr;                // Neumann
     SolveCache* fac[6] = {};                  // ilh_schur_factor caches per kind
     StokesCache* sto = nullptr;               // Stokes flow (vector cache) solve matrices
+    StokesSources* sto_src = nullptr;         // and its source terms, their buffers kept for the next geometry
     MovingCache* mov = nullptr;               // moving-body Dirichlet solves (kept across update_points)
     unsigned gen = 0;                         // incremented whenever the geometry caches are dropped
     ilh::DevBuf mask;                         // mask(cache) on Nodes{Primal} (built lazily)
@@ -309,7 +312,7 @@ struct SourceSet {
     int4* pinfo = nullptr;     // device, per nonzero row pair p: {j0, first cell, first cell of row j0+1, end}
     int* slot_of_row = nullptr;  // device: field row -> row of the compacted spectrum, or -1
     int npairs = 0;            // upper bound of the live row pairs ((ny + 1) / 2)
-    int* npairs_dev = nullptr; // device: live row pairs (after slot_of_row's rows)
+    int* npairs_dev = nullptr; // device: live row pairs, cells (after slot_of_row's rows)
     size_t cap_pairs = 0, cap_rows = 0;   // allocated sizes of pinfo and slot_of_row
     // The first INL_K contributions of every cell, copied by slot (built by
     // pin_source_pairs; null otherwise): inl_ai[u inl_stride + c] and
@@ -332,7 +335,7 @@ struct SourceJob {
     SourceSet* src;
 };
 void merge_sources_batched(ilh_ctx* ctx, const std::vector<SourceJob>& jobs, int op0, int op1, int extra_op, int gk);
-void pin_source_pairs(ilh_plan* pl, SourceSet& s);
+void pin_source_pairs(ilh_plan* pl, std::initializer_list<SourceSet*> sets);
 void conv_sources(ilh_plan* pl, int gk, const SourceSet& src, const double* amp, double* out,
                   hipEvent_t* ev = nullptr);
 void conv_stage(ilh_plan* pl, int gk, const SourceSet& src, const double* amp, double* out, int stage);

@@ -815,11 +815,11 @@ void pairs_prepare(SourceSet& s)
         s.cap_pairs = np + 1;
         ILH_HIP(hipMalloc(&s.pinfo, sizeof(int4) * s.cap_pairs));
     }
-    if ((size_t)ny + 1 > s.cap_rows) {
+    if ((size_t)ny + 2 > s.cap_rows) {
         if (s.slot_of_row) (void)hipFree(s.slot_of_row);
         s.slot_of_row = nullptr;
-        s.cap_rows = (size_t)ny + 1;
-        ILH_HIP(hipMalloc(&s.slot_of_row, sizeof(int) * s.cap_rows));   // rows, then the live count
+        s.cap_rows = (size_t)ny + 2;
+        ILH_HIP(hipMalloc(&s.slot_of_row, sizeof(int) * s.cap_rows));   // rows, then the live pairs and the cells
     }
     s.npairs = (int)np;
     s.npairs_dev = s.slot_of_row + ny;
@@ -885,7 +885,8 @@ void free_sources(SourceSet& s)
 // Row pairs (2p, 2p+1) with at least one entry, compacted in order: pinfo[k]
 // = {2p, first cell of row 2p, first cell of row 2p+1, end of the pair's
 // cells}, slot_of_row[2p] = 2k, slot_of_row[2p+1] = 2k+1 (-1 for rows of idle
-// pairs), *npairs = live pairs.  One work-group of 1024 threads.
+// pairs), npairs[0] = live pairs, npairs[1] = cells.  One work-group of 1024
+// threads.
 __device__ __forceinline__ void k_source_pairs_body(const int* __restrict__ row_ptr, const int* __restrict__ cell_ptr,
                                                     int ny, int4* __restrict__ pinfo, int* __restrict__ slot_of_row,
                                                     int* __restrict__ npairs)
@@ -924,7 +925,10 @@ __device__ __forceinline__ void k_source_pairs_body(const int* __restrict__ row_
         if (t == 1023) carry = k + f;
         __syncthreads();
     }
-    if (t == 0) *npairs = carry;
+    if (t == 0) {
+        npairs[0] = carry;
+        npairs[1] = cell_ptr[ny];
+    }
 }
 
 __global__ void __launch_bounds__(1024) k_source_pairs(const int* __restrict__ row_ptr,
@@ -947,8 +951,6 @@ void build_source_pairs(ilh_plan* pl, SourceSet& s)
     ILH_HIP(hipGetLastError());
 }
 
-// The exact live pair count on the host (one read-back; for caches built
-// once and used by many solves): the row pass then launches exactly.
 // the first INL_K contributions of cells [0, ncells), by slot (layout of
 // SourceSet::inl_ai)
 __global__ void k_inline_contribs(const int4* __restrict__ cells, const int* __restrict__ cai,
@@ -966,35 +968,45 @@ __global__ void k_inline_contribs(const int4* __restrict__ cells, const int* __r
     }
 }
 
-void pin_source_pairs(ilh_plan* pl, SourceSet& s)
+// The exact live pair counts on the host (for caches built once and used by
+// many solves): the row pass then launches exactly.  One wait for all the sets.
+void pin_source_pairs(ilh_plan* pl, std::initializer_list<SourceSet*> sets)
 {
-    if (!s.npairs_dev) return;
     hipStream_t st = pl->ctx->stream;
-    int n = 0, ncells = 0;
-    ILH_HIP(hipMemcpyAsync(&n, s.npairs_dev, sizeof(int), hipMemcpyDeviceToHost, st));
-    ILH_HIP(hipMemcpyAsync(&ncells, s.bins.cell_ptr + s.bins.ny, sizeof(int), hipMemcpyDeviceToHost, st));
-    ILH_HIP(hipStreamSynchronize(st));
-    s.npairs = n;
-    s.npairs_dev = nullptr;
-    // the cells' first contributions copied by slot, for the row pass
-    s.inl_stride = 0;
-    if (ncells <= 0) return;
-    const size_t cap = ((size_t)ncells + 255) / 256 * 256;
-    if (cap > s.inl_cap) {
-        if (s.inl_ai) (void)hipFree(s.inl_ai);
-        s.inl_ai = nullptr;
-        s.inl_w = nullptr;
-        s.inl_cap = 0;
-        void* p = nullptr;
-        ILH_HIP(hipMalloc(&p, (sizeof(int) + sizeof(double)) * INL_K * cap));
-        s.inl_ai = (int*)p;
-        s.inl_w = (double*)((char*)p + sizeof(int) * INL_K * cap);
-        s.inl_cap = cap;
+    std::vector<int> h(2 * sets.size(), 0);
+    int* c = h.data();
+    for (SourceSet* s : sets) {
+        if (s->npairs_dev) ILH_HIP(hipMemcpyAsync(c, s->npairs_dev, 2 * sizeof(int), hipMemcpyDeviceToHost, st));
+        c += 2;
     }
-    k_inline_contribs<<<(ncells + 255) / 256, 256, 0, st>>>(s.bins.cells, s.bins.cai, s.bins.cw, ncells,
-                                                            (int)s.inl_cap, s.inl_ai, s.inl_w);
-    ILH_HIP(hipGetLastError());
-    s.inl_stride = (int)s.inl_cap;
+    ILH_HIP(hipStreamSynchronize(st));
+    c = h.data();
+    for (SourceSet* s : sets) {
+        const int n = c[0], ncells = c[1];
+        c += 2;
+        if (!s->npairs_dev) continue;
+        s->npairs = n;
+        s->npairs_dev = nullptr;
+        // the cells' first contributions copied by slot, for the row pass
+        s->inl_stride = 0;
+        if (ncells <= 0) continue;
+        const size_t cap = ((size_t)ncells + 255) / 256 * 256;
+        if (cap > s->inl_cap) {
+            if (s->inl_ai) (void)hipFree(s->inl_ai);
+            s->inl_ai = nullptr;
+            s->inl_w = nullptr;
+            s->inl_cap = 0;
+            void* p = nullptr;
+            ILH_HIP(hipMalloc(&p, (sizeof(int) + sizeof(double)) * INL_K * cap));
+            s->inl_ai = (int*)p;
+            s->inl_w = (double*)((char*)p + sizeof(int) * INL_K * cap);
+            s->inl_cap = cap;
+        }
+        k_inline_contribs<<<(ncells + 255) / 256, 256, 0, st>>>(s->bins.cells, s->bins.cai, s->bins.cw, ncells,
+                                                                (int)s->inl_cap, s->inl_ai, s->inl_w);
+        ILH_HIP(hipGetLastError());
+        s->inl_stride = (int)s->inl_cap;
+    }
 }
 
 
