@@ -181,6 +181,16 @@ struct MovingCache {
     }
 };
 
+// The previous geometry's Dirichlet buffers are freed: a plan that goes on with
+// solves of another kind needs the memory for those.
+void ilh::drop_spare(ilh_plan* pl)
+{
+    if (!pl->dir_spare) return;
+    (void)hipStreamSynchronize(pl->ctx->stream);   // they may still be in use
+    delete pl->dir_spare;
+    pl->dir_spare = nullptr;
+}
+
 // Geometry caches become stale; row-bin buffers are kept for the next
 // geometry unless `release` (plan destruction).
 static void drop_caches(ilh_plan* pl, bool release = false)
@@ -189,11 +199,11 @@ static void drop_caches(ilh_plan* pl, bool release = false)
     if (pl->mov) pl->mov->drop_sources();
     // the Dirichlet solve data's buffers (the factor and the solve matrices,
     // four N x N or more) serve the next geometry: freeing and allocating them
-    // at every one took 1.6 of a new-geometry solve's 6.0 ms (N = 1885)
-    if (pl->dir) {
-        delete pl->dir_spare;
-        pl->dir_spare = pl->dir;
-    }
+    // at every one took 1.6 of a new-geometry solve's 6.0 ms (N = 1885).  They
+    // are given back when that geometry ends without such a solve, and when the
+    // plan turns to other solves on it (drop_spare)
+    delete pl->dir_spare;
+    pl->dir_spare = pl->dir;
     if (release) {
         delete pl->dir_spare;
         pl->dir_spare = nullptr;
@@ -418,7 +428,7 @@ extern "C" int ilh_plan_update_points(ilh_plan* pl, const double* X, const doubl
         ILH_HIP(hipSetDevice(pl->ctx->device));
         // caches that are freed may still be in use; those kept for the next
         // geometry, and the points themselves, are rewritten in stream order
-        bool frees = pl->neu || pl->sto || (pl->dir && pl->dir_spare);
+        bool frees = pl->neu || pl->sto || pl->dir_spare;
         for (const auto* f : pl->fac) frees = frees || f;
         if (frees) ILH_HIP(hipStreamSynchronize(pl->ctx->stream));
         drop_caches(pl);
@@ -1037,8 +1047,11 @@ void factor_into(ilh_plan* pl, SolveCache* sc, int kind)
         sc->M[0].ensure(sizeof(double) * (size_t)N * solve_ld(N));
         if (sym_rtlinvr(pl, sc->sym, sc->M[0].as<double>())) {
             sc->use_sym = true;
+            sc->LU.release();
             return;
         }
+        sc->sym.W.release();   // A stays: the solve matrices are formed in it
+        sc->sym.T.release();
     }
     sc->use_sym = false;
     sc->LU.ensure(sizeof(double) * (size_t)N * N);
@@ -1127,6 +1140,7 @@ SolveCache* prepare_neumann(ilh_plan* pl)
 {
     if (pl->neu) return pl->neu;
     need_margin(pl, "Neumann solve");
+    drop_spare(pl);
     const int N = pl->N;
     SolveCache* sc = new SolveCache();
     try {
@@ -1204,12 +1218,15 @@ extern "C" int ilh_schur_factor(ilh_plan* pl, int kind)
         Io io(pl, ILH_MEM_DEVICE);
         if (kind < 0 || kind > ILH_SCHUR_GLINVD_SYMM) fail(ILH_ERR_ARG, "unknown Schur kind");
         if (kind != ILH_SCHUR_NRTRN) need_margin(pl, "Schur factor");
+        drop_spare(pl);
         delete pl->fac[kind];
         pl->fac[kind] = nullptr;
         SolveCache* sc = new SolveCache();
         try {
             if (pl->N > 0) factor_into(pl, sc, kind);
-            sc->M[0].release();   // the factorisation's scratch: no solve matrix is formed here
+            // the factorisation's scratch: no solve matrix is formed here
+            sc->M[0].release();
+            sc->sym.A.release();
         } catch (...) {
             delete sc;
             throw;
@@ -2065,6 +2082,7 @@ StokesCache* prepare_stokes(ilh_plan* pl)
 {
     if (pl->sto) return pl->sto;
     need_margin(pl, "Stokes solve");
+    drop_spare(pl);
     StokesCache* sc = new StokesCache();
     try {
         const int N = pl->N, n2 = 2 * N;
@@ -3662,6 +3680,7 @@ static MovingCache* moving_setup(ilh_plan* pl, int m)
     const int N = pl->N;
     const size_t ng = pl->g.n(GK_PRIMAL);
     need_margin(pl, "Dirichlet solve");
+    drop_spare(pl);
     if (!pl->mov) pl->mov = new MovingCache();
     MovingCache* mc = pl->mov;
     mc->amp.ensure(sizeof(double) * 2 * (size_t)N);

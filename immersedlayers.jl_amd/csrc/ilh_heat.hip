@@ -641,6 +641,7 @@ extern "C" int ilh_heat_create(ilh_plan* pl, double kappa, double dt, ilh_heat**
         if (!(kappa > 0.0) || !(dt > 0.0) || !std::isfinite(kappa * dt)) fail(ILH_ERR_ARG, "kappa and dt must be positive");
         ILH_HIP(hipSetDevice(pl->ctx->device));
         if (pl->N > 0) need_margin(pl, "heat conduction");
+        drop_spare(pl);
         const double a13 = kappa * dt / 3.0 / (pl->g.dx * pl->g.dx);
         const std::vector<double> K13 = heat_kernel_1d(a13), K23 = heat_kernel_1d(2.0 * a13);
         if ((int)K23.size() > 256) fail(ILH_ERR_ARG, "time step too large for the integrating-factor filter (a > ~40)");

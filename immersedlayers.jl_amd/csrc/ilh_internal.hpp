@@ -251,6 +251,7 @@ namespace ilh {
 void ctx_retain(ilh_ctx* c);
 void ctx_release(ilh_ctx* c);
 void plan_retain(ilh_plan* pl);
+void drop_spare(ilh_plan* pl);   // the previous geometry's Dirichlet buffers, kept for a next Dirichlet solve
 void plan_release(ilh_plan* pl);
 
 // ---------------------------------------------------------------- launchers

@@ -809,6 +809,7 @@ extern "C" int ilh_lpc_add_geometry(ilh_lpc* m, ilh_plan* pl)
         ILH_HIP(hipSetDevice(pl->ctx->device));
         if (m->stats_ok) fail(ILH_ERR_STATE, "training rows must be added before the first training step");
         need_margin(pl, "learned preconditioner training");
+        drop_spare(pl);
         const int N = pl->N;
         if (N < m->W) fail(ILH_ERR_ARG, "too few points for the band");
         hipStream_t st = pl->ctx->stream;

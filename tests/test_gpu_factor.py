@@ -89,3 +89,54 @@ def test_factor_net_charge(ctx, N):
         err = abs(float(x.astype(np.longdouble).sum() - q @ b.astype(np.longdouble)))
         print("  error / (eps |x|): %.1f" % (err / (np.finfo(float).eps * np.linalg.norm(x))), flush=True)
         assert err <= N * np.finfo(float).eps * np.linalg.norm(x)
+
+
+def test_solve_buffers_given_back(ctx):
+    """The Dirichlet buffers of the previous geometry wait for a next Dirichlet
+    solve for one geometry, and go as soon as the plan takes another solve:
+    the factor and the solve matrix are four N x N arrays."""
+    import ctypes as C
+    import gc
+
+    import ilhip
+    N = 1500
+    g, s, th = ring(N, 1.4, 0.02)
+    moved = ring(N, 1.4, 0.02, 0.011)[1]
+    b = 0.3 + np.cos(th)
+    mat = 8 * N * N
+    print("buffers", flush=True)
+
+    def used():
+        gc.collect()
+        ctx.synchronize()
+        free, total = C.c_size_t(), C.c_size_t()
+        assert ilhip.load_library().hipMemGetInfo(C.byref(free), C.byref(total)) == 0   # from the HIP runtime it links
+        return total.value - free.value
+
+    def plan(solve, other):
+        c = ilhip.SurfaceScalarCache(s, g, ctx=ctx)
+        p = ilhip.DirichletPoisson(c)
+        p.solve(b, filter_power=0)
+        u = [used()]
+        c.update_points(moved)
+        if solve:
+            p.solve(b, filter_power=0)
+        u.append(used())
+        c.update_points(s)
+        if other:
+            other(c)
+        u.append(used())
+        return u
+
+    full, again, moving = plan(True, lambda c: ilhip.DirichletPoisson(c).solve_moving(b))
+    assert abs(again - full) < mat   # reused, not allocated beside the old ones
+    full, idle, gone = plan(False, None)
+    assert abs(idle - full) < mat and gone < full - 3 * mat
+
+    def moving_only():
+        c = ilhip.SurfaceScalarCache(s, g, ctx=ctx)
+        before = used()
+        ilhip.DirichletPoisson(c).solve_moving(b)
+        return used() - before
+
+    assert moving - full < moving_only() - 3 * mat
