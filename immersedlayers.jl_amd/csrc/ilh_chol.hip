@@ -64,21 +64,19 @@ struct GemmBatch {
     int m_total = 0, m_step = 0;
     int k_is_m = 0;
 };
-// Epilogues: EPI_RANK1 C = alpha AB - 2 u[m] v[n]; EPI_DOT C = AB, and the sums
-// of C[m, n] v[n] over each 32 columns of a tile at dots + M (2 n-tile + half)
-// (for gridDim.z = 1).
-enum { EPI_NONE = 0, EPI_RANK1 = 1, EPI_DOT = 2 };
-struct GemmEpi {
-    const double *u = nullptr, *v = nullptr;
+// With DOT, also the sums of C[m, n] v[n] over each 32 columns of a tile, at
+// dots + M (2 n-tile + half) (gridDim.z = 1).
+struct GemmDots {
+    const double* v = nullptr;
     double* dots = nullptr;
 };
 
-template <int TA, int TB, bool BETA0, int EPI>
+template <int TA, int TB, bool BETA0, bool DOT>
 // (A or B may be C itself when every work-group reads all the entries it
 // overwrites; hence no __restrict__.)
 __global__ void __launch_bounds__(256) k_dgemm(int M, int Nc, int K, double alpha, const double* A, int lda,
                                                const double* B, int ldb, double* C, int ldc, int tri, GemmBatch bt,
-                                               GemmEpi ep)
+                                               GemmDots ep)
 {
     __shared__ double As[2][GKC][GT + 2];   // As[k][m]
     __shared__ double Bs[2][GKC][GT + 2];   // Bs[k][n]
@@ -199,7 +197,7 @@ __global__ void __launch_bounds__(256) k_dgemm(int M, int Nc, int K, double alph
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int gm = m0 + wm + 16 * i + (lane & 15);
-        if (EPI == EPI_DOT) {
+        if (DOT) {
             double q = 0.0;
 #pragma unroll
             for (int j = 0; j < 2; ++j)
@@ -213,7 +211,6 @@ __global__ void __launch_bounds__(256) k_dgemm(int M, int Nc, int K, double alph
             if (lane < 16 && gm < M) ep.dots[gm + (size_t)M * (2 * by + (wave >> 1))] = q;
         }
         if (gm >= M) continue;
-        const double e0 = EPI == EPI_RANK1 ? ep.u[gm] : 0.0;
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -221,8 +218,7 @@ __global__ void __launch_bounds__(256) k_dgemm(int M, int Nc, int K, double alph
                 const int gn = n0 + wn + 16 * j + (lane >> 4) + 4 * r;
                 if (gn >= Nc) continue;
                 double* p = C + gm + (size_t)ldc * gn;
-                if (EPI == EPI_RANK1) *p = alpha * acc[i][j][r] - 2.0 * e0 * ep.v[gn];
-                else *p = BETA0 ? alpha * acc[i][j][r] : *p + alpha * acc[i][j][r];
+                *p = BETA0 ? alpha * acc[i][j][r] : *p + alpha * acc[i][j][r];
             }
     }
 }
@@ -235,7 +231,7 @@ void dgemm(hipStream_t st, int ta, int tb, int M, int Nc, int K, double alpha, c
     const dim3 grid((M + GT - 1) / GT, (Nc + GT - 1) / GT);
     const bool b0 = beta == 0.0;
 #define ILH_DG(TA_, TB_, B0_) \
-    k_dgemm<TA_, TB_, B0_, EPI_NONE><<<grid, 256, 0, st>>>(M, Nc, K, alpha, A, lda, B, ldb, C, ldc, tri, GemmBatch(), GemmEpi())
+    k_dgemm<TA_, TB_, B0_, false><<<grid, 256, 0, st>>>(M, Nc, K, alpha, A, lda, B, ldb, C, ldc, tri, GemmBatch(), GemmDots())
     if (K <= 0) {
         if (!b0) return;
         alpha = 0.0;   // C = 0
@@ -573,47 +569,36 @@ static void chol_factor(hipStream_t st, double* A, int lda, int m, double* W, do
         bt.m_step = 2 * s;
         const dim3 grid((std::min(s, m - s) + GT - 1) / GT, s / GT, pairs);
         // T21 = L21 W11
-        k_dgemm<0, 0, true, EPI_NONE><<<grid, 256, 0, st>>>(std::min(s, m - s), s, s, 1.0, Lb + off, m, W, m, T + off, m,
-                                                           TRI_B_LOWER, bt, GemmEpi());
+        k_dgemm<0, 0, true, false><<<grid, 256, 0, st>>>(std::min(s, m - s), s, s, 1.0, Lb + off, m, W, m, T + off, m,
+                                                           TRI_B_LOWER, bt, GemmDots());
         // W21 = -W22 T21
         bt.k_is_m = 1;
-        k_dgemm<0, 0, true, EPI_NONE><<<grid, 256, 0, st>>>(std::min(s, m - s), s, s, -1.0, W + off + (size_t)m * s, m,
-                                                           T + off, m, W + off, m, TRI_A_LOWER, bt, GemmEpi());
+        k_dgemm<0, 0, true, false><<<grid, 256, 0, st>>>(std::min(s, m - s), s, s, -1.0, W + off + (size_t)m * s, m,
+                                                           T + off, m, W + off, m, TRI_A_LOWER, bt, GemmDots());
     }
     ILH_HIP(hipGetLastError());
 }
 
-// ---------------------------------------- products of W with a few vectors
-// Y[r + ldy v] = sum_{k <= r} W[r + m k] X[k + ldx v] - 2 u[r] s[v]  (u may be
-// null), v < NV: one work-group of 16 waves per 16 rows; a wave takes four
-// columns of 16 rows at a time, every 64th, and the 64 partial sums are added
-// in a fixed order.  (One wave per 64 rows and column: 79 us at m = 1884, two
-// vectors, too few work-groups and loads in flight.)
-template <int NV>
-__global__ void __launch_bounds__(1024) k_wmv(const double* __restrict__ W, int m, const double* __restrict__ X, int ldx,
-                                              const double* __restrict__ u, const double* __restrict__ s,
-                                              double* __restrict__ Y, int ldy)
+// ---------------------------------------------- products of W with a vector
+// Y[r] = sum_{k <= r} W[r + m k] X[k]: one work-group of 16 waves per 16 rows; a
+// wave takes four columns of 16 rows at a time, every 64th, and the 64 partial
+// sums are added in a fixed order.  (One wave per 64 rows and column: 79 us at
+// m = 1884, two vectors, too few work-groups and loads in flight.)
+__global__ void __launch_bounds__(1024) k_wmv(const double* __restrict__ W, int m, const double* __restrict__ X,
+                                              double* __restrict__ Y)
 {
-    __shared__ double part[NV][64][17];
+    __shared__ double part[64][17];
     const int tid = threadIdx.x, lr = tid & 15, kq = tid >> 4;   // kq: column of the round, 0..63
     const int r = blockIdx.x * 16 + lr, rc = min(r, m - 1), kend = min(m, (int)(blockIdx.x * 16 / 64 + 1) * 64);
-    double acc[NV];
-#pragma unroll
-    for (int v = 0; v < NV; ++v) acc[v] = 0.0;
+    double acc = 0.0;
 #pragma unroll 8
-    for (int k = kq; k < kend; k += 64) {
-        const double w = W[rc + (size_t)m * k];
-#pragma unroll
-        for (int v = 0; v < NV; ++v) acc[v] = __builtin_fma(w, X[k + (size_t)ldx * v], acc[v]);
-    }
-#pragma unroll
-    for (int v = 0; v < NV; ++v) part[v][kq][lr] = acc[v];
+    for (int k = kq; k < kend; k += 64) acc = __builtin_fma(W[rc + (size_t)m * k], X[k], acc);
+    part[kq][lr] = acc;
     __syncthreads();
-    if (tid < 16 * NV) {
-        const int v = tid >> 4;
+    if (tid < 16) {
         double t = 0.0;
-        for (int q = 0; q < 64; ++q) t += part[v][q][lr];
-        if (r < m) Y[r + (size_t)ldy * v] = u ? t - 2.0 * u[r] * s[v] : t;
+        for (int q = 0; q < 64; ++q) t += part[q][lr];
+        if (r < m) Y[r] = t;
     }
 }
 
@@ -689,24 +674,15 @@ __global__ void k_rank2(double* __restrict__ A, int n, int lda, const double* __
     A[i + (size_t)lda * j] -= w[i] * p[j] + p[i] * w[j];
 }
 
-// xt[0..m) = w1, xt[m..2m) = beta (columns of the products with W)
-__global__ void k_defl_vecs(const double* __restrict__ w, const double* __restrict__ A, int m, double* __restrict__ xt)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    xt[i] = w[1 + i];
-    xt[m + i] = A[1 + i];
-}
-
 // sig = {alpha - beta . wt, w1 . wt}
-__global__ void __launch_bounds__(1024) k_sigma(const double* __restrict__ A, const double* __restrict__ xt,
+__global__ void __launch_bounds__(1024) k_sigma(const double* __restrict__ A, const double* __restrict__ w,
                                                 const double* __restrict__ wt, int m, double* __restrict__ sig)
 {
     __shared__ double red[2][1024];
     double s[2] = {0.0, 0.0};
     for (int i = threadIdx.x; i < m; i += 1024) {
-        s[0] += xt[m + i] * wt[i];
-        s[1] += xt[i] * wt[i];
+        s[0] += A[1 + i] * wt[i];
+        s[1] += w[1 + i] * wt[i];
     }
     for (int v = 0; v < 2; ++v) red[v][threadIdx.x] = s[v];
     __syncthreads();
@@ -728,7 +704,7 @@ bool sym_factor(ilh_plan* pl, SymFactor& F, int n, double* scratch, bool deflate
     F.ok = false;
     const int m = n - 1, mc = std::max(m, 1);
     F.w.ensure(sizeof(double) * (size_t)n);
-    F.vec.ensure(sizeof(double) * (size_t)(2 * n + 5 * mc));
+    F.vec.ensure(sizeof(double) * (size_t)(2 * n + mc));
     F.W.ensure(sizeof(double) * (size_t)mc * mc);
     F.T.ensure(sizeof(double) * (size_t)mc * n);   // also the product W B of a full solve
     F.info.ensure(3 * sizeof(double));   // {sigma, w1.wt}, then the pivot flag
@@ -736,7 +712,6 @@ bool sym_factor(ilh_plan* pl, SymFactor& F, int n, double* scratch, bool deflate
     double* w = F.w.as<double>();
     double* y = F.vec.as<double>();
     double* p = y + n;
-    double *xt = F.xt(), *wx = F.ww();
     double* sig = F.info.as<double>();
     int* info = (int*)(sig + 2);
     k_house_vec<<<(n + 255) / 256, 256, 0, st>>>(w, n, deflate, info);
@@ -748,11 +723,11 @@ bool sym_factor(ilh_plan* pl, SymFactor& F, int n, double* scratch, bool deflate
     ILH_HIP(hipGetLastError());
     if (m > 0) {
         chol_factor(st, A + 1 + (size_t)n, n, m, F.W.as<double>(), scratch, F.T.as<double>(), info);
-        k_defl_vecs<<<(m + 255) / 256, 256, 0, st>>>(w, A, m, xt);
-        k_wmv<2><<<(m + 15) / 16, 1024, 0, st>>>(F.W.as<double>(), m, xt, m, nullptr, nullptr, wx, m);
-        k_wtmv<<<(m + 3) / 4, 256, 0, st>>>(F.W.as<double>(), m, wx + m, F.wt());
+        // wt = Mt^-1 beta (y is free)
+        k_wmv<<<(m + 15) / 16, 1024, 0, st>>>(F.W.as<double>(), m, A + 1, y);
+        k_wtmv<<<(m + 3) / 4, 256, 0, st>>>(F.W.as<double>(), m, y, F.wt());
     }
-    k_sigma<<<1, 1024, 0, st>>>(A, xt, F.wt(), m, sig);
+    k_sigma<<<1, 1024, 0, st>>>(A, w, F.wt(), m, sig);
     ILH_HIP(hipGetLastError());
     double h[3];
     ILH_HIP(hipMemcpyAsync(h, sig, sizeof(h), hipMemcpyDeviceToHost, st));
@@ -764,33 +739,30 @@ bool sym_factor(ilh_plan* pl, SymFactor& F, int n, double* scratch, bool deflate
     return true;
 }
 
-// The first scalars of each column j of the deflated solve M^-1 B (B n x ncols),
-// one wave per column:  r = w . B and y1 = (X'0 - wt . X'1) / sigma with
-// X' = B - 2 w r.
+// The deflated solve's first reflection, X' = B - 2 w (w . B) in place, and its
+// first coordinate y1 = (X'0 - wt . X'1) / sigma; one wave per column j of B
+// (n x ncols), read once from memory and again from the cache.
 __global__ void __launch_bounds__(256) k_defl_cols(const double* __restrict__ w, const double* __restrict__ wt,
-                                                   const double* __restrict__ sig, const double* __restrict__ B, int n,
-                                                   int ncols, double* __restrict__ rv, double* __restrict__ y1v)
+                                                   const double* __restrict__ sig, double* __restrict__ B, int n,
+                                                   int ncols, double* __restrict__ y1v)
 {
     const int j = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (j >= ncols) return;
-    const double* col = B + (size_t)n * j;
-    double s0 = 0.0, s1 = 0.0;
-#pragma unroll 4
-    for (int i = 1 + lane; i < n; i += 64) {
-        const double b = col[i];
-        s0 = __builtin_fma(w[i], b, s0);
-        s1 = __builtin_fma(wt[i - 1], b, s1);
+    double* col = B + (size_t)n * j;
+    double r = 0.0;
+#pragma unroll 8
+    for (int i = lane; i < n; i += 64) r = __builtin_fma(w[i], col[i], r);
+    for (int off = 32; off > 0; off >>= 1) r += __shfl_xor(r, off, 64);
+    double s = 0.0, x0 = 0.0;   // x0: lane 0's first entry
+#pragma unroll 8
+    for (int i = lane; i < n; i += 64) {
+        const double x = __builtin_fma(-2.0 * w[i], r, col[i]);
+        col[i] = x;
+        if (i == 0) x0 = x;
+        else s = __builtin_fma(wt[i - 1], x, s);
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        s0 += __shfl_xor(s0, off, 64);
-        s1 += __shfl_xor(s1, off, 64);
-    }
-    if (lane == 0) {
-        const double w0 = w[0], b0 = col[0];
-        const double r = s0 + w0 * b0;
-        rv[j] = r;
-        y1v[j] = ((b0 - 2.0 * w0 * r) - (s1 - 2.0 * sig[1] * r)) / sig[0];
-    }
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (lane == 0) y1v[j] = (x0 - s) / sig[0];
 }
 
 // The last step of the deflated solve: the second reflection, of [y1; Z - wt y1],
@@ -846,14 +818,13 @@ __global__ void __launch_bounds__(1024) k_defl_vec(const double* __restrict__ w,
 }
 
 // Out[j + ldo p] = (M^-1 B)[p, j] / (c d[p]) for B (n x ncols, leading
-// dimension n): the rows of diag(1 / (c d)) M^-1 B, each contiguous.  The first
-// reflection is a rank-one correction of the product W B, applied as that is
-// written; the second one needs the whole of W^T W B (its dots come with the
-// product, 32 columns of a tile at a time) and is a pass over the result.  A
-// single column (ldo = 1) goes through the vector products instead of 64-wide
-// tiles, and Out may be B then.
-void sym_solve_rows(ilh_plan* pl, SymFactor& F, const double* B, int ncols, const double* d, double c, double* Out,
-                    int ldo)
+// dimension n, overwritten): the rows of diag(1 / (c d)) M^-1 B, each
+// contiguous.  The second reflection needs the whole of W^T W X' (its dots come
+// with the product, 32 columns of a tile at a time) and is a pass over the
+// result.  A single column (ldo = 1) goes through the vector products instead
+// of 64-wide tiles, and Out may be B then.  The reflections are the 26 and 20
+// of a solve's 390 us at N = 1885, all columns.
+void sym_solve_rows(ilh_plan* pl, SymFactor& F, double* B, int ncols, const double* d, double c, double* Out, int ldo)
 {
     if (!F.ok) fail(ILH_ERR_STATE, "symmetric factor not built");
     if (ncols <= 0) return;
@@ -861,29 +832,27 @@ void sym_solve_rows(ilh_plan* pl, SymFactor& F, const double* B, int ncols, cons
     const int n = F.n, m = n - 1;
     const bool vec = ncols == 1 && ldo == 1;
     const int nt = (m + GT - 1) / GT, nd = vec ? 0 : 2 * nt;
-    F.r.ensure(sizeof(double) * (size_t)(2 + nd) * ncols);
-    double *r = F.r.as<double>(), *y1 = r + ncols, *dots = y1 + ncols;
+    F.r.ensure(sizeof(double) * (size_t)(1 + nd) * ncols);
+    double *y1 = F.r.as<double>(), *dots = y1 + ncols;
     const double* w = F.w.as<double>();
     const double* sig = F.info.as<double>();
-    k_defl_cols<<<(ncols + 3) / 4, 256, 0, st>>>(w, F.wt(), sig, B, n, ncols, r, y1);
+    k_defl_cols<<<(ncols + 3) / 4, 256, 0, st>>>(w, F.wt(), sig, B, n, ncols, y1);
     ILH_HIP(hipGetLastError());
     const double* W = F.W.as<double>();
     if (m > 0) {
         F.T.ensure(sizeof(double) * (size_t)m * ncols);
         double* T = F.T.as<double>();
         if (vec) {
-            k_wmv<1><<<(m + 15) / 16, 1024, 0, st>>>(W, m, B + 1, n, F.ww(), r, T, m);
+            k_wmv<<<(m + 15) / 16, 1024, 0, st>>>(W, m, B + 1, T);
             k_wtmv<<<(m + 3) / 4, 256, 0, st>>>(W, m, T, Out + 1);
         } else {
-            GemmEpi e1, e2;
-            e1.u = F.ww();
-            e1.v = r;
-            k_dgemm<0, 0, true, EPI_RANK1><<<dim3(nt, (ncols + GT - 1) / GT), 256, 0, st>>>(
-                m, ncols, m, 1.0, W, m, B + 1, n, T, m, TRI_A_LOWER, GemmBatch(), e1);
-            e2.v = w + 1;
-            e2.dots = dots;
-            k_dgemm<1, 0, true, EPI_DOT><<<dim3((ncols + GT - 1) / GT, nt), 256, 0, st>>>(
-                ncols, m, m, 1.0, T, m, W, m, Out + ldo, ldo, TRI_B_LOWER, GemmBatch(), e2);
+            GemmDots e;
+            e.v = w + 1;
+            e.dots = dots;
+            k_dgemm<0, 0, true, false><<<dim3(nt, (ncols + GT - 1) / GT), 256, 0, st>>>(
+                m, ncols, m, 1.0, W, m, B + 1, n, T, m, TRI_A_LOWER, GemmBatch(), GemmDots());
+            k_dgemm<1, 0, true, true><<<dim3((ncols + GT - 1) / GT, nt), 256, 0, st>>>(
+                ncols, m, m, 1.0, T, m, W, m, Out + ldo, ldo, TRI_B_LOWER, GemmBatch(), e);
         }
         ILH_HIP(hipGetLastError());
     }

@@ -442,21 +442,17 @@ struct SymFactor {
     int n = 0;
     bool ok = false;
     DevBuf A, W, T, w, vec, r, info;
-    // vec: n-vectors y, p (scratch), then of m = n - 1 entries each w1, beta,
-    // W w1, W beta, Mt^-1 beta
-    double* xt() const { return vec.as<double>() + 2 * n; }
-    double* ww() const { return xt() + 2 * (n - 1); }
-    double* wt() const { return xt() + 4 * (n - 1); }
+    // vec: n-vectors y, p (scratch), then wt = Mt^-1 beta (n - 1)
+    double* wt() const { return vec.as<double>() + 2 * n; }
 };
 // A is free for other use after it; scratch: n x n entries (the factor's
 // blocks below the diagonal ones while W = L^-1 is formed).  deflate = false:
 // M is positive definite outright and is factored without the reflection.
 bool sym_factor(ilh_plan* pl, SymFactor& F, int n, double* scratch, bool deflate = true);
-// with S = M diag(c d): the rows of S^-1 B (B n x ncols), row p at Out + ldo p
-// (Out may be B for one column and ldo = 1), and Minv = S^-1 row-major
+// with S = M diag(c d): the rows of S^-1 B (B n x ncols, overwritten), row p at
+// Out + ldo p (Out may be B for one column and ldo = 1), and Minv = S^-1 row-major
 // (leading dimension solve_ld(n), padding columns zero)
-void sym_solve_rows(ilh_plan* pl, SymFactor& F, const double* B, int ncols, const double* d, double c, double* Out,
-                    int ldo);
+void sym_solve_rows(ilh_plan* pl, SymFactor& F, double* B, int ncols, const double* d, double c, double* Out, int ldo);
 void sym_inverse_rowmajor(ilh_plan* pl, SymFactor& F, const double* d, double c, double* Minv);
 // columns [n, ld) of the n rows of a row-major matrix = 0
 void zero_pad_columns(hipStream_t st, double* A, int n, int ld);
