@@ -674,15 +674,19 @@ __global__ void k_rank2(double* __restrict__ A, int n, int lda, const double* __
     A[i + (size_t)lda * j] -= w[i] * p[j] + p[i] * w[j];
 }
 
-// sig = {alpha - beta . wt, w1 . wt}
+// sig = {alpha - beta . wt, w1 . wt}; a pivot of Mt of at most tol (1 / W_ii^2)
+// sets *info if no pivot did
 __global__ void __launch_bounds__(1024) k_sigma(const double* __restrict__ A, const double* __restrict__ w,
-                                                const double* __restrict__ wt, int m, double* __restrict__ sig)
+                                                const double* __restrict__ wt, const double* __restrict__ W, double tol,
+                                                int m, double* __restrict__ sig, int* __restrict__ info)
 {
     __shared__ double red[2][1024];
     double s[2] = {0.0, 0.0};
     for (int i = threadIdx.x; i < m; i += 1024) {
         s[0] += A[1 + i] * wt[i];
         s[1] += w[1 + i] * wt[i];
+        const double r = W[i + (size_t)m * i];
+        if (r * r * tol >= 1.0) atomicCAS(info, 0, i + 1);
     }
     for (int v = 0; v < 2; ++v) red[v][threadIdx.x] = s[v];
     __syncthreads();
@@ -727,14 +731,18 @@ bool sym_factor(ilh_plan* pl, SymFactor& F, int n, double* scratch, bool deflate
         k_wmv<<<(m + 15) / 16, 1024, 0, st>>>(F.W.as<double>(), m, A + 1, y);
         k_wtmv<<<(m + 3) / 4, 256, 0, st>>>(F.W.as<double>(), m, y, F.wt());
     }
-    k_sigma<<<1, 1024, 0, st>>>(A, w, F.wt(), m, sig);
+    // without the deflation every pivot, sigma the last of them, has to stand
+    // clear of rounding (M's entries are at most about 1): a pivot of coinciding
+    // points comes out as rounding of either sign
+    const double tol = deflate ? 0.0 : n * 2.220446049250313e-16;
+    k_sigma<<<1, 1024, 0, st>>>(A, w, F.wt(), F.W.as<double>(), tol, m, sig, info);
     ILH_HIP(hipGetLastError());
     double h[3];
     ILH_HIP(hipMemcpyAsync(h, sig, sizeof(h), hipMemcpyDeviceToHost, st));
     ILH_HIP(hipStreamSynchronize(st));
     int bad;
     std::memcpy(&bad, h + 2, sizeof(bad));
-    if (bad || !(h[0] != 0.0) || !std::isfinite(h[0])) return false;
+    if (bad || !std::isfinite(h[0]) || (deflate ? h[0] == 0.0 : h[0] <= tol)) return false;
     F.ok = true;
     return true;
 }

@@ -565,7 +565,7 @@ static void heat_apply(ilh_plan* pl, const double* K, int M, const double* a, do
 // positive definite (H the heat kernel, or the identity): inverted through the
 // Cholesky of M, LU of E H R if that meets a non-positive pivot, and packed.
 // F, inv: storage shared by the stages.
-static void schur_inverse(ilh_plan* pl, const std::vector<double>& K, bool identity, bool deflate_first, SymFactor& F, DevBuf& inv,
+static void schur_inverse(ilh_plan* pl, const std::vector<double>& K, bool identity, bool deflate, SymFactor& F, DevBuf& inv,
                           StageInverse& out)
 {
     const int N = pl->N;
@@ -592,14 +592,13 @@ static void schur_inverse(ilh_plan* pl, const std::vector<double>& K, bool ident
     // dense reflection its inverse keeps the stage matrix's decay: so for
     // filters of at most 16 taps a side (condition numbers of some tens).
     // Longer ones make it all but singular (4e15 at Fo = 50), where deflating
-    // the constant mode first keeps an order of magnitude more of the
-    // solution; it also takes over from a non-positive pivot, LU from its own.
-    bool ok = false;
-    for (int deflate = deflate_first; deflate < 2 && !ok; ++deflate) {
-        build(OP_E_PRIMAL, F.A.as<double>());
-        ok = sym_factor(pl, F, N, inv.as<double>(), deflate);
-    }
-    if (ok) {
+    // the constant mode first keeps an order of magnitude more of the solution.
+    // LU takes over from a non-positive pivot, and from one at rounding level of
+    // a short filter's matrix: that is points that coincide or are so close that
+    // the pivot's sign is chance; LU refuses the former (of 90 geometries with
+    // one point twice, the deflated factor as a second attempt took half).
+    build(OP_E_PRIMAL, F.A.as<double>());
+    if (sym_factor(pl, F, N, inv.as<double>(), deflate)) {
         sym_inverse_rowmajor(pl, F, pl->ds.as<double>(), 1.0 / (pl->g.dx * pl->g.dx), inv.as<double>());
     } else {
         DevBuf S;

@@ -447,7 +447,8 @@ struct SymFactor {
 };
 // A is free for other use after it; scratch: n x n entries (the factor's
 // blocks below the diagonal ones while W = L^-1 is formed).  deflate = false:
-// M is positive definite outright and is factored without the reflection.
+// M is positive definite outright and is factored without the reflection;
+// false then also for a pivot of at most n eps.
 bool sym_factor(ilh_plan* pl, SymFactor& F, int n, double* scratch, bool deflate = true);
 // with S = M diag(c d): the rows of S^-1 B (B n x ncols, overwritten), row p at
 // Out + ldo p (Out may be B for one column and ldo = 1), and Minv = S^-1 row-major

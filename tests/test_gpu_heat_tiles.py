@@ -52,3 +52,25 @@ def test_heat_tiles(ctx, n, m, fo, N):
             ilhip.interpolate(Eb, T, c)
             assert np.abs(Eb.flat() - 0.5 * (a + (0 if b is None else b))).max() < 1e-12
     heat.close()
+
+
+@pytest.mark.parametrize("N", [30, 47, 64, 90])
+def test_heat_first_point_twice(ctx, N):
+    """Two points at one place: the stage matrices are singular, and the last
+    pivots of their factorisation (the first point's among them) are rounding
+    of either sign, which must not pass for a positive one."""
+    import ilhip
+    from ilhip import geometry as G
+    dx = 0.02
+    g = G.GridSpec(131, 111, 66, 56, dx)
+    r = N * 1.4 * dx / (2 * np.pi)
+    th = np.concatenate([[0.0], 2 * np.pi * np.arange(N) / N])
+    ds = np.full(N + 1, 1.4 * dx)
+    ds[:2] *= 0.5
+    for shift in (0.0, 0.003, 0.0071):
+        s = G.Surface(r * np.cos(th) + shift, r * np.sin(th), np.cos(th), np.sin(th), ds, np.zeros(N + 1, int))
+        c = ilhip.SurfaceScalarCache(s, g, ctx=ctx)
+        for fo in (0.1, 0.5, 1.0):
+            print("heat, one point twice", N, shift, fo, flush=True)
+            with pytest.raises(ilhip.SingularError):
+                ilhip.DirichletHeatConduction(c, 1.0, fo * dx * dx, np.cos(th))
