@@ -32,14 +32,12 @@ namespace ilh {
 typedef double double4_t __attribute__((ext_vector_type(4)));
 
 // ------------------------------------------------------------------ GEMM
-// C (M x Nc) = beta C + alpha opA(A) opB(B), column-major, beta in {0, 1}
-// (BETA0: C is not read).  opA(A)[m][k] = A[m + lda k] (TA = 0) or
-// A[k + lda m] (TA = 1); opB(B)[k][n] = B[k + ldb n] (TB = 0) or B[n + ldb k]
-// (TB = 1).  tri restricts the K range of each tile to where a triangular
-// operand is nonzero (entries of its other triangle outside its 64 x 64
-// diagonal blocks are never read): TRI_A_LOWER opA(A)[m][k] = 0 for k > m,
-// TRI_A_UPPER for k < m, TRI_B_LOWER opB(B)[k][n] = 0 for k < n, TRI_B_UPPER
-// for k > n.
+// C (M x Nc) = beta C + alpha opA(A) B, column-major, beta in {0, 1} (BETA0: C
+// is not read).  opA(A)[m][k] = A[m + lda k] (TA = 0) or A[k + lda m] (TA = 1),
+// B[k][n] at k + ldb n.  tri restricts the K range of each tile to where a
+// triangular operand is nonzero (entries of its other triangle outside its
+// 64 x 64 diagonal blocks are never read): TRI_A_LOWER opA(A)[m][k] = 0 for
+// k > m, TRI_B_LOWER B[k][n] = 0 for k < n.
 //
 // 64 x 64 tile per work-group of four waves, each wave a 32 x 32 quadrant of
 // 2 x 2 blocks of 16 x 16.  K runs in chunks of 16 through two LDS buffers:
@@ -56,6 +54,7 @@ typedef double double4_t __attribute__((ext_vector_type(4)));
 // X[i][k] at lane i + 16 k, second Y[k][j] at lane j + 16 k; lane l, item r
 // of the result holds D[l / 16 + 4 r][l % 16].
 static constexpr int GT = 64, GKC = 16;
+enum { TRI_NONE = 0, TRI_A_LOWER = 1, TRI_B_LOWER = 2 };
 
 // A batch runs over blockIdx.z: operands at z times the strides, M (and K,
 // when k_is_m) clipped to what is left of m_total rows z m_step on.
@@ -71,7 +70,7 @@ struct GemmDots {
     double* dots = nullptr;
 };
 
-template <int TA, int TB, bool BETA0, bool DOT>
+template <int TA, bool BETA0, bool DOT>
 // (A or B may be C itself when every work-group reads all the entries it
 // overwrites; hence no __restrict__.)
 __global__ void __launch_bounds__(256) k_dgemm(int M, int Nc, int K, double alpha, const double* A, int lda,
@@ -96,23 +95,19 @@ __global__ void __launch_bounds__(256) k_dgemm(int M, int Nc, int K, double alph
         int t = blockIdx.x + gridDim.x * blockIdx.y;
         const int r0 = t & ~255;
         if (r0 & 256) t = r0 + min(256, total - r0) - 1 - (t - r0);
-        if (tri == TRI_A_LOWER || tri == TRI_A_UPPER) {
-            bx = t / gridDim.y;
+        if (tri == TRI_A_LOWER) {
+            bx = gridDim.x - 1 - t / gridDim.y;
             by = t % gridDim.y;
-            if (tri == TRI_A_LOWER) bx = gridDim.x - 1 - bx;
         } else {
             by = t / gridDim.x;
             bx = t % gridDim.x;
-            if (tri == TRI_B_UPPER) by = gridDim.y - 1 - by;
         }
     }
     const int m0 = bx * GT, n0 = by * GT;
     if (m0 >= M || n0 >= Nc) return;
     int klo = 0, khi = K;
     if (tri == TRI_A_LOWER) khi = min(K, m0 + GT);
-    else if (tri == TRI_A_UPPER) klo = m0;
     else if (tri == TRI_B_LOWER) klo = n0;
-    else if (tri == TRI_B_UPPER) khi = min(K, n0 + GT);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
     // this thread's four elements of each operand's chunk.  Rows and columns
@@ -121,35 +116,34 @@ __global__ void __launch_bounds__(256) k_dgemm(int M, int Nc, int K, double alph
     // LDS: the loads themselves carry no branch or use, so that three chunks
     // of them stay in flight
     const int am = TA == 0 ? tid & 63 : tid >> 4, ak = TA == 0 ? tid >> 6 : tid & 15;
-    const int bn = TB == 0 ? tid >> 4 : tid & 63, bk = TB == 0 ? tid & 15 : tid >> 6;
+    const int bn = tid >> 4, bk = tid & 15;
     const double *pa[4], *pb[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const int m = min(m0 + am + (TA == 0 ? 0 : 16 * j), M - 1), n = min(n0 + bn + (TB == 0 ? 16 * j : 0), Nc - 1);
-        const int k = klo + ak + (TA == 0 ? 4 * j : 0), kb = klo + bk + (TB == 0 ? 0 : 4 * j);
+        const int m = min(m0 + am + (TA == 0 ? 0 : 16 * j), M - 1), n = min(n0 + bn + 16 * j, Nc - 1);
+        const int k = klo + ak + (TA == 0 ? 4 * j : 0);
         pa[j] = TA == 0 ? A + m + (size_t)lda * k : A + k + (size_t)lda * m;
-        pb[j] = TB == 0 ? B + kb + (size_t)ldb * n : B + n + (size_t)ldb * kb;
+        pb[j] = B + (klo + bk) + (size_t)ldb * n;
     }
-    const size_t step_a = TA == 0 ? (size_t)lda * GKC : GKC, step_b = TB == 0 ? GKC : (size_t)ldb * GKC;
+    const size_t step_a = TA == 0 ? (size_t)lda * GKC : GKC;
     double pre[3][8];   // three chunks on the way: [0..3] of A, [4..7] of B
     auto load = [&](int k0, double* r) {   // the chunk at k0 (in order: the pointers advance with it)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             r[j] = *(k0 + ak + (TA == 0 ? 4 * j : 0) < khi ? pa[j] : A);
-            r[4 + j] = *(k0 + bk + (TB == 0 ? 0 : 4 * j) < khi ? pb[j] : B);
+            r[4 + j] = *(k0 + bk < khi ? pb[j] : B);
             pa[j] += step_a;
-            pb[j] += step_b;
+            pb[j] += GKC;
         }
     };
     auto store = [&](int k0, int buf, const double* r) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const double va = k0 + ak + (TA == 0 ? 4 * j : 0) < khi ? r[j] : 0.0;
-            const double vb = k0 + bk + (TB == 0 ? 0 : 4 * j) < khi ? r[4 + j] : 0.0;
+            const double vb = k0 + bk < khi ? r[4 + j] : 0.0;
             if (TA == 0) As[buf][(tid >> 6) + 4 * j][tid & 63] = va;
             else As[buf][tid & 15][(tid >> 4) + 16 * j] = va;
-            if (TB == 0) Bs[buf][tid & 15][(tid >> 4) + 16 * j] = vb;
-            else Bs[buf][(tid >> 6) + 4 * j][tid & 63] = vb;
+            Bs[buf][tid & 15][(tid >> 4) + 16 * j] = vb;
         }
     };
     double4_t acc[2][2];
@@ -223,29 +217,11 @@ __global__ void __launch_bounds__(256) k_dgemm(int M, int Nc, int K, double alph
     }
 }
 
-void dgemm(hipStream_t st, int ta, int tb, int M, int Nc, int K, double alpha, const double* A, int lda,
-           const double* B, int ldb, double beta, double* C, int ldc, int tri)
+void gemm_sub(hipStream_t st, int M, int Nc, int K, const double* A, int lda, const double* B, int ldb, double* C, int ldc)
 {
-    if (M <= 0 || Nc <= 0) return;
-    if (beta != 0.0 && beta != 1.0) fail(ILH_ERR_ARG, "dgemm: beta must be 0 or 1");
-    const dim3 grid((M + GT - 1) / GT, (Nc + GT - 1) / GT);
-    const bool b0 = beta == 0.0;
-#define ILH_DG(TA_, TB_, B0_) \
-    k_dgemm<TA_, TB_, B0_, false><<<grid, 256, 0, st>>>(M, Nc, K, alpha, A, lda, B, ldb, C, ldc, tri, GemmBatch(), GemmDots())
-    if (K <= 0) {
-        if (!b0) return;
-        alpha = 0.0;   // C = 0
-    }
-    if (ta == 0 && tb == 0) {
-        if (b0) ILH_DG(0, 0, true); else ILH_DG(0, 0, false);
-    } else if (ta == 0 && tb == 1) {
-        if (b0) ILH_DG(0, 1, true); else ILH_DG(0, 1, false);
-    } else if (ta == 1 && tb == 0) {
-        if (b0) ILH_DG(1, 0, true); else ILH_DG(1, 0, false);
-    } else {
-        if (b0) ILH_DG(1, 1, true); else ILH_DG(1, 1, false);
-    }
-#undef ILH_DG
+    if (M <= 0 || Nc <= 0 || K <= 0) return;
+    k_dgemm<0, false, false><<<dim3((M + GT - 1) / GT, (Nc + GT - 1) / GT), 256, 0, st>>>(
+        M, Nc, K, -1.0, A, lda, B, ldb, C, ldc, TRI_NONE, GemmBatch(), GemmDots());
     ILH_HIP(hipGetLastError());
 }
 
@@ -342,7 +318,7 @@ __device__ __forceinline__ void sub_update(Block& T, int i, int j, int b, int la
 // readlane, so the rows below the diagonal sub-block cost nothing extra; the
 // next panel's update comes first, and everything else (the remaining
 // updates, the inverse's finished rows) runs on the other waves beside the
-// next panel.  Seven barriers; the chain of 64 pivot steps bounds it.
+// next panel.  Eight barriers; the chain of 64 pivot steps bounds it.
 // A pivot that is not positive records its 1-based column col0 + ... in *info
 // (the first one only) and is replaced by 1, so that the kernel still runs to
 // its end.
@@ -569,11 +545,11 @@ static void chol_factor(hipStream_t st, double* A, int lda, int m, double* W, do
         bt.m_step = 2 * s;
         const dim3 grid((std::min(s, m - s) + GT - 1) / GT, s / GT, pairs);
         // T21 = L21 W11
-        k_dgemm<0, 0, true, false><<<grid, 256, 0, st>>>(std::min(s, m - s), s, s, 1.0, Lb + off, m, W, m, T + off, m,
+        k_dgemm<0, true, false><<<grid, 256, 0, st>>>(std::min(s, m - s), s, s, 1.0, Lb + off, m, W, m, T + off, m,
                                                            TRI_B_LOWER, bt, GemmDots());
         // W21 = -W22 T21
         bt.k_is_m = 1;
-        k_dgemm<0, 0, true, false><<<grid, 256, 0, st>>>(std::min(s, m - s), s, s, -1.0, W + off + (size_t)m * s, m,
+        k_dgemm<0, true, false><<<grid, 256, 0, st>>>(std::min(s, m - s), s, s, -1.0, W + off + (size_t)m * s, m,
                                                            T + off, m, W + off, m, TRI_A_LOWER, bt, GemmDots());
     }
     ILH_HIP(hipGetLastError());
@@ -857,9 +833,9 @@ void sym_solve_rows(ilh_plan* pl, SymFactor& F, double* B, int ncols, const doub
             GemmDots e;
             e.v = w + 1;
             e.dots = dots;
-            k_dgemm<0, 0, true, false><<<dim3(nt, (ncols + GT - 1) / GT), 256, 0, st>>>(
+            k_dgemm<0, true, false><<<dim3(nt, (ncols + GT - 1) / GT), 256, 0, st>>>(
                 m, ncols, m, 1.0, W, m, B + 1, n, T, m, TRI_A_LOWER, GemmBatch(), GemmDots());
-            k_dgemm<1, 0, true, true><<<dim3((ncols + GT - 1) / GT, nt), 256, 0, st>>>(
+            k_dgemm<1, true, true><<<dim3((ncols + GT - 1) / GT, nt), 256, 0, st>>>(
                 ncols, m, m, 1.0, T, m, W, m, Out + ldo, ldo, TRI_B_LOWER, GemmBatch(), e);
         }
         ILH_HIP(hipGetLastError());

@@ -356,15 +356,6 @@ void assemble_table(ilh_plan* pl, int opA, int opB, const double* tab, int Tn, d
     launch_assemble(pl, opA, opB, tab, Tn, factor, false, K, pl->N, false);
 }
 
-// C[M x Nc] -= A[M x K] B[K x Nc] on stream st (the trailing updates of the
-// blocked LU and of its multi-right-hand-side solves), on the FP64 matrix cores
-static void gemm_sub(hipStream_t st, int M, int Nc, int K, const double* A, int lda, const double* B, int ldb,
-                     double* C, int ldc)
-{
-    if (M <= 0 || Nc <= 0 || K <= 0) return;
-    dgemm(st, 0, 0, M, Nc, K, -1.0, A, lda, B, ldb, 1.0, C, ldc);
-}
-
 // ------------------------------------------------------------------- LU
 static constexpr int NB = 32;
 

@@ -101,7 +101,6 @@ enum OpKind {
 };
 int op_terms_per_point(int op);
 int op_amps_per_point(int op);   // amplitudes a point carries (2: VectorData, or two tensor components)
-bool op_is_scatter(int op);
 
 // Row-binned index of scatter terms on one component grid:
 // entries[row_ptr[j] .. row_ptr[j+1]) are term indices whose window touches
@@ -427,12 +426,10 @@ void assemble(ilh_plan* pl, int opA, int opB, int gk, double scale, bool delta_k
 void assemble_table(ilh_plan* pl, int opA, int opB, const double* tab, int Tn, double factor,
                     double* K /* N x N col-major */);
 int  lu_factor(ilh_plan* pl, double* A, int n, int* piv_dev, int* info_dev);
-// C (M x Nc) = beta C + alpha opA(A) opB(B) on the FP64 matrix cores (ilh_chol.hip),
-// column-major, ta/tb = 1 for a transposed operand, beta 0 or 1;
-// tri: the K range of each tile restricted to a triangular operand's nonzero half
-enum { TRI_NONE = 0, TRI_A_LOWER = 1, TRI_A_UPPER = 2, TRI_B_LOWER = 3, TRI_B_UPPER = 4 };
-void dgemm(hipStream_t st, int ta, int tb, int M, int Nc, int K, double alpha, const double* A, int lda,
-           const double* B, int ldb, double beta, double* C, int ldc, int tri = TRI_NONE);
+// C (M x Nc) -= A (M x K) B (K x Nc), column-major, on the FP64 matrix cores
+// (ilh_chol.hip): the trailing updates of the blocked LU and of its
+// multi-right-hand-side solves
+void gemm_sub(hipStream_t st, int M, int Nc, int K, const double* A, int lda, const double* B, int ldb, double* C, int ldc);
 // A symmetric matrix M that is positive definite on the vectors orthogonal to
 // the constant one (the symmetrised Schur matrices E K E^T), factored as a
 // Householder-deflated Cholesky (ilh_chol.hip).  The caller fills A (n x n,

@@ -294,15 +294,6 @@ int op_amps_per_point(int op)
     }
 }
 
-bool op_is_scatter(int op)
-{
-    switch (op) {
-    case OP_R_PRIMAL: case OP_R_DUAL: case OP_R_EDGES: case OP_RN: case OP_RNX:
-    case OP_DS: case OP_CST: case OP_CXT: case OP_CVT: case OP_DSYM: case OP_RNSYM: case OP_CDSYM: return true;
-    default: return false;
-    }
-}
-
 void build_terms(ilh_plan* pl, int op)
 {
     const int T = op_terms_per_point(op);
