@@ -1,6 +1,6 @@
 """The Stokes solve where its launches differ: bodies at the edge of the allowed
-margin, thin grids, odd and even point counts, periods of the potential and of
-the streamfunction that differ, other DDFs.
+margin, thin grids, odd and even point counts, source periods below the grid's
+own (which the potential always takes), other DDFs.
 
 Bars as the vector cache's Stokes tests: relative L2 1e-10 for the velocity and
 for the streamfunction up to a constant, 1e-9 for the traction.
