@@ -34,7 +34,8 @@
 //   E T = r2 + ...                       -> sigma_3,  T += dt b3 R sigma_3
 // the scheme's stages with the filter's linearity used: F and the W_i are zero
 // away from the bodies, and the intermediate stages are needed only where E
-// reads them, so two passes over the grid serve a step (of five).
+// reads them, so two passes over the grid serve a step (of five).  With a filter
+// of more than 16 taps a side a step keeps the five passes (ilh_heat_advance).
 #include "ilh_internal.hpp"
 
 #include <algorithm>
@@ -256,7 +257,9 @@ constexpr int HTH = 512; // threads per tile
 // kernel read and write it twice.  2048^2: 23 us at M = 10, 27 us at M = 12
 // (an x and a y kernel: 41 us), of which memory's share (33.5 MB in and out)
 // is about 12 us and FP64 issue's about 8; two work-groups of eight waves per
-// CU overlap them (of four waves each: 28 and 33 us).
+// CU overlap them (of four waves each: 28 and 33 us).  The forms for 14 and 16
+// taps spill 15 and 38 registers under that cap; a step at 2048^2 with 3000
+// points takes 105 us at 12 taps, 114 at 14 and 130 at 16.
 template <int MB>
 __global__ void __launch_bounds__(HTH, 4) k_heat_xy(TilePass P)
 {
