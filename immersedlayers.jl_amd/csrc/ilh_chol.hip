@@ -724,29 +724,48 @@ bool sym_factor(ilh_plan* pl, SymFactor& F, int n, double* scratch, bool deflate
 }
 
 // The deflated solve's first reflection, X' = B - 2 w (w . B) in place, and its
-// first coordinate y1 = (X'0 - wt . X'1) / sigma; one wave per column j of B
-// (n x ncols), read once from memory and again from the cache.
+// first coordinate y1 = (X'0 - wt . X'1) / sigma; a work-group per column of B
+// (n rows), its first 2048 entries kept in registers between the two dots.
+// Bound by the latency of one round of loads and two reductions; N = 1885:
+// 12 us (a wave per column that read it twice: 26).
 __global__ void __launch_bounds__(256) k_defl_cols(const double* __restrict__ w, const double* __restrict__ wt,
                                                    const double* __restrict__ sig, double* __restrict__ B, int n,
-                                                   int ncols, double* __restrict__ y1v)
+                                                   double* __restrict__ y1v)
 {
-    const int j = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (j >= ncols) return;
-    double* col = B + (size_t)n * j;
-    double r = 0.0;
-#pragma unroll 8
-    for (int i = lane; i < n; i += 64) r = __builtin_fma(w[i], col[i], r);
-    for (int off = 32; off > 0; off >>= 1) r += __shfl_xor(r, off, 64);
-    double s = 0.0, x0 = 0.0;   // x0: lane 0's first entry
-#pragma unroll 8
-    for (int i = lane; i < n; i += 64) {
-        const double x = __builtin_fma(-2.0 * w[i], r, col[i]);
-        col[i] = x;
-        if (i == 0) x0 = x;
-        else s = __builtin_fma(wt[i - 1], x, s);
+    constexpr int E = 8;
+    __shared__ double red[2][4];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    double* col = B + (size_t)n * blockIdx.x;
+    auto total = [&](double a, double* q) {
+        for (int off = 32; off > 0; off >>= 1) a += __shfl_xor(a, off, 64);
+        if (lane == 0) q[wave] = a;
+        __syncthreads();
+        return (q[0] + q[1]) + (q[2] + q[3]);
+    };
+    double x[E], ww[E], r = 0.0;
+#pragma unroll
+    for (int u = 0; u < E; ++u) {
+        const int i = t + 256 * u;
+        x[u] = i < n ? col[i] : 0.0;
+        ww[u] = i < n ? w[i] : 0.0;
     }
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if (lane == 0) y1v[j] = (x0 - s) / sig[0];
+#pragma unroll
+    for (int u = 0; u < E; ++u) r = __builtin_fma(ww[u], x[u], r);
+    for (int i = t + 256 * E; i < n; i += 256) r = __builtin_fma(w[i], col[i], r);
+    r = total(r, red[0]);
+    double s = 0.0, x0 = 0.0;   // x0: the first entry, thread 0's
+    auto reflect = [&](int i, double wi, double b) {
+        const double v = __builtin_fma(-2.0 * wi, r, b);
+        col[i] = v;
+        if (i == 0) x0 = v;
+        else s = __builtin_fma(wt[i - 1], v, s);
+    };
+#pragma unroll
+    for (int u = 0; u < E; ++u)
+        if (t + 256 * u < n) reflect(t + 256 * u, ww[u], x[u]);
+    for (int i = t + 256 * E; i < n; i += 256) reflect(i, w[i], col[i]);
+    s = total(s, red[1]);
+    if (t == 0) y1v[blockIdx.x] = (x0 - s) / sig[0];
 }
 
 // The last step of the deflated solve: the second reflection, of [y1; Z - wt y1],
@@ -806,8 +825,8 @@ __global__ void __launch_bounds__(1024) k_defl_vec(const double* __restrict__ w,
 // contiguous.  The second reflection needs the whole of W^T W X' (its dots come
 // with the product, 32 columns of a tile at a time) and is a pass over the
 // result.  A single column (ldo = 1) goes through the vector products instead
-// of 64-wide tiles, and Out may be B then.  The reflections are the 26 and 20
-// of a solve's 390 us at N = 1885, all columns.
+// of 64-wide tiles, and Out may be B then.  The reflections are 12 and 20 of a
+// solve's 370 us at N = 1885, all columns.
 void sym_solve_rows(ilh_plan* pl, SymFactor& F, double* B, int ncols, const double* d, double c, double* Out, int ldo)
 {
     if (!F.ok) fail(ILH_ERR_STATE, "symmetric factor not built");
@@ -820,7 +839,7 @@ void sym_solve_rows(ilh_plan* pl, SymFactor& F, double* B, int ncols, const doub
     double *y1 = F.r.as<double>(), *dots = y1 + ncols;
     const double* w = F.w.as<double>();
     const double* sig = F.info.as<double>();
-    k_defl_cols<<<(ncols + 3) / 4, 256, 0, st>>>(w, F.wt(), sig, B, n, ncols, y1);
+    k_defl_cols<<<ncols, 256, 0, st>>>(w, F.wt(), sig, B, n, y1);
     ILH_HIP(hipGetLastError());
     const double* W = F.W.as<double>();
     if (m > 0) {
